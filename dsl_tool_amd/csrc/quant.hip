@@ -4,7 +4,8 @@
 // All kernels read x[r*sr + c*sc] (bf16 or fp32) and write K-major codes
 // q[r*C + c] (FP8) or packed nibbles q[r*C/2 + c/2] (FP4).  fp32 sources
 // divide with the IEEE division: contiguous rows on the fp32 team kernel
-// (quant_f32_rowgroup_kernel), anything else on the strided kernels.  bf16
+// (quant_f32_rowgroup_kernel), [K,N] sources on the transposed one, anything
+// else on the strided kernels.  bf16
 // code paths, fastest first:
 //   * packed path (sc == 1, sr == C, C % 8 == 0, 16-B aligned x, fewer than
 //     2^31 chunks; row groups also need C % group == 0): the input is one run
@@ -16,15 +17,18 @@
 //     one workgroup holds its tile in registers, so x is read once;
 //   * team path (vector-aligned rows, any C): a team of T lanes owns one
 //     group of 8*T elements of a row;
-//   * strided path (anything else, e.g. the reference's B[K,N] given as a
-//     contiguous [K,N] tensor): one thread per scale group, threads ordered
-//     so that the unit-stride axis is the fast one across lanes.
+//   * transposed path (unit row stride: the reference's B[K,N] read as its
+//     [N,K] view; bf16 and fp32): tiles loaded along the contiguous axis and
+//     turned through LDS;
+//   * strided path (anything else): one thread per scale group, threads
+//     ordered so that the unit-stride axis is the fast one across lanes.
 // Arithmetic is the bit-exact contract of include/dsl_gemm.h (fp32 scales,
 // codes of the IEEE quotient x / scale, RNE).  The vector paths encode with
 // the gfx950 converters and the corrected reciprocal quotient of common.h
 // (quot), which give the same codes; the strided path divides and encodes in
 // software.
 #include <mutex>
+#include <utility>
 
 #include "launch.h"
 #include "quant_core.h"
@@ -591,6 +595,236 @@ __global__ __launch_bounds__(256) void quant_fp8_tile_kernel(
 }
 
 // ---------------------------------------------------------------------------
+// Transposed path: unit row stride, i.e. a [K, N] matrix in memory (the
+// reference's B) read as the K-major operand x[r + c*ld].  One workgroup takes
+// 8*NC rows x 32*KE columns (KE = 4 FP8, 8 FP4 columns per thread): thread
+// (c, kk) loads columns kk*KE .. +KE-1 of the 8 rows 8c .. 8c+7, 16 bytes of
+// bf16 per column, so a wave reads whole 128-byte lines along the contiguous
+// axis.  It packs each row's KE codes into one 32-bit word; the words cross
+// through LDS (16-byte chunks XOR-swizzled by row / 8) and every row leaves
+// in 128-byte runs.  HBM-bound: x is read once (twice where one scale covers
+// more than a tile: pass A takes the amax, pass B reads the tiles again,
+// mostly from L2), codes written once.  The one-thread-per-group kernels this
+// replaces wrote single bytes K apart.  bf16 4096 x 4096 per tensor: amax 33.4
+// -> 7.4 us, encode 86.1 -> 11.4 us (4.4 TB/s); 5000 x 2880 fp32 in 1 x 128
+// groups: 174 -> 20.5 us.
+//
+// KIND_FP8: NC = 8: 1 x gc groups, gc a multiple of 128 (or >= cols);
+//           NC = 16: 128 x 128 tiles.
+// ---------------------------------------------------------------------------
+template <bool VEC, typename T, int KE>
+struct TransTile;
+
+// bf16: column j of the thread's 8 rows as packed pairs
+template <bool VEC, int KE>
+struct TransTile<VEC, uint16_t, KE> {
+  uint4 v[KE];
+  DSL_DEV void load(const uint16_t *x, int64_t ld, int nrow, int ncol) {
+#pragma unroll
+    for (int j = 0; j < KE; ++j) {
+      v[j] = make_uint4(0, 0, 0, 0);
+      if (j < ncol && nrow > 0) {
+        const uint16_t *p = x + j * ld;
+        if constexpr (VEC) {
+          v[j] = *reinterpret_cast<const uint4 *>(p);
+        } else {
+          uint32_t w[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) w[i] = i < nrow ? p[i] : 0;
+          v[j] = make_uint4(w[0] | (w[1] << 16), w[2] | (w[3] << 16), w[4] | (w[5] << 16),
+                            w[6] | (w[7] << 16));
+        }
+      }
+    }
+  }
+  DSL_DEV float at(int i, int j) const {
+    const uint32_t w = i < 2 ? v[j].x : i < 4 ? v[j].y : i < 6 ? v[j].z : v[j].w;
+    return u2f((i & 1) ? (w & 0xffff0000u) : (w << 16));
+  }
+};
+
+template <bool VEC, int KE>
+struct TransTile<VEC, float, KE> {
+  float v[KE][8];
+  DSL_DEV void load(const float *x, int64_t ld, int nrow, int ncol) {
+#pragma unroll
+    for (int j = 0; j < KE; ++j) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[j][i] = 0.f;
+      if (j < ncol && nrow > 0) {
+        const float *p = x + j * ld;
+        if constexpr (VEC) {
+          load8(p, v[j]);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) v[j][i] = i < nrow ? p[i] : 0.f;
+        }
+      }
+    }
+  }
+  DSL_DEV float at(int i, int j) const { return v[j][i]; }
+};
+
+template <int KIND, bool VEC, typename T, int NC>
+__global__ __launch_bounds__(NC * 32) void quant_trans_kernel(
+    const T *__restrict__ x, int64_t rows, int64_t cols, int64_t ld, int64_t gc,
+    uint8_t *__restrict__ q, void *__restrict__ scales, const float *__restrict__ partial, int np,
+    float *__restrict__ sout) {
+  constexpr bool FP4 = KIND == KIND_MX || KIND == KIND_NV;
+  constexpr bool F32 = sizeof(T) == 4;
+  constexpr bool TILE = NC == 16;               // one scale per 128 x 128 tile
+  constexpr int KE = FP4 ? 8 : 4, KT = 32 * KE, NR = 8 * NC, NT = 32 * NC, NW = NT / 64;
+  static_assert(!TILE || KIND == KIND_FP8, "128-row tiles: block scales");
+  __shared__ __align__(16) uint32_t stg[NR * 32];
+  __shared__ float sh[NW * NR];
+  float st = 1.f, rt = 1.f;
+  if constexpr (KIND == KIND_TENSOR || KIND == KIND_NV) {
+    const float am = reduce_partials(partial, np, sh);
+    if constexpr (KIND == KIND_TENSOR) st = F32 ? fp8_scale_ieee(am) : fp8_scale_of(am);
+    else st = F32 ? nv_global_ieee(am) : nv_global_of(am);
+    rt = rcp_approx(st);
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *sout = st;
+  }
+  const int t = threadIdx.x, c = t % NC, kk = t / NC;
+  const int64_t n0 = (int64_t)blockIdx.x * NR;
+  const int nrow = (int)(rows - n0 - 8 * c < 8 ? rows - n0 - 8 * c : 8);   // rows of this thread
+  const T *xt = x + n0 + 8 * c;
+  const int64_t span = KIND == KIND_FP8 ? gc : KT;                         // columns of this block
+  const int64_t c0 = (int64_t)blockIdx.y * span, c1 = c0 + span < cols ? c0 + span : cols;
+  TransTile<VEC, T, KE> d;
+  auto load = [&](int64_t k0) {
+    const int64_t k = k0 + kk * KE;
+    const int64_t left = c1 - k;
+    d.load(xt + k * ld, ld, nrow, (int)(left < 0 ? 0 : (left < KE ? left : KE)));
+  };
+  float s[8], r[8];               // FP8: the row's scale and its reciprocal
+  if constexpr (KIND == KIND_FP8) {
+    float m[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) m[i] = 0.f;
+    for (int64_t k0 = c0; k0 < c1; k0 += KT) {
+      load(k0);
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < KE; ++j) m[i] = fmaxf(m[i], __builtin_fabsf(d.at(i, j)));
+    }
+    if constexpr (TILE) {
+#pragma unroll
+      for (int i = 1; i < 8; ++i) m[0] = fmaxf(m[0], m[i]);
+      const float am = block_max(m[0], sh);
+      s[0] = F32 ? fp8_scale_ieee(am) : fp8_scale_of(am);
+      if (t == 0)
+        reinterpret_cast<float *>(scales)[blockIdx.x * ((cols + gc - 1) / gc) + blockIdx.y] = s[0];
+      r[0] = rcp_approx(s[0]);
+#pragma unroll
+      for (int i = 1; i < 8; ++i) {
+        s[i] = s[0];
+        r[i] = r[0];
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+#pragma unroll
+        for (int o = NC; o < 64; o <<= 1) m[i] = fmaxf(m[i], __shfl_xor(m[i], o));
+      }
+      if ((t & 63) < NC) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) sh[(t >> 6) * NR + 8 * c + i] = m[i];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        float am = sh[8 * c + i];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) am = fmaxf(am, sh[w * NR + 8 * c + i]);
+        s[i] = F32 ? fp8_scale_ieee(am) : fp8_scale_of(am);
+        r[i] = rcp_approx(s[i]);
+      }
+      if (kk == 0) {
+        const int64_t gpr = (cols + gc - 1) / gc;
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if (i < nrow)
+            reinterpret_cast<float *>(scales)[(n0 + 8 * c + i) * gpr + blockIdx.y] = s[i];
+      }
+    }
+  } else if constexpr (KIND == KIND_TENSOR) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      s[i] = st;
+      r[i] = rt;
+    }
+  }
+  const bool one = c1 - c0 <= KT;               // FP8: the tile is still in registers
+  const int64_t rowb = FP4 ? cols / 2 : cols;   // code bytes per row
+  for (int64_t k0 = c0; k0 < c1; k0 += KT) {
+    if (KIND != KIND_FP8 || !one) load(k0);
+    if constexpr (FP4) {
+      constexpr int GL = KIND == KIND_MX ? 4 : 2;          // threads (kk) per scale group
+      const int64_t g = (k0 + kk * KE) / (GL * KE), gpr = cols / (GL * KE);
+      const bool put = kk % GL == 0 && k0 + kk * KE < c1;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        float f[8], m = 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          f[j] = d.at(i, j);
+          m = fmaxf(m, __builtin_fabsf(f[j]));
+        }
+#pragma unroll
+        for (int o = NC; o < NC * GL; o <<= 1) m = fmaxf(m, __shfl_xor(m, o));
+        uint32_t code, sb;
+        if constexpr (KIND == KIND_MX) {
+          const int e = mx_exponent(m);
+          sb = (uint32_t)(e + 127);
+          code = e2m1_mul8(f, pow2_neg(e));
+        } else {
+          sb = F32 ? (uint32_t)e4m3_encode(__fdiv_rn(__fdiv_rn(m, 6.0f), st)) : nv_block_code(m, st, rt);
+          const float dd = e4m3_value(sb) * st;
+          code = dd != 0.f ? (F32 ? e2m1_div8(f, dd) : e2m1_quot8(f, dd, rcp_approx(dd))) : 0u;
+        }
+        if (put && i < nrow) reinterpret_cast<uint8_t *>(scales)[(n0 + 8 * c + i) * gpr + g] = (uint8_t)sb;
+        stg[(8 * c + i) * 32 + (((kk >> 2) ^ (c & 7)) << 2) + (kk & 3)] = code;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float f0 = d.at(i, 0), f1 = d.at(i, 1), f2 = d.at(i, 2), f3 = d.at(i, 3);
+        uint32_t code;
+        if constexpr (F32) {
+          code = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(__fdiv_rn(f0, s[i]), __fdiv_rn(f1, s[i]), 0, false);
+          code = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(__fdiv_rn(f2, s[i]), __fdiv_rn(f3, s[i]), (int)code, true);
+        } else {
+          code = e4m3_quot4(f0, f1, f2, f3, s[i], r[i]);
+        }
+        stg[(8 * c + i) * 32 + (((kk >> 2) ^ (c & 7)) << 2) + (kk & 3)] = code;
+      }
+    }
+    __syncthreads();
+    const int64_t b0 = FP4 ? k0 / 2 : k0;
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+      const int idx = t + it * NT, row = idx >> 3, ch = idx & 7;
+      const int64_t b = b0 + ch * 16, left = rowb - b;      // bytes of the row from here on
+      if (n0 + row < rows && left > 0) {
+        const uint4 w = *reinterpret_cast<const uint4 *>(stg + row * 32 + ((ch ^ ((row >> 3) & 7)) << 2));
+        uint8_t *dst = q + (n0 + row) * rowb + b;
+        if ((rowb & 15) == 0) {
+          *reinterpret_cast<uint4 *>(dst) = w;
+        } else {
+          const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+          for (int e = 0; e < 16; ++e)
+            if (e < left) dst[e] = (uint8_t)(ww[e >> 2] >> (8 * (e & 3)));
+        }
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Host launchers (validated by capi.hip before they are called).
 // ---------------------------------------------------------------------------
 static bool vec_ok(const void *x, int64_t cols, int64_t sr, int64_t sc) {
@@ -618,6 +852,49 @@ static int grid_for(int64_t work, int per_block) {
 static bool f32_vec_ok(const void *x, int64_t cols, int64_t sr, int64_t sc) {
   return sc == 1 && (cols % 8) == 0 && (sr % 4) == 0 &&
          (reinterpret_cast<uintptr_t>(x) % 16) == 0;
+}
+
+// Unit row stride: a [cols][sc] matrix in memory whose contiguous axis is the
+// rows (rows > 1, else the row kernels read it as well).
+static bool trans_ok(int64_t rows, int64_t cols, int64_t sr, int64_t sc) {
+  return sr == 1 && sc >= rows && rows > 1 && cols > 1 && (rows + 63) / 64 < ((int64_t)1 << 31) &&
+         (cols + 127) / 128 <= 65535;
+}
+
+template <int KIND, int NC, typename T>
+static void launch_trans(const T *x, int64_t rows, int64_t cols, int64_t ld, int64_t gc, uint8_t *q,
+                         void *scales, const float *partial, int np, float *sout, hipStream_t st) {
+  constexpr int KT = (KIND == KIND_MX || KIND == KIND_NV) ? 256 : 128;
+  const int64_t span = KIND == KIND_FP8 ? gc : KT;
+  const dim3 grid((unsigned)((rows + 8 * NC - 1) / (8 * NC)), (unsigned)((cols + span - 1) / span));
+  // 16-byte loads of 8 rows (bf16; fp32: two) need whole 8-row runs and
+  // aligned columns; rows past the end are masked 8 at a time
+  const bool vec = rows % 8 == 0 && ld % (16 / sizeof(T)) == 0 &&
+                   reinterpret_cast<uintptr_t>(x) % 16 == 0;
+  if (vec)
+    quant_trans_kernel<KIND, true, T, NC><<<grid, 32 * NC, 0, st>>>(x, rows, cols, ld, gc, q, scales,
+                                                                    partial, np, sout);
+  else
+    quant_trans_kernel<KIND, false, T, NC><<<grid, 32 * NC, 0, st>>>(x, rows, cols, ld, gc, q, scales,
+                                                                     partial, np, sout);
+}
+
+// FP8 scale groups the transposed kernel takes: 1 x gc with gc whole 128-column
+// tiles (or one group per row), 128 x 128.
+template <typename T>
+static bool launch_trans_fp8(const T *x, int64_t rows, int64_t cols, int64_t sr, int64_t sc,
+                             int64_t gr, int64_t gc, uint8_t *q, float *scales, hipStream_t st) {
+  if (!trans_ok(rows, cols, sr, sc)) return false;
+  if (gr == 1 && (gc % 128 == 0 || gc >= cols)) {
+    const int64_t g = gc >= cols ? (cols + 127) / 128 * 128 : gc;
+    launch_trans<KIND_FP8, 8>(x, rows, cols, sc, g, q, scales, nullptr, 0, nullptr, st);
+    return true;
+  }
+  if (gr == 128 && gc == 128) {
+    launch_trans<KIND_FP8, 16>(x, rows, cols, sc, gc, q, scales, nullptr, 0, nullptr, st);
+    return true;
+  }
+  return false;
 }
 
 template <int KIND, int T, int U>
@@ -649,6 +926,10 @@ static int partial_blocks(int64_t elems) {
 static hipError_t launch_amax_partials(const void *xv, bool f32, int64_t rows, int64_t cols,
                                        int64_t sr, int64_t sc, float *partial, int *nparts,
                                        hipStream_t st) {
+  if (trans_ok(rows, cols, sr, sc)) {   // the maximum of B[K, N] along its contiguous axis
+    std::swap(rows, cols);
+    std::swap(sr, sc);
+  }
   if (f32) {
     *nparts = partial_blocks(rows * cols);
     if (f32_vec_ok(xv, cols, sr, sc))
@@ -730,6 +1011,9 @@ hipError_t launch_quant_fp8_tensor(const void *xv, bool f32, int64_t rows, int64
     if (f32_vec_ok(xv, cols, sr, sc))
       launch_f32_rows<KIND_TENSOR, 1, 1>(static_cast<const float *>(xv), rows, cols, sr, q, nullptr,
                                          partial, np, scale, st);
+    else if (trans_ok(rows, cols, sr, sc))
+      launch_trans<KIND_TENSOR, 8>(static_cast<const float *>(xv), rows, cols, sc, 128, q, nullptr,
+                                   partial, np, scale, st);
     else
       quant_fp8_tensor_kernel<false, float><<<grid_for(rows * cols, 256 * 16), 256, 0, st>>>(
           static_cast<const float *>(xv), rows, cols, sr, sc, partial, np, q, scale);
@@ -741,6 +1025,8 @@ hipError_t launch_quant_fp8_tensor(const void *xv, bool f32, int64_t rows, int64
   else if (vec_ok(x, cols, sr, sc))
     quant_fp8_tensor_kernel<true, uint16_t><<<grid_for(rows * cols / 8, 256 * 4), 256, 0, st>>>(
         x, rows, cols, sr, sc, partial, np, q, scale);
+  else if (trans_ok(rows, cols, sr, sc))
+    launch_trans<KIND_TENSOR, 8>(x, rows, cols, sc, 128, q, nullptr, partial, np, scale, st);
   else
     quant_fp8_tensor_kernel<false, uint16_t><<<grid_for(rows * cols, 256 * 16), 256, 0, st>>>(
         x, rows, cols, sr, sc, partial, np, q, scale);
@@ -771,6 +1057,7 @@ hipError_t launch_quant_fp8_blocks(const void *xv, bool f32, int64_t rows, int64
       }
       return hipGetLastError();
     }
+    if (launch_trans_fp8(xf, rows, cols, sr, sc, gr, gc, q, scales, st)) return hipGetLastError();
     if (gr == 1 && gc <= 256)
       quant_group_scalar_kernel<KIND_FP8, float><<<grid_for(tiles, 256), 256, 0, st>>>(
           xf, rows, cols, sr, sc, gc, q, scales, nullptr, 0, nullptr);
@@ -800,6 +1087,7 @@ hipError_t launch_quant_fp8_blocks(const void *xv, bool f32, int64_t rows, int64
     }
     return hipGetLastError();
   }
+  if (!vec && launch_trans_fp8(x, rows, cols, sr, sc, gr, gc, q, scales, st)) return hipGetLastError();
   if (gr == 1 && !vec && gc <= 256) {
     quant_group_scalar_kernel<KIND_FP8, uint16_t><<<grid_for(tiles, 256), 256, 0, st>>>(
         x, rows, cols, sr, sc, gc, q, scales, nullptr, 0, nullptr);
@@ -841,6 +1129,8 @@ hipError_t launch_quant_mxfp4(const void *xv, bool f32, int64_t rows, int64_t co
     if (f32_vec_ok(xv, cols, sr, sc))
       launch_f32_rows<KIND_MX, 4, 1>(static_cast<const float *>(xv), rows, cols, sr, q, e8m0,
                                      nullptr, 0, nullptr, st);
+    else if (trans_ok(rows, cols, sr, sc))
+      launch_trans<KIND_MX, 8>(static_cast<const float *>(xv), rows, cols, sc, 256, q, e8m0, nullptr, 0, nullptr, st);
     else
       quant_group_scalar_kernel<KIND_MX, float><<<grid_for(rows * (cols / 32), 256), 256, 0, st>>>(
           static_cast<const float *>(xv), rows, cols, sr, sc, 32, q, e8m0, nullptr, 0, nullptr);
@@ -851,6 +1141,8 @@ hipError_t launch_quant_mxfp4(const void *xv, bool f32, int64_t rows, int64_t co
     launch_packed<KIND_MX, 4, 4, 4>(x, rows, cols, q, e8m0, nullptr, 0, nullptr, st);
   } else if (vec_ok(x, cols, sr, sc)) {
     launch_team<KIND_MX, 4>(x, rows, cols, sr, q, e8m0, nullptr, 0, nullptr, st);
+  } else if (trans_ok(rows, cols, sr, sc)) {
+    launch_trans<KIND_MX, 8>(x, rows, cols, sc, 256, q, e8m0, nullptr, 0, nullptr, st);
   } else {
     const int64_t ngroups = rows * (cols / 32);
     quant_group_scalar_kernel<KIND_MX, uint16_t><<<grid_for(ngroups, 256), 256, 0, st>>>(
@@ -869,6 +1161,8 @@ hipError_t launch_quant_nvfp4(const void *xv, bool f32, int64_t rows, int64_t co
     if (f32_vec_ok(xv, cols, sr, sc))
       launch_f32_rows<KIND_NV, 2, 1>(static_cast<const float *>(xv), rows, cols, sr, q, e4m3s,
                                      partial, np, gscale, st);
+    else if (trans_ok(rows, cols, sr, sc))
+      launch_trans<KIND_NV, 8>(static_cast<const float *>(xv), rows, cols, sc, 256, q, e4m3s, partial, np, gscale, st);
     else
       quant_group_scalar_kernel<KIND_NV, float><<<grid_for(rows * (cols / 16), 256), 256, 0, st>>>(
           static_cast<const float *>(xv), rows, cols, sr, sc, 16, q, e4m3s, partial, np, gscale);
@@ -879,6 +1173,8 @@ hipError_t launch_quant_nvfp4(const void *xv, bool f32, int64_t rows, int64_t co
     launch_packed<KIND_NV, 2, 1, 2>(x, rows, cols, q, e4m3s, partial, np, gscale, st);
   } else if (vec_ok(x, cols, sr, sc)) {
     launch_team<KIND_NV, 2>(x, rows, cols, sr, q, e4m3s, partial, np, gscale, st);
+  } else if (trans_ok(rows, cols, sr, sc)) {
+    launch_trans<KIND_NV, 8>(x, rows, cols, sc, 256, q, e4m3s, partial, np, gscale, st);
   } else {
     const int64_t ngroups = rows * (cols / 16);
     quant_group_scalar_kernel<KIND_NV, uint16_t><<<grid_for(ngroups, 256), 256, 0, st>>>(

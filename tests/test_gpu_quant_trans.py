@@ -1,0 +1,67 @@
+"""Quantizers on [K, N] sources (the reference's B, read as its [N, K] view):
+the transposed-tile kernels, bit for bit against the oracle, at the edges of
+their 64- and 128-row x 128- and 256-column tiles."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import quant as OQ
+from dsl_tool_amd import quant as Q
+from tests.util import np_f32, np_u8
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+# rows (N), columns (K)
+SHAPES = [(2, 32), (8, 128), (63, 96), (64, 128), (65, 160), (72, 256), (127, 288), (128, 512),
+          (136, 544), (200, 1056), (513, 128)]
+
+
+def _source(r, c, dt, pad, off):
+    """([r, c] view with unit row stride on the GPU, its values in fp32)."""
+    g = torch.Generator().manual_seed(1000 * r + c + pad)
+    x = torch.randn((c, r), generator=g) * torch.exp(torch.empty((1, r)).uniform_(-3, 3, generator=g))
+    x = torch.where(torch.rand((c, r), generator=g) < 2e-3, x * 50, x)
+    x[:, r // 2] = 0.0                         # an all-zero row: the scale floors
+    x = x.to(dt)
+    buf = torch.zeros(c * (r + pad) + off, dtype=dt, device=DEV)
+    view = buf[off:].view(c, r + pad)[:, :r]
+    view.copy_(x)
+    return view.t(), x.t().float().contiguous().numpy()
+
+
+@pytest.mark.parametrize("r,c", SHAPES)
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("pad,off", [(0, 0), (8, 0), (3, 1)])
+def test_transposed_sources_match_oracle(r, c, dt, pad, off):
+    x, ref = _source(r, c, dt, pad, off)
+    q, s = Q.quant_fp8_tensor(x)
+    q_ref, s_ref = OQ.quant_fp8_per_tensor(ref)
+    assert np_f32(s)[0] == s_ref and np.array_equal(np_u8(q), q_ref)
+    for gr, gc in ((1, 128), (1, 256), (1, c), (128, 128)):
+        q, s = Q.quant_fp8_blocks(x, gr, gc)
+        q_ref, s_ref = OQ.quant_fp8_blockwise(ref, gr, gc)
+        assert np.array_equal(np_f32(s), s_ref), (gr, gc)
+        assert np.array_equal(np_u8(q), q_ref), (gr, gc)
+    q, s = Q.quant_mxfp4(x)
+    q_ref, s_ref = OQ.quant_mxfp4(ref)
+    assert np.array_equal(np_u8(s), s_ref) and np.array_equal(np_u8(q), q_ref)
+    q, s, sg = Q.quant_nvfp4(x)
+    q_ref, s_ref, sg_ref = OQ.quant_nvfp4(ref)
+    assert np_f32(sg)[0] == sg_ref
+    assert np.array_equal(np_u8(s), s_ref) and np.array_equal(np_u8(q), q_ref)
+
+
+@pytest.mark.parametrize("c", [40, 130, 272])
+def test_transposed_sources_odd_columns(c):
+    """Code rows of no whole 16 bytes (FP8 any K; NVFP4 an odd number of blocks)."""
+    x, ref = _source(72, c, torch.bfloat16, 0, 0)
+    for gr, gc in ((1, 128), (128, 128)):
+        q, s = Q.quant_fp8_blocks(x, gr, gc)
+        q_ref, s_ref = OQ.quant_fp8_blockwise(ref, gr, gc)
+        assert np.array_equal(np_f32(s), s_ref) and np.array_equal(np_u8(q), q_ref)
+    if c % 16 == 0:
+        q, s, sg = Q.quant_nvfp4(x)
+        q_ref, s_ref, sg_ref = OQ.quant_nvfp4(ref)
+        assert np_f32(sg)[0] == sg_ref
+        assert np.array_equal(np_u8(s), s_ref) and np.array_equal(np_u8(q), q_ref)
