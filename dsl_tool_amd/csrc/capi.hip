@@ -431,7 +431,7 @@ LoraPlan lora_plan(int64_t m, int64_t n, int64_t k, int64_t lr) {
   p.ld2 = (2 * lr + 63) / 64 * 64;
   // T^T = A^T X^T on the streaming kernel when the adapter columns are few
   // enough to be its skinny M; its epilogue writes hi | lo itself.
-  p.tt = lr <= 256 && dsl::stream_supported(dsl::MODE_BF16, (int)lr, (int)m, (int)k, (int)(2 * k), true);
+  p.tt = lr <= 256 && (k % 128 == 0 || k % 64 != 0) && dsl::stream_supported(dsl::MODE_BF16, (int)lr, (int)m, (int)k, (int)(2 * k), true);
   // One pass (the adapter term as a second K segment of the persistent
   // kernel) unless both the base GEMM and the adapter add would take the
   // streaming kernel or the 128x128 pipelined tiles (up to 1024 rows at

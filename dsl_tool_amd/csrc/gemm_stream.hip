@@ -44,15 +44,29 @@
 // LDS rows are CHUNK bytes; row r's 16-byte chunk c sits in slot c ^ r
 // (r < 16), so the 16 lanes that read one logical chunk of 16 rows hit
 // distinct bank groups.
+//
+// Ragged rows (TAIL): any K of whole 16-byte chunks, and scale rows of any
+// pitch.  The last chunk of a row is partly past K: its copies re-read the
+// row's last 16 bytes and the fragments read from them are replaced by zero
+// in registers (A and W both, so that no byte past K reaches a product).
+// FP8 group scales move 4 bytes per lane; E8M0 / E4M3 scale rows, which then
+// start at any byte, move as the aligned words that cover them and are
+// shifted into place where they are read (v_alignbyte).  The selects cost a
+// few VALU operations per fragment of a kernel that waits for memory; these
+// shapes used to take the register-staged split-K tiles.  N=4096, K=4224, us
+// before -> now: M=16 block 12.2 -> 6.6, MXFP4 13.4 -> 5.2, NVFP4 26.2 -> 7.5,
+// per-tensor 11.4 -> 6.1; M=1 per-tensor 10.3 -> 5.5 (K=4160: 10.1 -> 5.8);
+// M=256 MXFP4 76.3 -> 12.4.
 #include <cstdlib>
 
 #include "stream_core.h"
 
 namespace dsl {
 
-template <int MODE_, int TMA_, int TN_, int CHUNK_, int NR_>
+template <int MODE_, int TMA_, int TN_, int CHUNK_, int NR_, bool TAIL_ = false>
 struct StreamCfg {
   static constexpr int MODE = MODE_;
+  static constexpr bool TAIL = TAIL_;                // ragged K / unaligned scale rows
   static constexpr int TMA = TMA_, TN = TN_;         // 16-row activation / W tiles
   static constexpr int BM = 16 * TMA, BN = 16 * TN;
   static constexpr int NW = 4, NT = NW * 64;         // waves split K
@@ -70,9 +84,12 @@ struct StreamCfg {
   // scale bytes per row per chunk: E8M0 per 32 elements, fp32 per 128-K
   // group, E4M3 per 16 elements
   static constexpr int SROW = MX ? CHUNK / 16 : (BLOCK ? 4 * STEPS : (NV ? CHUNK / 8 : 0));
-  static constexpr bool SC16 = SROW >= 16;           // scales move 16 (else 4) bytes per lane
-  static constexpr int AUX = SROW ? (SC16 ? 1024 : 256) : 0;
-  static constexpr int DPI = DATA_DMA + (AUX ? 1 : 0);   // direct loads per item
+  static constexpr bool SC16 = SROW >= 16 && !TAIL;  // scales move 16 (else 4) bytes per lane
+  // TAIL, byte scales: the SW aligned words that cover a row's SROW bytes
+  static constexpr bool SCU = TAIL && (MX || NV);
+  static constexpr int SW = SROW / 4 + 1, SCU_DMA = SCU ? (16 * SW + 63) / 64 : 0;
+  static constexpr int AUX = SROW ? (SCU ? SCU_DMA * 256 : (SC16 ? 1024 : 256)) : 0;
+  static constexpr int DPI = DATA_DMA + (SCU ? SCU_DMA : (AUX ? 1 : 0));   // direct loads per item
   static constexpr int REGION = 16 * CHUNK + AUX;
   static constexpr int NR = NR_;                     // regions per wave
   static constexpr int P = TN + TMA;                 // items per chunk: W tiles, then A tiles
@@ -83,6 +100,7 @@ struct StreamCfg {
   static constexpr int LDS = RING > RED + TILE ? RING : RED + TILE;
   static constexpr int CPT = BM * BN / NT;           // output columns per thread
   static_assert(CHUNK == 256 || CHUNK == 512, "chunk bytes");
+  static_assert(!TAIL || CHUNK == 256, "ragged rows use the 256-byte chunks");
   static_assert(!MX || CHUNK >= 256, "whole MXFP4 superblocks");
   static_assert(LDS <= 160 * 1024, "LDS budget");
   static_assert(NR >= 2 && (NR - 1) * DPI < 64, "vmcnt range");
@@ -115,12 +133,12 @@ DSL_DEV void stream_tile(const GemmArgs &p, const int m0, const int n0, const fl
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, g = lane >> 4;
-  const int nchunks = p.Kb / CHUNK;
+  const int nchunks = Cfg::TAIL ? (p.Kb + CHUNK - 1) / CHUNK : p.Kb / CHUNK;
   const int c_begin = nchunks * wave / NW, c_end = nchunks * (wave + 1) / NW;
   const int nitems = (c_end - c_begin) * P;
   uint8_t *my = lds + wave * NR * Cfg::REGION;
   const uint32_t R0 = dec::lds_addr(my);
-  const int nkg = p.K / 128;                 // FP8 block: scale groups per row
+  const int nkg = (p.K + 127) / 128;         // FP8 block: scale groups per row
   const int64_t sld = p.K / 32;              // MXFP4: E8M0 bytes per row
   // GATHER: the activation row each of the lane's direct loads reads, per
   // activation tile, as loaded; clamped and scaled to a byte offset only
@@ -163,11 +181,28 @@ DSL_DEV void stream_tile(const GemmArgs &p, const int m0, const int n0, const fl
           roff = (tok >= (uint32_t)xrows ? (uint32_t)xrows - 1 : tok) * (uint32_t)p.Kb;
         }
       }
-      const uint8_t *s = src + roff + kb0 + ((slot ^ r) << 4);
+      int64_t koff = kb0 + ((slot ^ r) << 4);
+      if constexpr (Cfg::TAIL) koff = koff < p.Kb ? koff : p.Kb - 16;   // past K: the last chunk again
+      const uint8_t *s = src + roff + koff;
       if (isW) dec::dma16_nt(s, dst + j * 1024);
       else dec::dma16(s, dst + j * 1024);
     }
-    if constexpr (Cfg::AUX) {
+    if constexpr (Cfg::SCU) {
+      // row r's scale bytes of the chunk as SW aligned words from the one
+      // holding the first byte, at aux + r*SW*4; words past the array re-read
+      // its last one (their bytes belong to blocks past K)
+      const int64_t pitch = Cfg::MX ? p.K / 32 : p.K / 16;
+      const uintptr_t sc0 = reinterpret_cast<uintptr_t>(isW ? p.sb : p.sa);
+      const uintptr_t end = (sc0 + (uintptr_t)((int64_t)(rlim + 1) * pitch) - 1) & ~(uintptr_t)3;
+#pragma unroll
+      for (int d = 0; d < Cfg::SCU_DMA; ++d) {
+        const int idx = d * 64 + lane, r = min(idx / Cfg::SW, 15), w = idx % Cfg::SW;
+        const int row = min(rbase + r, rlim);
+        const uintptr_t a =
+            ((sc0 + (uintptr_t)((int64_t)row * pitch + (int64_t)ch * SROW)) & ~(uintptr_t)3) + 4 * w;
+        dec::dma4(reinterpret_cast<const void *>(a < end ? a : end), dst + 16 * CHUNK + d * 256);
+      }
+    } else if constexpr (Cfg::AUX) {
       // the item's scales, row r at aux + r*SROW: 16-byte parts (lanes past
       // 16 rows repeat) or, with 8 bytes per row, 4-byte words
       constexpr int PARTS = Cfg::SC16 ? SROW / 16 : SROW / 4;
@@ -180,7 +215,7 @@ DSL_DEV void stream_tile(const GemmArgs &p, const int m0, const int n0, const fl
           // lane -> column lane % 16, group lane / 16 (repeated past STEPS),
           // stored [group][column]; 16 lanes read 64 contiguous bytes
           const int col = min(rbase + (lane & 15), rlim);
-          const int grp = ch * Cfg::STEPS + ((lane >> 4) & (Cfg::STEPS - 1));
+          const int grp = min(ch * Cfg::STEPS + ((lane >> 4) & (Cfg::STEPS - 1)), nkg - 1);
           dec::dma4(static_cast<const float *>(p.sb) + (int64_t)grp * p.N + col, dst + 16 * CHUNK);
           return;
         }
@@ -194,6 +229,10 @@ DSL_DEV void stream_tile(const GemmArgs &p, const int m0, const int n0, const fl
             isW ? static_cast<const float *>(p.sb) + (int64_t)(row / 128) * nkg
                 : static_cast<const float *>(p.sa) + (int64_t)row * nkg) +
              (int64_t)ch * Cfg::STEPS * 4;
+        if constexpr (Cfg::TAIL) {           // groups past K: the last one again
+          const int over = ch * Cfg::STEPS + part - (nkg - 1);
+          sc -= 4 * (over > 0 ? over : 0);
+        }
       }
       if constexpr (Cfg::SC16) dec::dma16(sc + part * 16, dst + 16 * CHUNK);
       else dec::dma4(sc + part * 4, dst + 16 * CHUNK);
@@ -206,8 +245,37 @@ DSL_DEV void stream_tile(const GemmArgs &p, const int m0, const int n0, const fl
 #pragma unroll
     for (int a = 0; a < TMA; ++a) st.acc[t][a] = (v4f){0.f, 0.f, 0.f, 0.f};
 
+  int vch = CHUNK / 16;              // TAIL: 16-byte chunks of the item that exist
+  int64_t cur = 0;                   // TAIL: the item's chunk
   auto chunk16 = [&](const uint8_t *base, int c) {      // row r16's logical chunk c
-    return *reinterpret_cast<const v4i *>(base + r16 * CHUNK + ((c ^ r16) << 4));
+    v4i v = *reinterpret_cast<const v4i *>(base + r16 * CHUNK + ((c ^ r16) << 4));
+    if constexpr (Cfg::TAIL) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = c < vch ? v[i] : 0;
+    }
+    return v;
+  };
+  // TAIL, byte scales: bytes 4w .. 4w+3 of row r16's scales of the item
+  // (first byte of the row's words: its address modulo 4)
+  auto scale_word = [&](const uint8_t *aux, int w, bool isW, int kind) {
+    const int64_t pitch = Cfg::MX ? p.K / 32 : p.K / 16;
+    const int row = isW ? min(n0 + kind * 16 + r16, p.N - 1) : min(m0 + (kind - TN) * 16 + r16, p.M - 1);
+    const uint32_t sh = (uint32_t)(reinterpret_cast<uintptr_t>(isW ? p.sb : p.sa) +
+                                   (uintptr_t)(row * pitch + cur * SROW)) & 3;
+    const uint32_t *q = reinterpret_cast<const uint32_t *>(aux) + r16 * Cfg::SW + w;
+    return __builtin_amdgcn_alignbyte(q[1], q[0], sh);
+  };
+  // MXFP4: the E8M0 word of lane group g; blocks past K get 2^0 (their codes are 0)
+  auto mx_word = [&](const uint8_t *aux, bool isW, int kind) {
+    const uint32_t w = scale_word(aux, g, isW, kind);
+    const int nv = vch - 4 * g;      // 16-byte chunk = one block
+    const uint32_t mask = nv >= 4 ? 0xffffffffu : (nv <= 0 ? 0u : (1u << (8 * nv)) - 1);
+    return (int)((w & mask) | (0x7f7f7f7fu & ~mask));
+  };
+  // NVFP4: the two E4M3 scales of chunk c (0 past K: a code of NaN must not reach it)
+  auto nv_pair = [&](const uint8_t *aux, int c, bool isW, int kind) {
+    const uint32_t w = scale_word(aux, c >> 1, isW, kind) >> (16 * (c & 1));
+    return c < vch ? w & 0xffffu : 0u;
   };
 
   auto consume = [&](auto kind_tag, const uint8_t *base) {
@@ -219,7 +287,8 @@ DSL_DEV void stream_tile(const GemmArgs &p, const int m0, const int n0, const fl
         for (int b = 0; b < Cfg::SBK; ++b) {
 #pragma unroll
           for (int j = 0; j < 4; ++j) st.wq[KIND][b][j] = chunk16(base, b * 16 + 4 * g + j);
-          st.ws[KIND][b] = *reinterpret_cast<const int *>(aux + r16 * SROW + b * 16 + g * 4);
+          if constexpr (Cfg::SCU) st.ws[KIND][b] = mx_word(aux, true, KIND);
+          else st.ws[KIND][b] = *reinterpret_cast<const int *>(aux + r16 * SROW + b * 16 + g * 4);
         }
       } else if constexpr (Cfg::NV) {
         // superblock b: lane group g takes 16-byte chunk 4b + g and its two
@@ -228,7 +297,8 @@ DSL_DEV void stream_tile(const GemmArgs &p, const int m0, const int n0, const fl
         for (int b = 0; b < Cfg::NSB; ++b) {
           const int c = 4 * b + g;
           st.wn[KIND][b] = chunk16(base, c);
-          st.wsn[KIND][b] = *reinterpret_cast<const uint16_t *>(aux + r16 * SROW + 2 * c);
+          if constexpr (Cfg::SCU) st.wsn[KIND][b] = nv_pair(aux, c, true, KIND);
+          else st.wsn[KIND][b] = *reinterpret_cast<const uint16_t *>(aux + r16 * SROW + 2 * c);
         }
       } else {
 #pragma unroll
@@ -255,8 +325,10 @@ DSL_DEV void stream_tile(const GemmArgs &p, const int m0, const int n0, const fl
         for (int b = 0; b < Cfg::NSB; ++b) {
           const int c = 4 * b + g;
           const v4i ad = chunk16(base, c);
-          const v2h as2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(
-              (uint32_t)*reinterpret_cast<const uint16_t *>(aux + r16 * SROW + 2 * c), 1.0f, false);
+          uint32_t asw;
+          if constexpr (Cfg::SCU) asw = nv_pair(aux, c, false, KIND);
+          else asw = *reinterpret_cast<const uint16_t *>(aux + r16 * SROW + 2 * c);
+          const v2h as2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(asw, 1.0f, false);
           v2h ws2[TN];
 #pragma unroll
           for (int t = 0; t < TN; ++t)
@@ -274,7 +346,9 @@ DSL_DEV void stream_tile(const GemmArgs &p, const int m0, const int n0, const fl
       } else if constexpr (Cfg::MX) {
 #pragma unroll
         for (int b = 0; b < Cfg::SBK; ++b) {
-          const int asv = *reinterpret_cast<const int *>(aux + r16 * SROW + b * 16 + g * 4);
+          int asv;
+          if constexpr (Cfg::SCU) asv = mx_word(aux, false, KIND);
+          else asv = *reinterpret_cast<const int *>(aux + r16 * SROW + b * 16 + g * 4);
           v4i ad[4];
 #pragma unroll
           for (int j = 0; j < 4; ++j) ad[j] = chunk16(base, b * 16 + 4 * g + j);
@@ -340,6 +414,11 @@ DSL_DEV void stream_tile(const GemmArgs &p, const int m0, const int n0, const fl
       // the region of item it-1 is free (its reads returned): refill it
       if (it + NR - 1 < nitems) issue(it + NR - 1);
       wait_item(nitems - 1 - it);
+      if constexpr (Cfg::TAIL) {
+        cur = c_begin + it / P;
+        const int left = (p.Kb - (int)cur * CHUNK) / 16;
+        vch = left < CHUNK / 16 ? left : CHUNK / 16;
+      }
       consume(kind_tag, my + (it % NR) * Cfg::REGION);
       dec::wait_lds();
     };
@@ -532,17 +611,34 @@ struct StreamPlan {
 };
 
 // Activation tiles by M (16, 32 or 64 rows per workgroup; 256-byte chunks
-// for the skinny ones, 512-byte chunks otherwise; rows of an odd number of
-// 256-byte chunks take the 32-row tiles), and the most W tiles
+// for the skinny ones, 512-byte chunks otherwise; whole rows of an odd number
+// of 256-byte chunks take the 32-row tiles), and the most W tiles
 // per workgroup (4, 2, 1) that still leave >= 192 workgroups: fewer but
 // larger workgroups read A and W fewer times (measured at M = 96..256), as
 // long as they cover most CUs.  DSL_GEMM_STREAM_TMA / DSL_GEMM_STREAM_TN
 // override them (tuning).
-StreamPlan plan_for(int mode, int M, int N, int Kb) {
+// K whose rows (or scale rows) take the TAIL form of the kernel: rows of no
+// whole 256-byte chunks, FP8 / MXFP4 scale rows of no whole 16 bytes (K %
+// 512), NVFP4 ones (K % 256), or scale arrays that are not 16-byte aligned;
+// and, from 97 rows, rows of an odd number of 256-byte chunks, for its
+// 64-row blocks (bf16 M=256 N=4096 K=4224: 22 us, on the 128x128 tiles 37).
+bool needs_tail(int mode, int M, int K, int Kb, bool scales16) {
+  if (Kb % 256 != 0 || (Kb % 512 != 0 && M > 96)) return true;
+  if (mode_grouped_k(mode) || mode == MODE_MXFP4) return !scales16 || K % 512 != 0;
+  if (mode == MODE_NVFP4) return !scales16 || K % 256 != 0;
+  return false;
+}
+
+bool stream_rows64(int M, int Kb, bool tail) { return tail ? M > 96 : Kb % 512 == 0; }
+
+StreamPlan plan_for(int mode, int M, int N, int Kb, bool tail) {
   StreamPlan pl;
-  pl.tma = M <= 16 ? 1 : ((M <= 32 || Kb % 512 != 0) ? 2 : 4);
+  // Ragged rows take the 64-row blocks from 97 rows (in 256-byte chunks):
+  // K = 4160, N = 4096: M = 64 per-tensor 8.5 us in 32-row blocks against
+  // 9.8, block 9.5 against 12.4; M = 128 level, M = 256 bf16 24.2 against 33.2.
+  pl.tma = M <= 16 ? 1 : ((M <= 32 || !stream_rows64(M, Kb, tail)) ? 2 : 4);
   const char *et = getenv("DSL_GEMM_STREAM_TMA");
-  const bool force_tma = et && (et[0] == '1' || et[0] == '2' || (et[0] == '4' && Kb % 512 == 0)) && !et[1];
+  const bool force_tma = et && (et[0] == '1' || et[0] == '2' || (et[0] == '4' && (tail || Kb % 512 == 0))) && !et[1];
   if (force_tma) pl.tma = et[0] - '0';
   const int64_t nmb = (M + 16 * pl.tma - 1) / (16 * pl.tma);
   pl.tn = 1;
@@ -568,9 +664,9 @@ StreamPlan plan_for(int mode, int M, int N, int Kb) {
   return pl;
 }
 
-template <int MODE, int TMA, int TN, int CHUNK>
+template <int MODE, int TMA, int TN, int CHUNK, bool TAIL = false>
 hipError_t launch_cfg(const GemmArgs &p, hipStream_t st) {
-  using Cfg = StreamCfg<MODE, TMA, TN, CHUNK, 4>;
+  using Cfg = StreamCfg<MODE, TMA, TN, CHUNK, 4, TAIL>;
   const int nmb = (p.M + Cfg::BM - 1) / Cfg::BM;
   const int nnb = (p.N + Cfg::BN - 1) / Cfg::BN;
   const int grid = 8 * nmb * ((nnb + 7) / 8);
@@ -578,28 +674,34 @@ hipError_t launch_cfg(const GemmArgs &p, hipStream_t st) {
   return hipGetLastError();
 }
 
-template <int MODE, int TMA, int CHUNK>
+template <int MODE, int TMA, int CHUNK, bool TAIL = false>
 hipError_t launch_tn(const GemmArgs &p, int tn, hipStream_t st) {
-  if (tn == 1) return launch_cfg<MODE, TMA, 1, CHUNK>(p, st);
+  if (tn == 1) return launch_cfg<MODE, TMA, 1, CHUNK, TAIL>(p, st);
   // four W tiles beside four activation tiles exceed the registers of the
   // FP8 block and NVFP4 forms (plan_for never asks for them)
   constexpr bool four = !(TMA == 4 && (mode_grouped_k(MODE) || MODE == MODE_NVFP4));
   if constexpr (four) {
-    if (tn == 4) return launch_cfg<MODE, TMA, 4, CHUNK>(p, st);
+    if (tn == 4) return launch_cfg<MODE, TMA, 4, CHUNK, TAIL>(p, st);
   }
-  return launch_cfg<MODE, TMA, 2, CHUNK>(p, st);
+  return launch_cfg<MODE, TMA, 2, CHUNK, TAIL>(p, st);
 }
 
 template <int MODE>
 hipError_t launch_mode(const GemmArgs &p, const StreamPlan &pl, hipStream_t st) {
+  const uintptr_t sc = reinterpret_cast<uintptr_t>(p.sa) | reinterpret_cast<uintptr_t>(p.sb);
+  if (needs_tail(MODE, p.M, p.K, p.Kb, (sc & 15) == 0)) {
+    if (pl.tma == 1) return launch_tn<MODE, 1, 256, true>(p, pl.tn, st);
+    if (pl.tma == 2) return launch_tn<MODE, 2, 256, true>(p, pl.tn, st);
+    return launch_tn<MODE, 4, 256, true>(p, pl.tn, st);
+  }
   if (pl.tma == 1) return launch_tn<MODE, 1, 256>(p, pl.tn, st);
   if (pl.tma == 2) return launch_tn<MODE, 2, 256>(p, pl.tn, st);
   return launch_tn<MODE, 4, 512>(p, pl.tn, st);
 }
 
-template <int TMA, int TN, int CHUNK>
+template <int TMA, int TN, int CHUNK, bool TAIL>
 hipError_t launch_grouped_cfg(const GroupedArgs &gp, hipStream_t st) {
-  using Cfg = StreamCfg<MODE_FP8_TENSOR, TMA, TN, CHUNK, 4>;
+  using Cfg = StreamCfg<MODE_FP8_TENSOR, TMA, TN, CHUNK, 4, TAIL>;
   const int64_t nnb = (gp.N + Cfg::BN - 1) / Cfg::BN;
   const int64_t blocks = (gp.rows + Cfg::BM - 1) / Cfg::BM + gp.G;   // >= sum of per-group blocks
   const int64_t grid = blocks * nnb;
@@ -615,7 +717,7 @@ hipError_t launch_grouped_cfg(const GroupedArgs &gp, hipStream_t st) {
 
 bool grouped_stream_supported(const GroupedArgs &gp) {
   if (gp.arow && (gp.xrows < 1 || (int64_t)gp.xrows * gp.K >= ((int64_t)1 << 32))) return false;
-  return gp.G >= 1 && gp.G <= kMaxGroups && gp.K % 256 == 0 && gp.K >= 256 && gp.N >= 1;
+  return gp.G >= 1 && gp.G <= kMaxGroups && gp.K % 16 == 0 && gp.K >= 16 && gp.N >= 1;
 }
 
 // Row blocks of 16 or 32 rows by the groups' average size (the router sends
@@ -629,26 +731,30 @@ bool grouped_stream_supported(const GroupedArgs &gp) {
 // rows per group (384 tokens: 62.2 against 62.7 us).
 hipError_t launch_grouped_stream(const GroupedArgs &gp, hipStream_t st) {
   if (!grouped_stream_supported(gp)) return hipErrorInvalidValue;
-  if (gp.rows / gp.G <= 4) return launch_grouped_cfg<1, 4, 256>(gp, st);
-  return launch_grouped_cfg<2, 4, 256>(gp, st);
+  const bool few = gp.rows / gp.G <= 4;
+  if (gp.K % 256 != 0)               // the last 256-byte chunk of a row is partial
+    return few ? launch_grouped_cfg<1, 4, 256, true>(gp, st) : launch_grouped_cfg<2, 4, 256, true>(gp, st);
+  return few ? launch_grouped_cfg<1, 4, 256, false>(gp, st) : launch_grouped_cfg<2, 4, 256, false>(gp, st);
 }
 
-bool stream_supported(int mode, int M, int N, int K, int Kb, bool scales16) {
+bool stream_supported(int mode, int M, int N, int K, int Kb, bool scales4) {
   if (M < 1 || M > 1024 || N < 1) return false;
-  if (Kb % 256 != 0) return false;   // 512-byte chunks where they fit, else 256
-  if (mode == MODE_FP8_TENSOR || mode == MODE_BF16) return true;
-  // block scales and E8M0 rows move by 16-byte direct loads (K % 512)
-  if (mode_grouped_k(mode) || mode == MODE_MXFP4) return scales16 && K % 512 == 0;
-  // E4M3 rows (K/16 bytes) move by 16-byte direct loads
-  if (mode == MODE_NVFP4) return scales16 && K % 256 == 0;
-  return false;
+  if (Kb < 16 || Kb % 16 != 0) return false;   // whole 16-byte chunks
+  if (mode_grouped_k(mode)) return scales4;     // fp32 scales move by 4-byte direct loads at least
+  // one E8M0 block, or two E4M3 ones, per 16-byte chunk
+  return (mode != MODE_MXFP4 && mode != MODE_NVFP4) || K % 32 == 0;
+}
+
+bool stream_blocks64(int mode, int M, int K, int Kb, bool scales16) {
+  return stream_rows64(M, Kb, needs_tail(mode, M, K, Kb, scales16));
 }
 
 hipError_t launch_gemm_stream(int mode, const GemmArgs &p, hipStream_t st) {
   if (p.lora_scales && (mode != MODE_BF16 || p.lora_rank < 1 || p.ldc < 2 * (int64_t)p.M))
     return hipErrorInvalidValue;
   if (p.accumulate && (!p.out_f32 || p.lora_scales)) return hipErrorInvalidValue;
-  const StreamPlan pl = plan_for(mode, p.M, p.N, p.Kb);
+  const uintptr_t sc = reinterpret_cast<uintptr_t>(p.sa) | reinterpret_cast<uintptr_t>(p.sb);
+  const StreamPlan pl = plan_for(mode, p.M, p.N, p.Kb, needs_tail(mode, p.M, p.K, p.Kb, (sc & 15) == 0));
   switch (mode) {
     case MODE_FP8_TENSOR: return launch_mode<MODE_FP8_TENSOR>(p, pl, st);
     case MODE_FP8_BLOCK: return launch_mode<MODE_FP8_BLOCK>(p, pl, st);

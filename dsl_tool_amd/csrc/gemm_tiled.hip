@@ -240,7 +240,7 @@ static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc1
     return (e && e[0] >= '1' && e[0] <= '9' && !e[1]) ? e[0] - '0' : -1;
   }();
   Route r{PATH_TILED, -1, plan_for(M, N, Kb)};
-  bool streamable = stream_on && stream_supported(mode, M, N, K, Kb, sc16);
+  bool streamable = stream_on && stream_supported(mode, M, N, K, Kb, sc4);
   // The streaming kernel's time grows with the number of 64-row activation
   // blocks times N (each block streams all of W, and each W slice re-reads
   // its activation rows), while the 128x128 / persistent tiles stay at about
@@ -255,7 +255,7 @@ static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc1
   const bool bf16_pipe_round = mode == MODE_BF16 && pipe_forced != -2 && Kb % 128 == 0 && M > 64 &&
                                N > 64 && t128 >= 40 && t128 <= device_cu_count();
   if (streamable && !skinny_stream && M > 32 && (mode != MODE_NVFP4 || M > 256)) {
-    const int bm = Kb % 512 == 0 ? 64 : 32;
+    const int bm = stream_blocks64(mode, M, K, Kb, sc16) ? 64 : 32;
     const int64_t span2 = 2 * (int64_t)((M + bm - 1) / bm) * N;   // twice the span
     // crossovers re-measured against the prefetching / eight-wave 128x128
     // tiles (same-box sweep, M = 256..1024, N = 2048..14336, K = 2048 and
@@ -401,7 +401,7 @@ hipError_t launch_gemm(int mode, GemmArgs p, hipStream_t st) {
   // the register-staged kernels
   if (p.accumulate) {
     if ((r.path == PATH_STREAM || r.path == PATH_DECODE || p.K <= kAccShortK) && p.out_f32 &&
-        stream_enabled() && stream_supported(mode, p.M, p.N, p.K, p.Kb, (sc & 15) == 0))
+        stream_enabled() && stream_supported(mode, p.M, p.N, p.K, p.Kb, (sc & 3) == 0))
       r.path = PATH_STREAM;
     else if (!(r.path == PATH_PIPE && p.out_f32 && !mode_grouped_k(mode)))
       r.path = PATH_TILED;

@@ -98,11 +98,12 @@ bool decode_supported(int mode, int M, int K, int Kb, bool scales4, bool scales1
 hipError_t launch_gemm_decode(int mode, const GemmArgs &p, hipStream_t st);
 
 // Streaming kernel for M <= 1024 (gemm_stream.hip), one launch, no
-// workspace, deterministic, Kb % 256 == 0: FP8_TENSOR and BF16; FP8_BLOCK,
-// FP8_GCOL and MXFP4 with 16-byte aligned scales and K % 512 == 0; NVFP4
-// with 16-byte aligned scales and K % 256 == 0.  The router takes it while
-// ceil(M/64) * N stays below a per-mode edge (gemm_tiled.hip, route_for).
-bool stream_supported(int mode, int M, int N, int K, int Kb, bool scales16);
+// workspace, deterministic, every mode and any Kb % 16 == 0 (FP8 group
+// scales 4-byte aligned).  The router takes it while ceil(M/64) * N stays
+// below a per-mode edge (gemm_tiled.hip, route_for).
+bool stream_supported(int mode, int M, int N, int K, int Kb, bool scales4);
+// Whether M > 32 rows stream in 64-row blocks, else in 32-row blocks.
+bool stream_blocks64(int mode, int M, int K, int Kb, bool scales16);
 hipError_t launch_gemm_stream(int mode, const GemmArgs &p, hipStream_t st);
 
 // Picks a kernel variant for the shape and launches it (plus the split-K
@@ -129,8 +130,8 @@ struct GroupedArgs {
   int out_f32;
   // gather form: x is [xrows][K] and sorted row r reads x row arow[r]
   // (persistent kernel, and the grouped streaming tiles; launch_grouped_fp8
-  // sends groups of fewer than 48 rows on average to the streaming tiles
-  // when K % 256 == 0, the rest to the persistent kernel)
+  // sends groups of fewer than 48 rows on average to the streaming tiles,
+  // the rest to the persistent kernel)
   const int32_t *arow = nullptr;
   int xrows = 0;
 };
@@ -138,7 +139,7 @@ hipError_t launch_grouped_fp8(GroupedArgs args, hipStream_t st);
 // Grouped FP8 on the persistent kernel (K % 128 == 0, K < 2^24).
 bool grouped_persist_supported(const GroupedArgs &args);
 hipError_t launch_grouped_persist(const GroupedArgs &args, hipStream_t st);
-// Grouped FP8 on the streaming tiles (few rows per group; K % 256 == 0).
+// Grouped FP8 on the streaming tiles (few rows per group; K % 16 == 0).
 bool grouped_stream_supported(const GroupedArgs &args);
 hipError_t launch_grouped_stream(const GroupedArgs &args, hipStream_t st);
 

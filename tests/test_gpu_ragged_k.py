@@ -1,0 +1,99 @@
+"""K that is no multiple of the kernels' 128- / 256-byte steps, on every mode:
+the last, partly filled step of a row must add nothing, and scale rows that
+start at any byte must reach their own blocks only."""
+import numpy as np
+import pytest
+import torch
+
+from dsl_tool_amd import gemm as G
+from dsl_tool_amd import quant as Q
+from dsl_tool_amd import workloads as W
+from tests.test_gpu_random_shapes import test_random_shape as check
+from tests.util import assert_close, np_f32
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+# K of 1..3 steps plus a remainder: one 16-byte chunk, half a step, one chunk short
+KS = {"tensor": (16, 272, 1152, 1280 + 112), "block": (16, 272, 1152, 1280 + 112),
+      "group": (16, 272, 1152, 1280 + 112), "mxfp4": (32, 544, 640, 1024 + 480),
+      "nvfp4": (32, 544, 640, 1024 + 480), "bf16": (8, 136, 1152, 1280 + 56)}
+
+
+@pytest.mark.parametrize("m", [1, 16, 17, 50, 100, 130])
+@pytest.mark.parametrize("mode", sorted(KS))
+def test_ragged_k_streamed(mode, m):
+    for k in KS[mode]:
+        check(mode, m, 200, k)
+        check(mode, m, 77, k)
+
+
+@pytest.mark.parametrize("m", [3, 40, 300])
+@pytest.mark.parametrize("mode", ["mxfp4", "nvfp4", "block", "group"])
+def test_nan_scales_stay_in_their_row(mode, m):
+    """A NaN scale of one row (its neighbours share the words that the copies
+    move) makes that row NaN and no other."""
+    n, k = 96, 544
+    a, w = W.randn_bf16((m, k), 1, 1.0).to(DEV), W.randn_bf16((n, k), 2, 0.02).to(DEV)
+    bad = m // 2
+    if mode in ("block", "group"):
+        qa, sa = Q.quant_fp8_blocks(a, 1, 128)
+        qw, sw = Q.quant_fp8_blocks(w, 128 if mode == "block" else 1, 128)
+        sw = sw if mode == "block" else sw.t().contiguous()
+        good = G.fp8_gemm_packed(qa, qw, sa, sw, block=mode == "block", group=mode == "group")
+        sa[bad] = float("nan")
+        c = G.fp8_gemm_packed(qa, qw, sa, sw, block=mode == "block", group=mode == "group")
+    elif mode == "mxfp4":
+        qa, sa = Q.quant_mxfp4(a)
+        qw, sw = Q.quant_mxfp4(w)
+        good = G.fp4_gemm_packed(qa, sa, qw, sw)
+        sa[bad] = 0xFF
+        c = G.fp4_gemm_packed(qa, sa, qw, sw)
+    else:
+        qa, sa, ga = Q.quant_nvfp4(a)
+        qw, sw, gw = Q.quant_nvfp4(w)
+        good = G.fp4_gemm_packed(qa, sa, qw, sw, fmt="nvfp4", global_a=ga, global_w=gw)
+        sa[bad] = 0x7F
+        c = G.fp4_gemm_packed(qa, sa, qw, sw, fmt="nvfp4", global_a=ga, global_w=gw)
+    rows = [i for i in range(m) if i != bad]
+    assert np.isnan(np_f32(c)[bad]).all()
+    assert torch.equal(c[rows], good[rows])
+
+
+@pytest.mark.parametrize("mode", ["mxfp4", "nvfp4"])
+def test_misaligned_scale_rows(mode):
+    """Scale arrays that start at an odd byte, over an aligned K."""
+    m, n, k = 20, 96, 1024
+    a, w = W.randn_bf16((m, k), 3, 1.0).to(DEV), W.randn_bf16((n, k), 4, 0.02).to(DEV)
+
+    def shifted(s):
+        buf = torch.zeros(s.numel() + 3, dtype=torch.uint8, device=DEV)
+        v = buf[3:].view(s.shape)
+        v.copy_(s)
+        return v
+
+    if mode == "mxfp4":
+        (qa, sa), (qw, sw) = Q.quant_mxfp4(a), Q.quant_mxfp4(w)
+        assert torch.equal(G.fp4_gemm_packed(qa, shifted(sa), qw, shifted(sw)),
+                           G.fp4_gemm_packed(qa, sa, qw, sw))
+    else:
+        (qa, sa, ga), (qw, sw, gw) = Q.quant_nvfp4(a), Q.quant_nvfp4(w)
+        kw = dict(fmt="nvfp4", global_a=ga, global_w=gw)
+        assert torch.equal(G.fp4_gemm_packed(qa, shifted(sa), qw, shifted(sw), **kw),
+                           G.fp4_gemm_packed(qa, sa, qw, sw, **kw))
+
+
+@pytest.mark.parametrize("k", [16, 144, 272, 1408])
+@pytest.mark.parametrize("counts", [(1, 0, 3, 2), (17, 5, 40, 1, 0)])
+def test_ragged_k_grouped_stream(counts, k):
+    """Groups of a few rows on the streaming tiles (and, where K is whole 128s, the row map)."""
+    g, n, t = len(counts), 136, sum(counts)
+    x, w = W.randn_bf16((t, k), 5).to(DEV), W.randn_bf16((g * n, k), 6, 0.02).to(DEV)
+    off = torch.tensor([0] + list(np.cumsum(counts)), dtype=torch.int32, device=DEV)
+    qx, sx = Q.quant_fp8_blocks(x, 1, k)
+    qw, sw = Q.quant_fp8_blocks(w, 1, k)
+    y = G.grouped_fp8_gemm_packed(qx, sx, qw.view(g, n, k), sw.view(g, n), off)
+    xd = qx.view(torch.float8_e4m3fn).double().cpu() * sx.double().cpu()
+    wd = (qw.view(torch.float8_e4m3fn).double().cpu() * sw.double().cpu()).view(g, n, k)
+    ref = torch.cat([xd[off[e]:off[e + 1]] @ wd[e].t() for e in range(g)])
+    assert_close(y, ref.float().numpy(), what=f"grouped stream {counts} K={k}")
