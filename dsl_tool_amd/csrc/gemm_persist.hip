@@ -52,6 +52,16 @@
 // significant bits, so the fp16 values are exact) and feeds 32x32x16 fp16
 // MFMAs; the fp32 global scales apply in the epilogue.
 //
+// Ragged K (RAG): K of whole 16-byte chunks but no whole pairs, or scale rows
+// that are no whole quads.  The copies of a row's last, partial pair re-read
+// its last chunk, and once that pair has landed its chunks past K are zeroed in
+// LDS, with one more barrier per tile (zeroing the fragments in registers
+// instead spilled in the loop).  FP8 block: a row's last scale quad
+// is the row's last 16 bytes, overlapping the quad before it; the readers take
+// their scale at its distance from the quad's first.  E8M0 / E4M3 scale rows
+// that are no whole quads are first copied to a padded pitch (gemm_tiled.hip;
+// overlapping quads there cost registers: 8-12 bytes of spill).
+//
 // Epilogue: each wave converts its accumulators (v_cvt_pk_bf16_f32),
 // regroups them across lanes (v_permlane32_swap, v_permlane16_swap) and
 // stores 16 bytes per lane, 16 rows x 64 contiguous bytes per store, straight
@@ -63,9 +73,10 @@
 
 namespace dsl {
 
-template <int MODE_, bool GROUPED_ = false, bool GATHER_ = false>
+template <int MODE_, bool GROUPED_ = false, bool GATHER_ = false, bool RAG_ = false>
 struct PersCfg {
   static constexpr int MODE = MODE_;
+  static constexpr bool RAG = RAG_;            // ragged K / scale rows
   static constexpr bool GROUPED = GROUPED_;    // FP8 grouped (MoE) tile walk
   static constexpr bool GATHER = GATHER_;      // grouped: A rows through a row table
   static constexpr int BM = 256, BN = 256, WGM = 2, WGN = 4;
@@ -98,6 +109,7 @@ struct PersCfg {
   static constexpr int DATA_DMA = A_DMA + B_DMA, SC_DMA = SA_DMA + SB_DMA;
   static constexpr int DD = DATA_DMA / NW, DS = (SC_DMA + NW - 1) / NW, D = DD + DS;
   static_assert(DATA_DMA % NW == 0 && A_DMA % DD == 0, "whole waves per operand");
+  static_assert(!RAG || NT == BM + BN, "one row per thread");
   static_assert(DS <= 1, "at most one scale DMA per wave and quad");
   static_assert(LDS <= 160 * 1024, "LDS budget");
   static_assert(!BLOCK || (WN <= 128 && 128 % WN == 0), "one weight-scale block per wave");
@@ -118,6 +130,16 @@ struct TileRef {
 };
 
 namespace pers {
+
+// bytes per scale row: fp32 per 128-K group, E8M0 per 32 elements, E4M3 per
+// 16 (or the pitch they were copied to)
+template <class Cfg>
+DSL_DEV int scale_row_bytes(const GemmArgs &p) {
+  if constexpr (Cfg::RAG) {
+    if constexpr (!Cfg::BLOCK) return p.sld;
+  }
+  return Cfg::BLOCK ? (p.K + 127) / 128 * 4 : (Cfg::MX ? p.K / 32 : p.K / 16);
+}
 
 // Pair-slot row swizzle: chunk c of row r lives in slot c ^ pair_swz(r).
 // Its readers (32x32 fragments: lane = row, chunks 4p + 2h and 4p + 2h + 1,
@@ -187,6 +209,8 @@ struct Ring {
   int lim;                       // last valid tile row of the operand (uniform)
   int kb;
   int kb2, nk1;                  // second segment: row stride, first pair
+  int lastq;                     // RAG: the row's last pair (partial)
+  int srowb;                     // RAG: bytes per scale row
   int rmask;                     // second segment: pair index mask (W2 repeating), else all ones
   uint32_t vsub;                 // lane's row within one DMA
   uint32_t vchunk;               // lane's chunk byte offset for even DMAs
@@ -200,6 +224,10 @@ struct Ring {
                       int ldb2_ = 0, int rep2_ = 0) {
     wave = wave_;
     nk1 = kb_ / Cfg::PKB;
+    if constexpr (Cfg::RAG) {
+      lastq = (kb_ - 1) / Cfg::PKB;
+      nk1 = lastq + 1;
+    }
     full = Cfg::DS > 0 && wave < Cfg::SC_DMA;
     isA = wave * Cfg::DD < Cfg::A_DMA;
     kb2 = isA || ldb2_ == 0 ? kb2_ : ldb2_;
@@ -219,10 +247,8 @@ struct Ring {
   // scale plan of a dense scaled tile at (m0, n0)
   DSL_DEV void target_scales(const GemmArgs &p, int m0, int n0, int lane) {
     if constexpr (Cfg::SCALED) {
-      // bytes per scale row: fp32 per 128-K group, E8M0 per 32 elements or
-      // E4M3 per 16
-      const int64_t rowb = Cfg::BLOCK ? (int64_t)(p.K / 128) * 4
-                                      : (Cfg::MX ? (int64_t)(p.K / 32) : (int64_t)(p.K / 16));
+      const int64_t rowb = pers::scale_row_bytes<Cfg>(p);
+      if constexpr (Cfg::RAG) srowb = (int)rowb;
       if (wave < Cfg::SA_DMA) {
         int grow = m0 + wave * 64 + lane;
         grow = grow < p.M ? grow : p.M - 1;
@@ -250,7 +276,11 @@ struct Ring {
     r = r < lim ? r : lim;           // rows past the edge re-read the last row
     // swz(wrow + j*RPI + vsub) = swz(wrow + vsub) ^ swz(j*RPI): the row
     // offset j*RPI only flips bit 2 of the swizzle, by the parity of j
-    const uint32_t ch = vchunk ^ (uint32_t)(pair_swz(j * Cfg::RPI) * 16);
+    uint32_t ch = vchunk ^ (uint32_t)(pair_swz(j * Cfg::RPI) * 16);
+    if constexpr (Cfg::RAG) {        // chunks past K re-read the row's last one
+      const uint32_t most = (uint32_t)(q == lastq ? kb - 16 - q * Cfg::PKB : Cfg::PKB - 16);
+      ch = ch < most ? ch : most;
+    }
     // r < 256 and Kb < 2^24 (checked at launch): a full-rate 24-bit multiply
     if constexpr (Cfg::BF16) {
       // pairs from nk1 on come from the second segment (selects, no branch)
@@ -297,7 +327,9 @@ struct Ring {
   // `sslot`, when `on` (uniform)
   DSL_DEV void issue_scales(int on, int c, uint32_t sslot) const {
     const uint32_t dst = (uint32_t)(wave * 1024);   // SA parts, then SB right after
-    dma16_if(on, sbase + (int64_t)c * 16, soff, sslot + dst);
+    int64_t at = (int64_t)c * 16;
+    if constexpr (Cfg::RAG && Cfg::BLOCK) at = at < srowb - 16 ? at : srowb - 16;   // the row's last quad
+    dma16_if(on, sbase + at, soff, sslot + dst);
   }
 };
 
@@ -607,7 +639,18 @@ void gemm_persist_kernel(const Args p) {
     ldb2 = p.ldb2;
     rep2 = p.rep2;
   }
-  const int nkp = (kb + kb2) / Cfg::PKB;          // pairs per tile, >= 1
+  const int nkp = Cfg::RAG ? (kb + Cfg::PKB - 1) / Cfg::PKB   // no second segment
+                           : (kb + kb2) / Cfg::PKB;   // pairs per tile, >= 1
+  const int nv = (kb - (nkp - 1) * Cfg::PKB) / 16;    // RAG: chunks of a row's last pair
+  // words between the start of pair q's scale quad and the pair's first scale
+  auto quad_word = [&](int q) __attribute__((always_inline)) {
+    constexpr int PW = Cfg::BLOCK ? 1 : (Cfg::MX ? 2 : 0);   // words per pair within a quad
+    if constexpr (Cfg::RAG && Cfg::BLOCK) {           // a row's last quad ends with its last group
+      const int at = q & ~3;
+      return q - (at < nkp - 4 ? at : nkp - 4);
+    }
+    return (q % Cfg::QP) * PW;
+  };
 
   auto tile_ref = [&](int t) __attribute__((always_inline)) {
     TileRef tr;
@@ -741,7 +784,7 @@ void gemm_persist_kernel(const Args p) {
   auto block_scale = [&](const uint8_t *sq, int q, int i) __attribute__((always_inline)) {
     const float *sa = reinterpret_cast<const float *>(sq);
     const float *sb = reinterpret_cast<const float *>(sq + Cfg::SQA);
-    const int g4 = q % Cfg::QP;
+    const int g4 = quad_word(q);
     return sa[(wm * Cfg::WM + i * 32 + r32) * 4 + g4] * sb[((wn * Cfg::WN) / 128) * 4 + g4];
   };
 
@@ -904,13 +947,28 @@ void gemm_persist_kernel(const Args p) {
   }
   pipe::wait_vmcnt<Cfg::DD>();                // pair 0 landed, pair 1 may be in flight
   __syncthreads();
+  // RAG: zero the chunks past K of a row's last pair in its slot, once it has
+  // landed and been published: every row of A and W is one thread's
+  auto cut_pair = [&](int slot) __attribute__((always_inline)) {
+    if (nv < 8) {
+      const int row = wave * 64 + pers::lane_id();
+      for (int c = nv; c < 8; ++c)
+        *reinterpret_cast<uint4 *>(smem + slot * Cfg::PAIR + row * Cfg::PKB +
+                                   ((c ^ pers::pair_swz(row)) << 4)) = make_uint4(0, 0, 0, 0);
+      pipe::wait_lds();
+      __syncthreads();
+    }
+  };
+  if constexpr (Cfg::RAG) {
+    if (nkp == 1) cut_pair(0);
+  }
   // compute cursor: the pair whose half 0 was read last is tile-local pair
   // cq, in quad slot cqc % 2
   int cq = 0, cqc = 0;
   pers::Frag<Cfg> fa, fb[2];
-  fb[0].load_b(smem, squad, 0, 0, wn, r32, h);
+  fb[0].load_b(smem, squad, quad_word(0), 0, wn, r32, h);
 #pragma unroll
-  for (int i = 0; i < TM; ++i) fa.load_a(smem, squad, 0, 0, i, wm, r32, h);
+  for (int i = 0; i < TM; ++i) fa.load_a(smem, squad, quad_word(0), 0, i, wm, r32, h);
   if constexpr (Cfg::BLOCK) {
 #pragma unroll
     for (int i = 0; i < TM; ++i) sc[i] = block_scale(squad, 0, i);
@@ -929,7 +987,7 @@ void gemm_persist_kernel(const Args p) {
     constexpr bool FRESH = decltype(tag)::value == 2;
     const uint8_t *st = smem + (gp & 1) * Cfg::PAIR;
     const uint8_t *sq = squad + (cqc & 1) * Cfg::SQ;
-    const int sw = (cq % Cfg::QP) * 2;              // MX: the pair's scale words
+    const int sw = quad_word(cq);                   // MX, NV: the pair's scale words
     fb[1].load_b(st, sq, sw, 1, wn, r32, h);
     fb[1].share_scales(fb[0]);
     __builtin_amdgcn_sched_barrier(0);
@@ -959,6 +1017,9 @@ void gemm_persist_kernel(const Args p) {
     pipe::wait_vmcnt<0>();
     pipe::wait_lds();
     __syncthreads();
+    if constexpr (Cfg::RAG) {
+      if ((KIND == 2 ? 0 : cq + 1) == nkp - 1) cut_pair((gp + 1) & 1);
+    }
     const uint8_t *stn = smem + ((gp + 1) & 1) * Cfg::PAIR;
     bool quad;
     int qq;
@@ -972,7 +1033,7 @@ void gemm_persist_kernel(const Args p) {
     cq = KIND == 2 ? 0 : cq + 1;
     if (cq % Cfg::QP == 0) ++cqc;
     const uint8_t *sqn = squad + (cqc & 1) * Cfg::SQ;
-    const int sw = (cq % Cfg::QP) * 2;              // MX: the pair's scale words
+    const int sw = quad_word(cq);                   // MX, NV: the pair's scale words
     if constexpr (KIND != 2) fb[0].load_b(stn, sqn, sw, 0, wn, r32, h);
     float sn[TM];
     if constexpr (Cfg::BLOCK) {
@@ -1052,9 +1113,9 @@ int device_cu_count() {
   return cached[dev];
 }
 
-template <int MODE>
-static hipError_t launch_persist_mode(const GemmArgs &p, hipStream_t st) {
-  using Cfg = PersCfg<MODE>;
+template <int MODE, bool RAG>
+static hipError_t launch_persist_cfg(const GemmArgs &p, hipStream_t st) {
+  using Cfg = PersCfg<MODE, false, false, RAG>;
   const int ntiles = ((p.M + Cfg::BM - 1) / Cfg::BM) * ((p.N + Cfg::BN - 1) / Cfg::BN);
   int grid = device_cu_count();
   if (grid > ntiles) grid = ntiles;
@@ -1062,16 +1123,32 @@ static hipError_t launch_persist_mode(const GemmArgs &p, hipStream_t st) {
   return hipGetLastError();
 }
 
-bool persist_supported(int mode, int M, int N, int K, int Kb, bool scales16) {
-  (void)M;
-  (void)N;
-  if (Kb % 128 != 0 || Kb < 128) return false;          // whole pairs of 64-byte steps
-  if (Kb >= (1 << 24)) return false;                     // 24-bit row offsets
-  if (mode == MODE_FP8_TENSOR || mode == MODE_BF16) return true;
-  // scaled modes: whole 16-byte scale quads per row, 16-byte aligned rows
+bool persist_whole(int mode, int K, int Kb, bool scales16) {
+  if (Kb % 128 != 0) return false;
   if (mode == MODE_FP8_BLOCK || mode == MODE_MXFP4) return scales16 && K % 512 == 0;
   if (mode == MODE_NVFP4) return scales16 && K % 256 == 0;   // 16 scale bytes per row and pair
-  return false;
+  return true;
+}
+
+template <int MODE>
+static hipError_t launch_persist_mode(const GemmArgs &p, hipStream_t st) {
+  const uintptr_t sc = reinterpret_cast<uintptr_t>(p.sa) | reinterpret_cast<uintptr_t>(p.sb);
+  if (p.sld == 0 && persist_whole(MODE, p.K, p.Kb, (sc & 15) == 0))
+    return launch_persist_cfg<MODE, false>(p, st);
+  // ragged E8M0 / E4M3 rows come at a padded, 16-byte aligned pitch
+  if ((MODE == MODE_MXFP4 || MODE == MODE_NVFP4) && (p.sld < 16 || p.sld % 16 != 0 || (sc & 15) != 0))
+    return hipErrorInvalidValue;
+  return launch_persist_cfg<MODE, true>(p, st);
+}
+
+bool persist_supported(int mode, int M, int N, int K, int Kb, bool scales4) {
+  (void)M;
+  (void)N;
+  if (Kb % 16 != 0 || Kb < 128) return false;            // whole chunks
+  if (Kb >= (1 << 24)) return false;                     // 24-bit row offsets
+  if (mode == MODE_FP8_TENSOR || mode == MODE_BF16) return true;
+  if (mode == MODE_FP8_BLOCK) return scales4 && K > 384;  // a scale row holds a quad
+  return mode == MODE_MXFP4 || mode == MODE_NVFP4;
 }
 
 hipError_t launch_gemm_persist(int mode, const GemmArgs &p, hipStream_t st) {
@@ -1086,7 +1163,7 @@ hipError_t launch_gemm_persist(int mode, const GemmArgs &p, hipStream_t st) {
 }
 
 bool grouped_persist_supported(const GroupedArgs &p) {
-  return p.K % 128 == 0 && p.K >= 128 && p.K < (1 << 24) && p.G >= 1 && p.G <= kMaxGroups;
+  return p.K % 16 == 0 && p.K >= 128 && p.K < (1 << 24) && p.G >= 1 && p.G <= kMaxGroups;
 }
 
 // The device-side tile count is not known here: the grid is one workgroup
@@ -1108,8 +1185,10 @@ hipError_t launch_grouped_persist(const GroupedArgs &p, hipStream_t st) {
     // x rows are addressed by 32-bit offsets row * K
     if (p.xrows < 1 || (int64_t)p.xrows * p.K >= ((int64_t)1 << 32) || p.xrows >= (1 << 24))
       return hipErrorInvalidValue;
+    if (p.K % 128 != 0) return launch_grouped_persist_cfg<PersCfg<MODE_FP8_TENSOR, true, true, true>>(p, st);
     return launch_grouped_persist_cfg<PersCfg<MODE_FP8_TENSOR, true, true>>(p, st);
   }
+  if (p.K % 128 != 0) return launch_grouped_persist_cfg<PersCfg<MODE_FP8_TENSOR, true, false, true>>(p, st);
   return launch_grouped_persist_cfg<PersCfg<MODE_FP8_TENSOR, true>>(p, st);
 }
 

@@ -175,7 +175,7 @@ void gemm_pipe_block_kernel(const GemmArgs p) {
   pipe::Ring<Cfg> ring;
   ring.init(p, m0, n0, wave, lane);
 
-  const int nks = p.Kb / SKB, nkg = p.K / 128;
+  const int nks = pipe::stages_of<Cfg>(p.Kb), nkg = Cfg::RAG ? (p.K + 127) / 128 : p.K / 128;
   const int wm = wave / Cfg::WGN, wn = wave % Cfg::WGN;
   const int r16 = lane & 15, g = lane >> 4;
   int sbrow = (n0 + wn * Cfg::WN) / 128;
@@ -217,6 +217,7 @@ void gemm_pipe_block_kernel(const GemmArgs p) {
     if (ks + NS - 2 < nks) pipe::wait_vmcnt<(NS - 2) * D>();
     else pipe::wait_vmcnt<0>();
     __syncthreads();
+    pipe::cut_stage<Cfg>(ks, p.Kb, smem);
     const uint8_t *st = smem + (ks % NS) * Cfg::STAGE;
     const uint8_t *sA = st, *sB = st + Cfg::A_BYTES;
     const float *sSa = reinterpret_cast<const float *>(st + Cfg::A_BYTES + Cfg::B_BYTES);
@@ -576,13 +577,28 @@ static hipError_t launch_pipe_cfg(const GemmArgs &p, hipStream_t st) {
 }
 
 // Dense FP8 (per-tensor, block-scaled), MXFP4 and NVFP4 GEMM through the
-// LDS-DMA pipeline.  Preconditions (checked by the caller): Kb % 128 == 0,
-// ksplit == 1, 4-byte aligned scales.  Variant 0 is the default for large
+// LDS-DMA pipeline.  Preconditions (checked by the caller): Kb % 128 == 0 or
+// the RAG forms, 128x128 tiles whatever the variant (Kb % 16 == 0, MXFP4 /
+// NVFP4 with padded scale rows; 256x256 per-column tiles spilled 80 bytes
+// there), ksplit == 1, 4-byte aligned scales.  Variant 0 is the default for large
 // grids, 1 the 128x128 tile for mid-sized ones; the others are kept as
 // alternatives for tuning (DSL_GEMM_PIPE).
 hipError_t launch_gemm_pipe(int mode, const GemmArgs &p, int variant, hipStream_t st) {
   // C += result: fp32 output through the plain epilogue only
   if (p.accumulate && (!p.out_f32 || mode_grouped_k(mode))) return hipErrorInvalidValue;
+  if (p.Kb % 128 != 0) {
+    switch (mode) {
+      case MODE_FP8_GCOL:
+        return launch_pipe_cfg<PipeCfg<MODE_FP8_GCOL, 128, 128, 2, 2, 2, 128, 2, 0, true>>(p, st);
+      case MODE_FP8_BLOCK:
+        return launch_pipe_cfg<PipeCfg<MODE_FP8_BLOCK, 128, 128, 2, 2, 2, 128, 2, 0, true>>(p, st);
+      case MODE_BF16: return launch_pipe_cfg<PipeCfg<MODE_BF16, 128, 128, 2, 2, 4, 64, 0, 1, true>>(p, st);
+      case MODE_FP8_TENSOR:
+        return launch_pipe_cfg<PipeCfg<MODE_FP8_TENSOR, 128, 128, 2, 2, 4, 64, 0, 1, true>>(p, st);
+      case MODE_NVFP4: return launch_pipe_cfg<PipeCfg<MODE_NVFP4, 128, 128, 2, 4, 4, 64, 0, 0, true>>(p, st);
+      default: return launch_pipe_cfg<PipeCfg<MODE_MXFP4, 128, 128, 2, 4, 4, 64, 0, 0, true>>(p, st);
+    }
+  }
   if (mode == MODE_FP8_GCOL) {
     // per-column weight scales: the per-stage partial kernel (4-byte
     // aligned scales, K % 128 == 0)

@@ -620,10 +620,12 @@ struct StreamPlan {
 // K whose rows (or scale rows) take the TAIL form of the kernel: rows of no
 // whole 256-byte chunks, FP8 / MXFP4 scale rows of no whole 16 bytes (K %
 // 512), NVFP4 ones (K % 256), or scale arrays that are not 16-byte aligned;
-// and, from 97 rows, rows of an odd number of 256-byte chunks, for its
-// 64-row blocks (bf16 M=256 N=4096 K=4224: 22 us, on the 128x128 tiles 37).
+// and, from 129 rows, long rows of an odd number of 256-byte chunks, for its
+// 64-row blocks (bf16 M=256 N=4096 K=4224: 22 us, on the 128x128 tiles 37;
+// M=128: 18.2 against 15.9 in 32-row blocks; the K=128 LoRA add at M=512 N=4096
+// is 4 us faster in 32-row blocks).
 bool needs_tail(int mode, int M, int K, int Kb, bool scales16) {
-  if (Kb % 256 != 0 || (Kb % 512 != 0 && M > 96)) return true;
+  if (Kb % 256 != 0 || (Kb % 512 != 0 && M > 128 && Kb >= 1024)) return true;
   if (mode_grouped_k(mode) || mode == MODE_MXFP4) return !scales16 || K % 512 != 0;
   if (mode == MODE_NVFP4) return !scales16 || K % 256 != 0;
   return false;

@@ -218,7 +218,31 @@ struct Route {
   int path;
   int variant;    // PATH_PIPE variant
   Plan tiled;     // PATH_TILED plan
+  bool pad_scales = false;   // PATH_PERSIST / PATH_PIPE: E8M0 / E4M3 rows first copied to a padded pitch
 };
+
+// E8M0 / E4M3 scale rows that are no whole 16-byte quads (persistent kernel)
+// or 4-byte words per stage (pipelined tiles): [rows][len] bytes -> [rows][pitch], `fill` past len (one launch for
+// both operands; 4 bytes per thread).
+__global__ void pad_scales_kernel(const uint8_t *__restrict__ a, int rows_a,
+                                  const uint8_t *__restrict__ b, int rows_b, int len, int pitch,
+                                  uint32_t fill, uint32_t *__restrict__ out) {
+  const int wpr = pitch / 4;
+  const int64_t total = ((int64_t)rows_a + rows_b) * wpr;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t row = i / wpr;
+    const int c = (int)(i - row * wpr) * 4;
+    const uint8_t *src = row < rows_a ? a + row * len : b + (row - rows_a) * len;
+    uint32_t v = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v |= (c + k < len ? (uint32_t)src[c + k] : fill) << (8 * k);
+    out[i] = v;
+  }
+}
+
+static int scale_row_len(int mode, int K) { return mode == MODE_MXFP4 ? K / 32 : K / 16; }
+static int padded_pitch(int mode, int K) { return (scale_row_len(mode, K) + 15) / 16 * 16; }
 
 constexpr int kAccShortK = 512;   // C += result with K up to this streams where it can
 
@@ -227,7 +251,8 @@ static bool stream_enabled() {
   return on;
 }
 
-static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc16) {
+// `padded`: a workspace for padded scale rows is there.
+static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc16, bool padded) {
   static const bool decode_on = !env_off("DSL_GEMM_DECODE");
   const bool stream_on = stream_enabled();
   const char *skinny = getenv("DSL_GEMM_SKINNY");      // read per launch (tests switch it)
@@ -252,7 +277,10 @@ static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc1
   // M=320 N=14336: 91.4 against 88.1).  Rows of an odd number of 256-byte
   // chunks stream in 32-row blocks: twice the blocks.
   const int64_t t128 = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
-  const bool bf16_pipe_round = mode == MODE_BF16 && pipe_forced != -2 && Kb % 128 == 0 && M > 64 &&
+  // (ragged K: from half the CUs; 768x1640x4168, 78 tiles, 58 us on them
+  // against about 40 streamed)
+  const bool bf16_pipe_round = mode == MODE_BF16 && pipe_forced != -2 && M > 64 &&
+                               (Kb % 128 == 0 || 2 * t128 >= device_cu_count()) &&
                                N > 64 && t128 >= 40 && t128 <= device_cu_count();
   if (streamable && !skinny_stream && M > 32 && (mode != MODE_NVFP4 || M > 256)) {
     const int bm = stream_blocks64(mode, M, K, Kb, sc16) ? 64 : 32;
@@ -318,12 +346,19 @@ static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc1
       r.path = PATH_PIPE;
       r.variant = 1;
     } else if (persist_on && 6 * t256 >= device_cu_count() && (int64_t)M * N >= 2400000 &&
-               persist_supported(mode, M, N, K, Kb, sc16)) {
+               persist_supported(mode, M, N, K, Kb, sc4)) {
       r.path = PATH_PERSIST;
     }
     return r;
   }
-  const bool pipe_ok = pipe_forced != -2 && Kb % 128 == 0 && (mode == MODE_FP8_TENSOR || sc4);
+  // K of no whole 128 bytes: the ragged forms of both kernels, MXFP4 and NVFP4
+  // with their scale rows at a padded pitch (the persistent kernel also where
+  // only the scale rows are ragged)
+  const bool fp4 = mode == MODE_MXFP4 || mode == MODE_NVFP4;
+  const bool rag = Kb % 128 != 0, pad = fp4 && !persist_whole(mode, K, Kb, sc16);
+  const bool pipe_ok = pipe_forced != -2 && (mode == MODE_FP8_TENSOR || sc4) && (!rag || !fp4 || padded);
+  const bool persist_ok = persist_on && pipe_forced < 0 &&
+                          persist_supported(mode, M, N, K, Kb, sc4) && (!pad || padded);
   if (pipe_ok) {
     const int64_t t256 = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
     // Rounds of tiles per CU: a round of 256x256 persistent tiles costs
@@ -345,30 +380,31 @@ static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc1
     if (persist_wins) {
       r.path = PATH_PIPE;
       r.variant = pipe_forced >= 0 ? pipe_forced : (t256 >= 240 ? 0 : 1);
-      if (persist_on && pipe_forced < 0 && persist_supported(mode, M, N, K, Kb, sc16))
-        r.path = PATH_PERSIST;
+      if (persist_ok) r.path = PATH_PERSIST;
     } else if (M > 64 && N > 64 && t128 >= 40) {
       r.path = PATH_PIPE;
       r.variant = 1;
     }
   }
+  r.pad_scales = (r.path == PATH_PERSIST && pad) || (r.path == PATH_PIPE && fp4 && rag);
   return r;
 }
 
 bool gemm_routes_to_stream(int mode, int64_t M, int64_t N, int64_t K, bool or_pipe, bool accumulate) {
   const int Kb = (mode == MODE_MXFP4 || mode == MODE_NVFP4) ? (int)(K / 2)
                                                             : (mode == MODE_BF16 ? (int)(2 * K) : (int)K);
-  int path = route_for(mode, (int)M, (int)N, (int)K, Kb, true, true).path;
+  int path = route_for(mode, (int)M, (int)N, (int)K, Kb, true, true, true).path;
   if (accumulate && K <= kAccShortK && stream_enabled() && stream_supported(mode, (int)M, (int)N, (int)K, Kb, true))
     path = PATH_STREAM;   // as launch_gemm routes C += result
   return path == PATH_STREAM || (or_pipe && path == PATH_PIPE && (!accumulate || !mode_grouped_k(mode)));
 }
 
-size_t gemm_workspace_bytes(int mode, int64_t M, int64_t N, int64_t K, bool accumulate) {
+size_t gemm_workspace_bytes(int mode, int64_t M, int64_t N, int64_t K, bool accumulate, bool padded) {
   const int Kb = (mode == MODE_MXFP4 || mode == MODE_NVFP4) ? (int)(K / 2)
                                                             : (mode == MODE_BF16 ? (int)(2 * K) : (int)K);
-  Route r = route_for(mode, (int)M, (int)N, (int)K, Kb, true, true);
+  Route r = route_for(mode, (int)M, (int)N, (int)K, Kb, true, true, padded);
   if (accumulate) r.path = PATH_TILED;
+  if (r.pad_scales && r.path != PATH_TILED) return (size_t)(M + N) * (size_t)padded_pitch(mode, (int)K);
   return (r.path == PATH_TILED && r.tiled.ksplit > 1)
              ? (size_t)r.tiled.ksplit * (size_t)splitk_slice(M, N) * sizeof(float)
              : 0;
@@ -388,7 +424,11 @@ hipError_t launch_gemm(int mode, GemmArgs p, hipStream_t st) {
     return launch_gemm_persist(mode, p, st);
   }
   if (p.rep2 != 0 || p.ldb2 != 0) return hipErrorInvalidValue;
-  Route r = route_for(mode, p.M, p.N, p.K, p.Kb, (sc & 3) == 0, (sc & 15) == 0);
+  // scale rows are padded only into a workspace that holds them
+  const bool padded = (mode == MODE_MXFP4 || mode == MODE_NVFP4) && p.ws &&
+                      (reinterpret_cast<uintptr_t>(p.ws) & 15) == 0 &&
+                      p.ws_bytes >= (size_t)((int64_t)p.M + p.N) * (size_t)padded_pitch(mode, p.K);
+  Route r = route_for(mode, p.M, p.N, p.K, p.Kb, (sc & 3) == 0, (sc & 15) == 0, padded);
   if (p.lora_scales) {   // the LoRA epilogue: the streaming kernel only
     if (mode != MODE_BF16 || !stream_supported(mode, p.M, p.N, p.K, p.Kb, true) || p.accumulate)
       return hipErrorInvalidValue;
@@ -409,8 +449,26 @@ hipError_t launch_gemm(int mode, GemmArgs p, hipStream_t st) {
   p.ksplit = 1;
   if (r.path == PATH_DECODE) return launch_gemm_decode(mode, p, st);
   if (r.path == PATH_STREAM) return launch_gemm_stream(mode, p, st);
-  if (r.path == PATH_PIPE) return launch_gemm_pipe(mode, p, r.variant, st);
-  if (r.path == PATH_PERSIST) return launch_gemm_persist(mode, p, st);
+  if (r.path == PATH_PERSIST || r.path == PATH_PIPE) {
+    if (r.pad_scales) {
+      const int pitch = padded_pitch(mode, p.K);
+      const int64_t words = ((int64_t)p.M + p.N) * (pitch / 4);
+      const unsigned g = (unsigned)std::min<int64_t>((words + 255) / 256, 4096);
+      uint8_t *out = reinterpret_cast<uint8_t *>(p.ws);
+      pad_scales_kernel<<<g, 256, 0, st>>>(static_cast<const uint8_t *>(p.sa), p.M,
+                                           static_cast<const uint8_t *>(p.sb), p.N,
+                                           scale_row_len(mode, p.K), pitch,
+                                           mode == MODE_MXFP4 ? 0x7fu : 0u,
+                                           reinterpret_cast<uint32_t *>(out));
+      const hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return e;
+      p.sa = out;
+      p.sb = out + (int64_t)p.M * pitch;
+      p.sld = pitch;
+    }
+    if (r.path == PATH_PIPE) return launch_gemm_pipe(mode, p, r.variant, st);
+    return launch_gemm_persist(mode, p, st);
+  }
   const Plan pl = r.tiled;
   // split-K into as many [M][N] fp32 slices as the workspace holds (at most
   // the plan's split count; fewer than two: one pass over K)

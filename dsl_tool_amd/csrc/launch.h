@@ -70,6 +70,10 @@ struct GemmArgs {
   // pairs after which W2's columns repeat (0: none; else a power of two): W2
   // = [B | B] is then read from B itself
   int ldb2 = 0, rep2 = 0;
+  // bytes per scale row of MXFP4 / NVFP4 scales copied to a padded pitch (a
+  // multiple of 16; 0: the natural K/32 or K/16); ragged forms of the
+  // persistent and pipelined kernels
+  int sld = 0;
   // Streaming kernel only, BF16 (the LoRA adapter product T^T = A^T X^T):
   // v = C[m][n] * lora_scales[m / lora_rank] is stored transposed, as bf16
   // hi at c[n * ldc + m] and lo = bf16(v - hi) at c[n * ldc + M + m], and
@@ -78,16 +82,19 @@ struct GemmArgs {
   int lora_rank = 1;
 };
 
-// LDS-DMA pipelined kernel (FP8_TENSOR / MXFP4, Kb % 64 == 0, no split-K);
+// LDS-DMA pipelined kernel (every mode, no split-K; Kb % 128 == 0, or the
+// ragged forms of variant 1);
 // variant 0: 256x256 tile, 8 waves; 1: 128x128 tile, 4 waves.
 hipError_t launch_gemm_pipe(int mode, const GemmArgs &p, int variant, hipStream_t st);
 
-// Persistent pipelined kernel (Kb % 128 == 0; FP8_TENSOR and BF16; FP8_BLOCK
-// and MXFP4 with 16-byte aligned scales and K % 512 == 0; NVFP4 with K % 256
-// == 0): one workgroup per CU
-// walks its 256x256 tiles with a ring of 128-byte-per-row pair slots running
-// across tile boundaries.
-bool persist_supported(int mode, int M, int N, int K, int Kb, bool scales16);
+// Persistent pipelined kernel (Kb >= 128 in whole 16-byte chunks; not
+// FP8_GCOL; FP8_BLOCK with K > 384): one workgroup per CU walks its 256x256
+// tiles with a ring of 128-byte-per-row pair slots running across tile
+// boundaries.
+bool persist_supported(int mode, int M, int N, int K, int Kb, bool scales4);
+// Rows of whole pairs and scale rows of whole quads.  Other MXFP4 / NVFP4
+// scale rows must come at a padded pitch (GemmArgs::sld).
+bool persist_whole(int mode, int K, int Kb, bool scales16);
 hipError_t launch_gemm_persist(int mode, const GemmArgs &p, hipStream_t st);
 
 // Skinny-M kernels, one launch, no workspace (Kb % 1024 == 0):
@@ -109,8 +116,10 @@ hipError_t launch_gemm_stream(int mode, const GemmArgs &p, hipStream_t st);
 // Picks a kernel variant for the shape and launches it (plus the split-K
 // finalize kernel, which adds the slices in split order, when ksplit > 1).
 hipError_t launch_gemm(int mode, GemmArgs args, hipStream_t st);
-// Workspace the launcher will need for this shape (0 if none).
-size_t gemm_workspace_bytes(int mode, int64_t M, int64_t N, int64_t K, bool accumulate = false);
+// Workspace the launcher will need for this shape (0 if none); padded false:
+// what it can do with where it cannot copy ragged scale rows to a padded pitch.
+size_t gemm_workspace_bytes(int mode, int64_t M, int64_t N, int64_t K, bool accumulate = false,
+                            bool padded = true);
 // Whether launch_gemm takes the streaming kernel (or_pipe: or the pipelined
 // tiles) for this shape (aligned scales; accumulate: C += result, fp32 out).
 bool gemm_routes_to_stream(int mode, int64_t M, int64_t N, int64_t K, bool or_pipe = false,
@@ -136,7 +145,7 @@ struct GroupedArgs {
   int xrows = 0;
 };
 hipError_t launch_grouped_fp8(GroupedArgs args, hipStream_t st);
-// Grouped FP8 on the persistent kernel (K % 128 == 0, K < 2^24).
+// Grouped FP8 on the persistent kernel (K % 16 == 0, 128 <= K < 2^24).
 bool grouped_persist_supported(const GroupedArgs &args);
 hipError_t launch_grouped_persist(const GroupedArgs &args, hipStream_t st);
 // Grouped FP8 on the streaming tiles (few rows per group; K % 16 == 0).

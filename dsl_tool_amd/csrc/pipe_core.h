@@ -18,6 +18,10 @@
 //     LDS read); completion is waited for explicitly with s_waitcnt vmcnt
 //     before the barrier that publishes a stage to the workgroup.
 //   * LDS rows are SKB bytes of 16-byte chunks, XOR-swizzled (swz below).
+//   * Ragged K (RAG): rows of no whole stages.  The copies of a partial stage
+//     re-read the row's last 16-byte chunk, and its chunks past K are zeroed
+//     in LDS once it has landed (cut_stage), so the fragments' readers stay
+//     the same; MXFP4 / NVFP4 scale rows then come at a padded pitch.
 //   * MXFP4 scales (SKB/16 E8M0 bytes per row per stage) ride along in the
 //     same ring via 4-byte direct loads and go straight into the scaled MFMA.
 //
@@ -95,8 +99,9 @@ DSL_DEV v16f mfma_fp4(const v4i &a, const v4i &b, const v16f &c, int sa, int sb)
 }  // namespace pipe
 
 template <int MODE_, int BM_, int BN_, int WGM_, int WGN_, int NS_, int SKB_ = 64, int OCC_ = 0,
-          int PF_ = 0>
+          int PF_ = 0, bool RAG_ = false>
 struct PipeCfg {
+  static constexpr bool RAG = RAG_;                         // ragged K
   static constexpr int MODE = MODE_, BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, NS = NS_;
   static constexpr bool PF = PF_ != 0;                      // fragment prefetch schedule
   static constexpr int SKB = SKB_;                          // stage bytes per row
@@ -161,10 +166,14 @@ struct Ring {
   int step[Cfg::D];
   bool has[Cfg::D];     // scale-word slot used by this wave
   bool full;
+  int kb, lane;         // RAG: bytes per row; the lane
 
-  DSL_DEV void init(const GemmArgs &p, int m0, int n0, int wave, int lane) {
+  DSL_DEV void init(const GemmArgs &p, int m0, int n0, int wave, int lane_) {
     constexpr int SKB = Cfg::SKB;
     full = true;
+    kb = p.Kb;
+    lane = lane_;
+    const int nkg = Cfg::RAG ? (p.K + 127) / 128 : p.K / 128;
 #pragma unroll
     for (int j = 0; j < Cfg::D; ++j) {
       src[j] = p.a;
@@ -200,7 +209,7 @@ struct Ring {
         if constexpr (Cfg::GCOL) {
           if (isA) {                       // fp32 sa[row][K/128]: one float per row per group
             src[j] = reinterpret_cast<const uint8_t *>(static_cast<const float *>(p.sa) +
-                                                       (int64_t)grow * (p.K / 128));
+                                                       (int64_t)grow * nkg);
             step[j] = 4;
           } else {                         // fp32 sb[K/128][N]: the tile's columns of a group
             src[j] = reinterpret_cast<const uint8_t *>(static_cast<const float *>(p.sb) + grow);
@@ -208,14 +217,14 @@ struct Ring {
           }
         } else if constexpr (Cfg::BLOCK) { // fp32 sa[row][K/128]: one float per row per group
           src[j] = reinterpret_cast<const uint8_t *>(static_cast<const float *>(p.sa) +
-                                                     (int64_t)grow * (p.K / 128));
+                                                     (int64_t)grow * nkg);
           step[j] = 4;
         } else if constexpr (Cfg::MX) {    // E8M0 [row][K/32]: SKB/16 bytes per row per stage
-          src[j] = static_cast<const uint8_t *>(isA ? p.sa : p.sb) + (int64_t)grow * (p.K / 32) +
+          src[j] = static_cast<const uint8_t *>(isA ? p.sa : p.sb) + (int64_t)grow * (Cfg::RAG && p.sld ? p.sld : p.K / 32) +
                    word * 4;
           step[j] = SKB / 16;
         } else {                           // E4M3 [row][K/16]: SKB/8 bytes per row per stage
-          src[j] = static_cast<const uint8_t *>(isA ? p.sa : p.sb) + (int64_t)grow * (p.K / 16) +
+          src[j] = static_cast<const uint8_t *>(isA ? p.sa : p.sb) + (int64_t)grow * (Cfg::RAG && p.sld ? p.sld : p.K / 16) +
                    word * 4;
           step[j] = SKB / 8;
         }
@@ -225,10 +234,21 @@ struct Ring {
     }
   }
 
+  // RAG: how far operand copy j of stage ks lies past the row's last chunk
+  DSL_DEV int past(int j, int ks) const {
+    if constexpr (!Cfg::RAG) return 0;
+    // the lane's row within the copied block: copies start at multiples of RPI
+    // rows, and swz<SKB> depends on the row within the operand
+    const int i = (int)(dst[j] >> 10);
+    const int lrow = (i < Cfg::A_DMA ? i : i - Cfg::A_DMA) * Cfg::RPI + lane / Cfg::CH;
+    const int chunk = (lane % Cfg::CH) ^ swz<Cfg::SKB>(lrow);
+    const int over = ks * Cfg::SKB + chunk * 16 - (kb - 16);
+    return over > 0 ? over : 0;
+  }
   // DMA instruction j of stage ks
   DSL_DEV void issue_one(int j, int ks, uint32_t lds0) const {
     const uint32_t base = lds0 + (uint32_t)((ks % Cfg::NS) * Cfg::STAGE);
-    if (j < Cfg::DD) dma16(src[j] + (int64_t)ks * step[j], base + dst[j]);
+    if (j < Cfg::DD) dma16(src[j] + (int64_t)ks * step[j] - past(j, ks), base + dst[j]);
     else if (has[j]) dma4(src[j] + (int64_t)(ks >> Cfg::SC_SHIFT) * step[j], base + dst[j]);
   }
   // The same copies for a caller that issues stages strictly in order: the
@@ -240,7 +260,7 @@ struct Ring {
 #pragma unroll
     for (int j = 0; j < Cfg::D; ++j) {
       if (j < Cfg::DD) {
-        dma16(src[j], base + dst[j]);
+        dma16(src[j] - past(j, ks), base + dst[j]);
         src[j] += step[j];
       } else if (has[j]) {
         dma4(src[j], base + dst[j]);
@@ -256,7 +276,7 @@ struct Ring {
     for (int j = 0; j < Cfg::D; ++j) {
       if (j < j0 || j >= j1) continue;
       if (j < Cfg::DD) {
-        dma16(src[j], base + dst[j]);
+        dma16(src[j] - past(j, ks), base + dst[j]);
         src[j] += step[j];
       } else if (has[j]) {
         dma4(src[j], base + dst[j]);
@@ -601,6 +621,34 @@ DSL_DEV void wait_stages_of(int n, bool full) {
   wait_stages<D, NMAX>(n);
 }
 
+// RAG: stages of a row (an even number of them, at least two, on the prefetch
+// schedule), and the zeroing of a published stage's chunks past K.  Every
+// thread of the workgroup calls cut_stage.
+template <class Cfg>
+DSL_DEV int stages_of(int kb) {
+  if constexpr (!Cfg::RAG) return kb / Cfg::SKB;
+  const int n = (kb + Cfg::SKB - 1) / Cfg::SKB;
+  return Cfg::PF ? (n + 1) / 2 * 2 : n;
+}
+template <class Cfg>
+DSL_DEV void cut_stage(int ks, int kb, uint8_t *smem) {
+  if constexpr (Cfg::RAG) {
+    const int left = (kb - ks * Cfg::SKB) / 16;      // chunks of the row from this stage on
+    if (left < Cfg::CH) {
+      const int nv = left > 0 ? left : 0;
+      uint8_t *st = smem + (ks % Cfg::NS) * Cfg::STAGE;
+      for (int r = (int)threadIdx.x; r < Cfg::BM + Cfg::BN; r += Cfg::NT) {
+        const int row = r < Cfg::BM ? r : r - Cfg::BM;
+        for (int c = nv; c < Cfg::CH; ++c)
+          *reinterpret_cast<uint4 *>(st + r * Cfg::SKB + ((c ^ swz<Cfg::SKB>(row)) << 4)) =
+              make_uint4(0, 0, 0, 0);
+      }
+      __builtin_amdgcn_s_waitcnt((15 << 0) | (7 << 4) | (0 << 8) | (3 << 14));
+      __syncthreads();
+    }
+  }
+}
+
 // Every LDS read this wave issued has returned (its data is in registers).
 DSL_DEV void wait_lds() { __builtin_amdgcn_s_waitcnt((15 << 0) | (7 << 4) | (0 << 8) | (3 << 14)); }
 
@@ -626,6 +674,7 @@ DSL_DEV void pf_step(int ks, int nks, const pipe::Ring<Cfg> &ring, uint32_t lds0
   }
   pipe::wait_lds();
   __syncthreads();
+  pipe::cut_stage<Cfg>(ks + 1, ring.kb, const_cast<uint8_t *>(smem));
   cur.template mma_prefetch<TR>(acc, nxt, smem + ((ks + 1) % NS) * Cfg::STAGE, wm, wn, r32, h, ring,
                    STEADY || ks + NS < nks, ks + NS, lds0);
 }
@@ -655,7 +704,7 @@ DSL_DEV void pipe_mainloop(const GemmArgs &p, int m0, int n0, uint8_t *smem, int
   const uint32_t lds0 = pipe::lds_addr(smem);
   pipe::Ring<Cfg> ring;
   ring.init(p, m0, n0, wave, lane);
-  const int nks = p.Kb / Cfg::SKB;
+  const int nks = pipe::stages_of<Cfg>(p.Kb);
   const int wm = wave / Cfg::WGN, wn = wave % Cfg::WGN;
   const int r32 = lane & 31, h = lane >> 5;
 #pragma unroll
@@ -678,6 +727,7 @@ DSL_DEV void pipe_mainloop(const GemmArgs &p, int m0, int n0, uint8_t *smem, int
       pipe::wait_stages_of<D, NS - 2>(pending, ring.full);
       __syncthreads();
       if (ks + NS - 1 < nks) ring.issue(ks + NS - 1, lds0);
+      pipe::cut_stage<Cfg>(ks, p.Kb, smem);
       const uint8_t *st = smem + (ks % NS) * Cfg::STAGE;
 #pragma unroll
       for (int k = 0; k < Cfg::KSTEPS; ++k) {
@@ -697,6 +747,7 @@ DSL_DEV void pipe_mainloop(const GemmArgs &p, int m0, int n0, uint8_t *smem, int
     // stages issued after the prologue: 0 .. min(NS, nks) - 1
     pipe::wait_stages_of<D, NS - 1>((nks < NS ? nks : NS) - 1, ring.full);
     __syncthreads();
+    pipe::cut_stage<Cfg>(0, p.Kb, smem);
     StageFrag<Cfg> f0, f1;
     f0.load(smem, wm, wn, r32, h);
     // steady state in pairs (f0 -> f1 -> f0), every step with a next stage;

@@ -97,3 +97,62 @@ def test_ragged_k_grouped_stream(counts, k):
     wd = (qw.view(torch.float8_e4m3fn).double().cpu() * sw.double().cpu()).view(g, n, k)
     ref = torch.cat([xd[off[e]:off[e + 1]] @ wd[e].t() for e in range(g)])
     assert_close(y, ref.float().numpy(), what=f"grouped stream {counts} K={k}")
+
+
+# the persistent tiles: more than one tile per workgroup at short K (partial
+# pairs as a tile's only, second and later one), ragged rows and columns
+@pytest.mark.parametrize("mode,k", [("tensor", 16 * 9), ("tensor", 400), ("tensor", 1168), ("block", 640),
+                                    ("block", 400), ("block", 1168), ("mxfp4", 288), ("mxfp4", 1056),
+                                    ("mxfp4", 1408), ("nvfp4", 288), ("nvfp4", 1056), ("nvfp4", 1344),
+                                    ("bf16", 72), ("bf16", 200), ("bf16", 584)])
+def test_ragged_k_persistent(mode, k):
+    check(mode, 4352, 4300, k)
+    check(mode, 1025, 1000, k)
+
+
+@pytest.mark.parametrize("k", [144, 400, 1168])
+def test_ragged_k_grouped_persistent(k):
+    counts, n = (300, 0, 97, 513), 264
+    g, t = len(counts), sum(counts)
+    x, w = W.randn_bf16((t, k), 7).to(DEV), W.randn_bf16((g * n, k), 8, 0.02).to(DEV)
+    off = torch.tensor([0] + list(np.cumsum(counts)), dtype=torch.int32, device=DEV)
+    qx, sx = Q.quant_fp8_blocks(x, 1, k)
+    qw, sw = Q.quant_fp8_blocks(w, 1, k)
+    y = G.grouped_fp8_gemm_packed(qx, sx, qw.view(g, n, k), sw.view(g, n), off)
+    xd = qx.view(torch.float8_e4m3fn).double().cpu() * sx.double().cpu()
+    wd = (qw.view(torch.float8_e4m3fn).double().cpu() * sw.double().cpu()).view(g, n, k)
+    ref = torch.cat([xd[off[e]:off[e + 1]] @ wd[e].t() for e in range(g)])
+    assert_close(y, ref.float().numpy(), what=f"grouped persistent {counts} K={k}")
+
+
+# one round of the 128x128 tiles: partial first, odd and even last stages
+@pytest.mark.parametrize("mode,k", [("tensor", 48), ("tensor", 336), ("tensor", 1072), ("block", 144),
+                                    ("block", 1072), ("group", 144), ("group", 1072), ("mxfp4", 96),
+                                    ("mxfp4", 672), ("mxfp4", 2144), ("nvfp4", 96), ("nvfp4", 672),
+                                    ("nvfp4", 2144), ("bf16", 24), ("bf16", 168), ("bf16", 536)])
+def test_ragged_k_pipelined(mode, k):
+    check(mode, 1100, 1000, k)
+    check(mode, 1200, 1029, k)
+
+
+def test_padded_scale_rows_need_their_workspace():
+    """The query covers the padded scale rows; a caller without them still runs."""
+    from dsl_tool_amd import _native as N
+    m, n, k = 1100, 1000, 2144
+    a, w = W.randn_bf16((m, k), 9).to(DEV), W.randn_bf16((n, k), 10, 0.02).to(DEV)
+    (qa, sa), (qw, sw) = Q.quant_mxfp4(a), Q.quant_mxfp4(w)
+    assert N.lib().dsl_gemm_workspace_bytes(N.OP_FP4, m, n, k) >= (m + n) * 80
+    want = G.fp4_gemm_packed(qa, sa, qw, sw)
+    c = torch.empty_like(want)
+    ws = torch.empty(16 * (m * n + 4), dtype=torch.float32, device=DEV)   # split-K's own size
+    for nb in (ws.numel() * 4, (m + n) * 64):
+        if nb < (m + n) * 80 and N.lib().dsl_gemm_workspace_bytes(N.OP_FP4, m, n, k) > 0:
+            with pytest.raises(N.DslError, match="workspace"):
+                N.call("dsl_fp4_gemm", qa.data_ptr(), qw.data_ptr(), c.data_ptr(), m, n, k, n, N.OUT_BF16,
+                       N.FMT_MXFP4, sa.data_ptr(), sw.data_ptr(), None, None, ws.data_ptr(), nb,
+                       N.stream_of(a.device))
+            continue
+        N.call("dsl_fp4_gemm", qa.data_ptr(), qw.data_ptr(), c.data_ptr(), m, n, k, n, N.OUT_BF16,
+               N.FMT_MXFP4, sa.data_ptr(), sw.data_ptr(), None, None, ws.data_ptr(), nb,
+               N.stream_of(a.device))
+        assert torch.equal(c, want)
