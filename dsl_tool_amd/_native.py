@@ -6,11 +6,14 @@ library links against, so the dynamic loader reuses torch's runtime and the
 two share devices, streams and allocations.
 
 There is no fallback: if the library is missing or fails to load, every
-entry point raises ``DslLibraryError``.
+entry point raises ``DslLibraryError``.  ``fast()`` is the CPython extension
+that makes the same calls for well-formed tensors without the ctypes layer.
 """
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import re
 import threading
@@ -19,6 +22,7 @@ import torch  # noqa: F401  (must precede loading the HIP library, see above)
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(PKG_DIR, "_lib", "libdsl_gemm.so")
+FAST_PATH = os.path.join(PKG_DIR, "_lib", "dsl_fast.so")
 HEADER_PATH = os.path.join(os.path.dirname(PKG_DIR), "include", "dsl_gemm.h")
 
 DSL_OK = 0
@@ -117,6 +121,42 @@ def lib():
                 raise DslLibraryError("libdsl_gemm.so ABI version mismatch; rebuild it")
             _lib = handle
     return _lib
+
+
+class _NoFast:
+    """Stands for the extension while the library is not built: every call is
+    left to the Python path, whose own checks come first."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+_fast = None
+
+
+def fast():
+    """The ``dsl_fast`` extension (loaded once): functions that take the
+    operands of a well-formed call and return its results, or None for the
+    Python path to handle the call."""
+    global _fast
+    if _fast is not None:
+        return _fast
+    if not os.path.exists(LIB_PATH):
+        return _NoFast()
+    lib()
+    with _lock:
+        if _fast is None:
+            if not os.path.exists(FAST_PATH):
+                raise DslLibraryError(
+                    f"extension not built: {FAST_PATH} (run `python -m dsl_tool_amd.build`)")
+            loader = importlib.machinery.ExtensionFileLoader("dsl_fast", FAST_PATH)
+            try:
+                mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("dsl_fast", loader))
+                loader.exec_module(mod)
+            except ImportError as exc:
+                raise DslLibraryError(f"cannot load {FAST_PATH}: {exc}") from exc
+            _fast = mod
+    return _fast
 
 
 def call(name: str, *args) -> None:

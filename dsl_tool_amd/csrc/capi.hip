@@ -213,9 +213,8 @@ static int run_gemm(const char *fn, int mode, const uint8_t *a, const uint8_t *b
   if (!c) return fail(DSL_ERR_ARG, "%s: c is NULL", fn);
   if (!aligned(c, out_dtype == DSL_OUT_F32 ? 4 : 2))
     return fail(DSL_ERR_ARG, "%s: c is misaligned", fn);
-  const size_t need = dsl::gemm_workspace_bytes(mode, m, n, k);
-  const size_t least = std::min(need, dsl::gemm_workspace_bytes(mode, m, n, k, false, false));
-  if (least && (!ws || ws_bytes < least || !aligned(ws, 16)))
+  const size_t need = dsl::gemm_workspace_required(mode, m, n, k);
+  if (need && (!ws || ws_bytes < need || !aligned(ws, 16)))
     return fail(DSL_ERR_WORKSPACE, "%s: workspace of %zu bytes (16-B aligned) required", fn, need);
   dsl::GemmArgs p;
   p.a = a;

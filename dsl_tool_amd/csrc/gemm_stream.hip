@@ -603,6 +603,12 @@ __global__ __launch_bounds__(Cfg::NT) void gemm_stream_grouped_kernel(const Grou
                            gp.sw + (int64_t)e * gp.N, GATHER ? gp.arow + lo : nullptr, gp.xrows);
 }
 
+bool stream_whole(int mode, int K, int Kb, bool scales16) {
+  if (Kb % 256 != 0) return false;
+  if (mode_grouped_k(mode) || mode == MODE_MXFP4) return scales16 && K % 512 == 0;
+  return mode != MODE_NVFP4 || (scales16 && K % 256 == 0);
+}
+
 // ---------------------------------------------------------------- plans --
 namespace {
 
@@ -625,10 +631,7 @@ struct StreamPlan {
 // M=128: 18.2 against 15.9 in 32-row blocks; the K=128 LoRA add at M=512 N=4096
 // is 4 us faster in 32-row blocks).
 bool needs_tail(int mode, int M, int K, int Kb, bool scales16) {
-  if (Kb % 256 != 0 || (Kb % 512 != 0 && M > 128 && Kb >= 1024)) return true;
-  if (mode_grouped_k(mode) || mode == MODE_MXFP4) return !scales16 || K % 512 != 0;
-  if (mode == MODE_NVFP4) return !scales16 || K % 256 != 0;
-  return false;
+  return !stream_whole(mode, K, Kb, scales16) || (Kb % 512 != 0 && M > 128 && Kb >= 1024);
 }
 
 bool stream_rows64(int M, int Kb, bool tail) { return tail ? M > 96 : Kb % 512 == 0; }

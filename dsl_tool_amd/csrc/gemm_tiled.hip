@@ -251,8 +251,11 @@ static bool stream_enabled() {
   return on;
 }
 
-// `padded`: a workspace for padded scale rows is there.
-static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc16, bool padded) {
+// `padded`: a workspace for padded scale rows is there.  `ragged` false: the
+// kernel that serves the shape without the ragged forms (rows and scale rows of
+// whole steps only); the workspace contract is that route's.
+static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc16, bool padded,
+                       bool ragged = true) {
   static const bool decode_on = !env_off("DSL_GEMM_DECODE");
   const bool stream_on = stream_enabled();
   const char *skinny = getenv("DSL_GEMM_SKINNY");      // read per launch (tests switch it)
@@ -265,7 +268,8 @@ static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc1
     return (e && e[0] >= '1' && e[0] <= '9' && !e[1]) ? e[0] - '0' : -1;
   }();
   Route r{PATH_TILED, -1, plan_for(M, N, Kb)};
-  bool streamable = stream_on && stream_supported(mode, M, N, K, Kb, sc4);
+  bool streamable = stream_on && stream_supported(mode, M, N, K, Kb, sc4) &&
+                    (ragged || stream_whole(mode, K, Kb, sc16));
   // The streaming kernel's time grows with the number of 64-row activation
   // blocks times N (each block streams all of W, and each W slice re-reads
   // its activation rows), while the 128x128 / persistent tiles stay at about
@@ -280,7 +284,7 @@ static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc1
   // (ragged K: from half the CUs; 768x1640x4168, 78 tiles, 58 us on them
   // against about 40 streamed)
   const bool bf16_pipe_round = mode == MODE_BF16 && pipe_forced != -2 && M > 64 &&
-                               (Kb % 128 == 0 || 2 * t128 >= device_cu_count()) &&
+                               (Kb % 128 == 0 || (ragged && 2 * t128 >= device_cu_count())) &&
                                N > 64 && t128 >= 40 && t128 <= device_cu_count();
   if (streamable && !skinny_stream && M > 32 && (mode != MODE_NVFP4 || M > 256)) {
     const int bm = stream_blocks64(mode, M, K, Kb, sc16) ? 64 : 32;
@@ -346,7 +350,7 @@ static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc1
       r.path = PATH_PIPE;
       r.variant = 1;
     } else if (persist_on && 6 * t256 >= device_cu_count() && (int64_t)M * N >= 2400000 &&
-               persist_supported(mode, M, N, K, Kb, sc4)) {
+               persist_supported(mode, M, N, K, Kb, sc4) && (ragged || Kb % 128 == 0)) {
       r.path = PATH_PERSIST;
     }
     return r;
@@ -356,9 +360,11 @@ static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc1
   // only the scale rows are ragged)
   const bool fp4 = mode == MODE_MXFP4 || mode == MODE_NVFP4;
   const bool rag = Kb % 128 != 0, pad = fp4 && !persist_whole(mode, K, Kb, sc16);
-  const bool pipe_ok = pipe_forced != -2 && (mode == MODE_FP8_TENSOR || sc4) && (!rag || !fp4 || padded);
+  const bool pipe_ok = pipe_forced != -2 && (mode == MODE_FP8_TENSOR || sc4) &&
+                       (!rag || (ragged && (!fp4 || padded)));
   const bool persist_ok = persist_on && pipe_forced < 0 &&
-                          persist_supported(mode, M, N, K, Kb, sc4) && (!pad || padded);
+                          persist_supported(mode, M, N, K, Kb, sc4) && (!pad || padded) &&
+                          (ragged || persist_whole(mode, K, Kb, sc16));
   if (pipe_ok) {
     const int64_t t256 = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
     // Rounds of tiles per CU: a round of 256x256 persistent tiles costs
@@ -399,15 +405,21 @@ bool gemm_routes_to_stream(int mode, int64_t M, int64_t N, int64_t K, bool or_pi
   return path == PATH_STREAM || (or_pipe && path == PATH_PIPE && (!accumulate || !mode_grouped_k(mode)));
 }
 
-size_t gemm_workspace_bytes(int mode, int64_t M, int64_t N, int64_t K, bool accumulate, bool padded) {
+size_t gemm_workspace_required(int mode, int64_t M, int64_t N, int64_t K, bool accumulate) {
   const int Kb = (mode == MODE_MXFP4 || mode == MODE_NVFP4) ? (int)(K / 2)
                                                             : (mode == MODE_BF16 ? (int)(2 * K) : (int)K);
-  Route r = route_for(mode, (int)M, (int)N, (int)K, Kb, true, true, padded);
+  Route r = route_for(mode, (int)M, (int)N, (int)K, Kb, true, true, false, false);
   if (accumulate) r.path = PATH_TILED;
-  if (r.pad_scales && r.path != PATH_TILED) return (size_t)(M + N) * (size_t)padded_pitch(mode, (int)K);
   return (r.path == PATH_TILED && r.tiled.ksplit > 1)
              ? (size_t)r.tiled.ksplit * (size_t)splitk_slice(M, N) * sizeof(float)
              : 0;
+}
+
+size_t gemm_workspace_bytes(int mode, int64_t M, int64_t N, int64_t K, bool accumulate) {
+  const size_t need = gemm_workspace_required(mode, M, N, K, accumulate);
+  if (accumulate || (mode != MODE_MXFP4 && mode != MODE_NVFP4)) return need;
+  const Route r = route_for(mode, (int)M, (int)N, (int)K, (int)(K / 2), true, true, true);
+  return r.pad_scales ? std::max(need, (size_t)(M + N) * (size_t)padded_pitch(mode, (int)K)) : need;
 }
 
 hipError_t launch_gemm(int mode, GemmArgs p, hipStream_t st) {

@@ -109,6 +109,8 @@ hipError_t launch_gemm_decode(int mode, const GemmArgs &p, hipStream_t st);
 // scales 4-byte aligned).  The router takes it while ceil(M/64) * N stays
 // below a per-mode edge (gemm_tiled.hip, route_for).
 bool stream_supported(int mode, int M, int N, int K, int Kb, bool scales4);
+// Whole 256-byte chunks and scale rows of whole 16-byte parts.
+bool stream_whole(int mode, int K, int Kb, bool scales16);
 // Whether M > 32 rows stream in 64-row blocks, else in 32-row blocks.
 bool stream_blocks64(int mode, int M, int K, int Kb, bool scales16);
 hipError_t launch_gemm_stream(int mode, const GemmArgs &p, hipStream_t st);
@@ -116,10 +118,12 @@ hipError_t launch_gemm_stream(int mode, const GemmArgs &p, hipStream_t st);
 // Picks a kernel variant for the shape and launches it (plus the split-K
 // finalize kernel, which adds the slices in split order, when ksplit > 1).
 hipError_t launch_gemm(int mode, GemmArgs args, hipStream_t st);
-// Workspace the launcher will need for this shape (0 if none); padded false:
-// what it can do with where it cannot copy ragged scale rows to a padded pitch.
-size_t gemm_workspace_bytes(int mode, int64_t M, int64_t N, int64_t K, bool accumulate = false,
-                            bool padded = true);
+// Workspace a call must bring for this shape (0 if none): the split-K slices
+// of the shapes that have no kernel for whole rows.  gemm_workspace_bytes adds
+// the room in which ragged MXFP4 / NVFP4 scale rows are copied to a padded
+// pitch; without it those take a kernel that does not need the copy.
+size_t gemm_workspace_required(int mode, int64_t M, int64_t N, int64_t K, bool accumulate = false);
+size_t gemm_workspace_bytes(int mode, int64_t M, int64_t N, int64_t K, bool accumulate = false);
 // Whether launch_gemm takes the streaming kernel (or_pipe: or the pipelined
 // tiles) for this shape (aligned scales; accumulate: C += result, fp32 out).
 bool gemm_routes_to_stream(int mode, int64_t M, int64_t N, int64_t K, bool or_pipe = false,

@@ -54,6 +54,10 @@ def rmsnorm_quant(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6, *,
                   fmt: str = "fp8", return_y: bool = False):
     """RMSNorm of ``x [rows, cols]`` (bf16) with ``weight [cols]`` (bf16 or
     fp32), quantized.  Returns ``(q, scales)`` or ``(q, scales, y)``."""
+    if not return_y and fmt in _FMTS:
+        r = N.fast().rmsnorm_quant(x, weight, eps, _FMTS[fmt])
+        if r is not None:
+            return r
     x = _rows2d(x, "rmsnorm_quant")
     rows, cols = x.shape
     if weight.dim() != 1 or weight.numel() != cols:
@@ -75,6 +79,10 @@ def rmsnorm_quant(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6, *,
 def swiglu_quant(input: torch.Tensor, *, fmt: str = "fp8", return_y: bool = False):
     """SwiGLU of ``input [rows, 2H]`` (bf16; gate = first H, up = last H),
     quantized.  Returns ``(q, scales)`` or ``(q, scales, y)``."""
+    if not return_y and fmt in _FMTS:
+        r = N.fast().swiglu_quant(input, _FMTS[fmt])
+        if r is not None:
+            return r
     x = _rows2d(input, "swiglu_quant")
     rows, two_h = x.shape
     if two_h % 2:

@@ -209,6 +209,11 @@ def fp8_gemm_packed(qa, qw, scale_a, scale_b, *, block: bool = False, group: boo
     """
     if block and group:
         raise ValueError("block and group scales are exclusive")
+    if out is None:
+        c = N.fast().fp8_gemm(qa, qw, scale_a, scale_b, N.SCALE_BLOCK128 if block else
+                              (N.SCALE_GROUP128 if group else N.SCALE_TENSOR), out_dtype)
+        if c is not None:
+            return c
     dev = _require_gpu(qa, qw, scale_a, scale_b)
     qa, qw = N.vec_rows(_u8(qa)), N.vec_rows(_u8(qw))
     M, K = qa.shape
@@ -239,6 +244,11 @@ def fp4_gemm_packed(qa, sa, qw, sw, *, fmt: str = "mxfp4", global_a=None, global
     """GEMM on packed E2M1 codes: qa [M, K/2], qw [N, K/2] uint8 (low nibble =
     even K).  MXFP4: sa [M, K/32], sw [N, K/32] E8M0 bytes.  NVFP4: sa [M, K/16],
     sw [N, K/16] E4M3 bytes plus 1-element float32 global scales."""
+    if out is None and (fmt == "mxfp4" or fmt == "nvfp4"):
+        c = N.fast().fp4_gemm(qa, sa, qw, sw, N.FMT_MXFP4 if fmt == "mxfp4" else N.FMT_NVFP4, global_a,
+                              global_w, out_dtype)
+        if c is not None:
+            return c
     dev = _require_gpu(qa, qw, sa, sw)
     qa, qw = N.vec_rows(_u8(qa)), N.vec_rows(_u8(qw))
     sa, sw = _u8(sa).contiguous(), _u8(sw).contiguous()
@@ -275,6 +285,10 @@ def grouped_fp8_gemm_packed(qx, sx, qw, sw, offsets, *, out_dtype=torch.bfloat16
     device (offsets[0] = 0, offsets[G] = T, non-decreasing), sx [T] per-row
     scales, sw [G, N] per-channel scales.  Returns y [T, N].
     """
+    if out is None:
+        y = N.fast().grouped_fp8_gemm(qx, sx, qw, sw, offsets, out_dtype)
+        if y is not None:
+            return y
     dev = _require_gpu(qx, qw, sx, sw, offsets)
     qx, qw = N.vec_rows(_u8(qx)), N.vec_rows(_u8(qw))
     T, K = qx.shape
@@ -306,6 +320,10 @@ def bf16_gemm(A: torch.Tensor, B: torch.Tensor, *, out_dtype: torch.dtype = torc
     contiguous W [N, K] is read in place; any other layout of B (or a
     non-contiguous A) is first copied to K-major rows on the GPU.
     """
+    if out is None:
+        c = N.fast().bf16_gemm(A, B, out_dtype)
+        if c is not None:
+            return c
     if A.dim() != 2 or B.dim() != 2:
         raise ValueError("bf16_gemm expects A [M, K] and B [K, N]")
     if A.dtype != torch.bfloat16 or B.dtype != torch.bfloat16:
@@ -334,6 +352,9 @@ def lora_fused_gemm(X: torch.Tensor, W: torch.Tensor, loraA: torch.Tensor, loraB
     place), loraA [L, K, R], loraB [L, R, N], all bf16; scales: L numbers or
     a float tensor [L].  K % 8 == 0 and L * R % 8 == 0.
     """
+    y = N.fast().lora_gemm(X, W, loraA, loraB, scales)
+    if y is not None:
+        return y
     for t, nm in ((X, "X"), (W, "W"), (loraA, "loraA"), (loraB, "loraB")):
         if t.dtype != torch.bfloat16:
             raise TypeError(f"lora_fused_gemm: {nm} must be bfloat16 (got {t.dtype})")

@@ -224,6 +224,10 @@ def routed_grouped_gemm(x: torch.Tensor, topk_ids: torch.Tensor, topk_weights: t
         raise ValueError("topk_ids must be [tokens, topk]")
     T, topk = topk_ids.shape
     if gather_applies(T, topk, E, qw.shape[2]):
+        out = N.fast().moe_projection(x, topk_ids, topk_weights, qw, sw,
+                                      route_quant_applies(T, topk, E, qw.shape[2]), out_dtype)
+        if out is not None:
+            return out
         # token-major codes, A rows through the row map: no permuted copy
         # (route and quantize in one launch at decode size)
         route, qx, sx = moe_route_quant_tokens(topk_ids, x, E)

@@ -45,6 +45,9 @@ def _workspace(x: torch.Tensor) -> torch.Tensor:
 
 
 def quant_fp8_tensor(x: torch.Tensor):
+    r = N.fast().quant_fp8_tensor(x)
+    if r is not None:
+        return r
     x, xd = _check(x, "quant_fp8_tensor")
     R, C = x.shape
     q = torch.empty((R, C), dtype=torch.uint8, device=x.device)
@@ -57,6 +60,9 @@ def quant_fp8_tensor(x: torch.Tensor):
 
 
 def quant_fp8_blocks(x: torch.Tensor, group_rows: int, group_cols: int):
+    r = N.fast().quant_fp8_blocks(x, group_rows, group_cols)
+    if r is not None:
+        return r
     x, xd = _check(x, "quant_fp8_blocks")
     R, C = x.shape
     q = torch.empty((R, C), dtype=torch.uint8, device=x.device)
@@ -69,6 +75,9 @@ def quant_fp8_blocks(x: torch.Tensor, group_rows: int, group_cols: int):
 
 
 def quant_mxfp4(x: torch.Tensor):
+    r = N.fast().quant_mxfp4(x)
+    if r is not None:
+        return r
     x, xd = _check(x, "quant_mxfp4")
     R, C = x.shape
     if C % 32:
@@ -82,6 +91,9 @@ def quant_mxfp4(x: torch.Tensor):
 
 
 def quant_nvfp4(x: torch.Tensor):
+    r = N.fast().quant_nvfp4(x)
+    if r is not None:
+        return r
     x, xd = _check(x, "quant_nvfp4")
     R, C = x.shape
     if C % 16:
