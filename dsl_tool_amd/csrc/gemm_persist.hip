@@ -73,13 +73,13 @@
 
 namespace dsl {
 
-template <int MODE_, bool GROUPED_ = false, bool GATHER_ = false, bool RAG_ = false>
+template <int MODE_, bool GROUPED_ = false, bool GATHER_ = false, bool RAG_ = false, int BN_ = 256>
 struct PersCfg {
   static constexpr int MODE = MODE_;
   static constexpr bool RAG = RAG_;            // ragged K / scale rows
   static constexpr bool GROUPED = GROUPED_;    // FP8 grouped (MoE) tile walk
   static constexpr bool GATHER = GATHER_;      // grouped: A rows through a row table
-  static constexpr int BM = 256, BN = 256, WGM = 2, WGN = 4;
+  static constexpr int BM = 256, BN = BN_, WGN = BN / 64, WGM = 8 / WGN;   // waves of 64 columns
   static constexpr int NW = WGM * WGN, NT = NW * 64, OCC = 2;
   static constexpr int WM = BM / WGM, WN = BN / WGN, TM = WM / 32, TN = WN / 32;
   static constexpr bool BLOCK = MODE == MODE_FP8_BLOCK;
@@ -108,11 +108,17 @@ struct PersCfg {
   static constexpr int SA_DMA = SQA / 1024, SB_DMA = SQB / 1024;
   static constexpr int DATA_DMA = A_DMA + B_DMA, SC_DMA = SA_DMA + SB_DMA;
   static constexpr int DD = DATA_DMA / NW, DS = (SC_DMA + NW - 1) / NW, D = DD + DS;
-  static_assert(DATA_DMA % NW == 0 && A_DMA % DD == 0, "whole waves per operand");
-  static_assert(!RAG || NT == BM + BN, "one row per thread");
+  static_assert(DATA_DMA % NW == 0, "the same copies per wave");
+  // 256x128 tiles: 48 copies per pair, six per wave, so a wave may copy rows of
+  // both operands
+  static constexpr bool MIXED = A_DMA % DD != 0;
+  static constexpr int PARTS = NV ? 4 : TM;            // MFMA rows of a step (NVFP4: its four block parts)
+  static_assert(BN == 256 || BN == 128, "tile width");
+  static_assert(!RAG || NT >= BM + BN, "one row per thread");
   static_assert(DS <= 1, "at most one scale DMA per wave and quad");
   static_assert(LDS <= 160 * 1024, "LDS budget");
   static_assert(!BLOCK || (WN <= 128 && 128 % WN == 0), "one weight-scale block per wave");
+  static_assert(!GROUPED || BN == 256, "grouped: 256x256 tiles");
   static_assert(!GROUPED || MODE == MODE_FP8_TENSOR, "grouped: FP8 with row x channel scales");
   static_assert(!GROUPED || NW == 8, "grouped: one epilogue-scale DMA per wave");
   static_assert(!GATHER || (GROUPED && A_DMA == 4 * DD), "gather: A copied by waves 0-3");
@@ -204,6 +210,8 @@ template <class Cfg>
 struct Ring {
   const uint8_t *dbase;          // operand rows of the tile, pair 0
   const uint8_t *dbase2;         // second K segment's rows (pairs nk1 ..), BF16
+                                 // (MIXED: W's rows; no second segment)
+  int lim2;                      // MIXED: last valid W row of the tile
   const uint8_t *sbase;          // scale rows of the tile, quad 0
   int wrow;                      // the wave's first tile row (uniform)
   int lim;                       // last valid tile row of the operand (uniform)
@@ -229,7 +237,7 @@ struct Ring {
       nk1 = lastq + 1;
     }
     full = Cfg::DS > 0 && wave < Cfg::SC_DMA;
-    isA = wave * Cfg::DD < Cfg::A_DMA;
+    isA = Cfg::MIXED || wave * Cfg::DD < Cfg::A_DMA;
     kb2 = isA || ldb2_ == 0 ? kb2_ : ldb2_;
     rmask = isA || rep2_ == 0 ? 0x7fffffff : rep2_ - 1;
     lim = (isA ? tr.arows : tr.brows) - 1;
@@ -238,6 +246,10 @@ struct Ring {
     dbase = isA ? tr.a : tr.b;
     dbase2 = isA ? tr.a2 : tr.b2;
     vsub = lane / Cfg::CH;
+    if constexpr (Cfg::MIXED) {
+      dbase2 = tr.b;
+      lim2 = tr.brows - 1;
+    }
     // DMA j covers tile rows wrow + j*RPI + vsub; RPI is even, so the row
     // swizzle only depends on vsub and the parity of wrow/RPI + j
     vchunk = (uint32_t)(((lane % Cfg::CH) ^ pair_swz(wrow + (int)vsub)) * 16);
@@ -272,6 +284,23 @@ struct Ring {
 
   // operand DMA j of tile-local pair q into the pair slot at `slot`
   DSL_DEV void issue_data(int j, int q, uint32_t slot) const {
+    if constexpr (Cfg::MIXED) {
+      // copy i of the pair: 8 rows of A, then of W (uniform selects); the
+      // rows' swizzle differs from the lane's by bit 2 on odd copies
+      const int i = wave * Cfg::DD + j;
+      const bool a = i < Cfg::A_DMA;
+      int r = (int)vsub + (a ? i : i - Cfg::A_DMA) * Cfg::RPI;
+      const int l = a ? lim : lim2;
+      r = r < l ? r : l;
+      uint32_t ch = vchunk ^ (uint32_t)(((i ^ wave * Cfg::DD) & 1) * 64);
+      if constexpr (Cfg::RAG) {
+        const uint32_t most = (uint32_t)(q == lastq ? kb - 16 - q * Cfg::PKB : Cfg::PKB - 16);
+        ch = ch < most ? ch : most;
+      }
+      dma16((a ? dbase : dbase2) + (int64_t)q * Cfg::PKB, __umul24((uint32_t)r, (uint32_t)kb) + ch,
+            slot + (uint32_t)(i * 1024));
+      return;
+    }
     int r = (int)vsub + (wrow + j * Cfg::RPI);
     r = r < lim ? r : lim;           // rows past the edge re-read the last row
     // swz(wrow + j*RPI + vsub) = swz(wrow + vsub) ^ swz(j*RPI): the row
@@ -756,9 +785,10 @@ void gemm_persist_kernel(const Args p) {
   auto issue_part = [&](int i, int qq, uint32_t islot, bool quad) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < Cfg::DD; ++j)
-      if (i < 0 || (j >= i * Cfg::DD / TM && j < (i + 1) * Cfg::DD / TM)) ring.issue_data(j, qq, islot);
+      if (i < 0 || (j >= i * Cfg::DD / Cfg::PARTS && j < (i + 1) * Cfg::DD / Cfg::PARTS))
+        ring.issue_data(j, qq, islot);
     if constexpr (Cfg::SCALED) {
-      if (i < 0 || i == TM - 1)
+      if (i < 0 || i == Cfg::PARTS - 1)
         ring.issue_scales(__builtin_amdgcn_readfirstlane((int)(quad && ring.full)), qq / Cfg::QP,
                           pipe::lds_addr(squad) + (uint32_t)((iqc & 1) * Cfg::SQ));
     }
@@ -952,7 +982,7 @@ void gemm_persist_kernel(const Args p) {
   auto cut_pair = [&](int slot) __attribute__((always_inline)) {
     if (nv < 8) {
       const int row = wave * 64 + pers::lane_id();
-      for (int c = nv; c < 8; ++c)
+      for (int c = nv; c < 8 && row < Cfg::BM + Cfg::BN; ++c)
         *reinterpret_cast<uint4 *>(smem + slot * Cfg::PAIR + row * Cfg::PKB +
                                    ((c ^ pers::pair_swz(row)) << 4)) = make_uint4(0, 0, 0, 0);
       pipe::wait_lds();
@@ -992,9 +1022,9 @@ void gemm_persist_kernel(const Args p) {
     fb[1].share_scales(fb[0]);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
+    for (int i = 0; i < Cfg::PARTS; ++i) {
       if constexpr (Cfg::NV) {
-        pers::nv_part<Cfg, FRESH>(i, fa, fb[0], acc, i == TM - 1,
+        pers::nv_part<Cfg, FRESH>(i, fa, fb[0], acc, i == Cfg::PARTS - 1,
                            [&](int r) __attribute__((always_inline)) { fa.load_a(st, sq, sw, 1, r, wm, r32, h); });
       } else {
         if constexpr (RESCALE) {
@@ -1042,9 +1072,9 @@ void gemm_persist_kernel(const Args p) {
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
+    for (int i = 0; i < Cfg::PARTS; ++i) {
       if constexpr (Cfg::NV) {
-        pers::nv_part<Cfg, false>(i, fa, fb[1], acc, KIND != 2 && i == TM - 1,
+        pers::nv_part<Cfg, false>(i, fa, fb[1], acc, KIND != 2 && i == Cfg::PARTS - 1,
                            [&](int r) __attribute__((always_inline)) { fa.load_a(stn, sqn, sw, 0, r, wm, r32, h); });
         issue_part(i, qq, islot, quad);
       } else {
@@ -1113,9 +1143,9 @@ int device_cu_count() {
   return cached[dev];
 }
 
-template <int MODE, bool RAG>
+template <int MODE, bool RAG, int BN>
 static hipError_t launch_persist_cfg(const GemmArgs &p, hipStream_t st) {
-  using Cfg = PersCfg<MODE, false, false, RAG>;
+  using Cfg = PersCfg<MODE, false, false, RAG, BN>;
   const int ntiles = ((p.M + Cfg::BM - 1) / Cfg::BM) * ((p.N + Cfg::BN - 1) / Cfg::BN);
   int grid = device_cu_count();
   if (grid > ntiles) grid = ntiles;
@@ -1130,15 +1160,15 @@ bool persist_whole(int mode, int K, int Kb, bool scales16) {
   return true;
 }
 
-template <int MODE>
+template <int MODE, int BN>
 static hipError_t launch_persist_mode(const GemmArgs &p, hipStream_t st) {
   const uintptr_t sc = reinterpret_cast<uintptr_t>(p.sa) | reinterpret_cast<uintptr_t>(p.sb);
   if (p.sld == 0 && persist_whole(MODE, p.K, p.Kb, (sc & 15) == 0))
-    return launch_persist_cfg<MODE, false>(p, st);
+    return launch_persist_cfg<MODE, false, BN>(p, st);
   // ragged E8M0 / E4M3 rows come at a padded, 16-byte aligned pitch
   if ((MODE == MODE_MXFP4 || MODE == MODE_NVFP4) && (p.sld < 16 || p.sld % 16 != 0 || (sc & 15) != 0))
     return hipErrorInvalidValue;
-  return launch_persist_cfg<MODE, true>(p, st);
+  return launch_persist_cfg<MODE, true, BN>(p, st);
 }
 
 bool persist_supported(int mode, int M, int N, int K, int Kb, bool scales4) {
@@ -1151,15 +1181,21 @@ bool persist_supported(int mode, int M, int N, int K, int Kb, bool scales4) {
   return mode == MODE_MXFP4 || mode == MODE_NVFP4;
 }
 
-hipError_t launch_gemm_persist(int mode, const GemmArgs &p, hipStream_t st) {
+template <int BN>
+static hipError_t launch_persist_bn(int mode, const GemmArgs &p, hipStream_t st) {
   switch (mode) {
-    case MODE_FP8_TENSOR: return launch_persist_mode<MODE_FP8_TENSOR>(p, st);
-    case MODE_FP8_BLOCK: return launch_persist_mode<MODE_FP8_BLOCK>(p, st);
-    case MODE_MXFP4: return launch_persist_mode<MODE_MXFP4>(p, st);
-    case MODE_NVFP4: return launch_persist_mode<MODE_NVFP4>(p, st);
-    case MODE_BF16: return launch_persist_mode<MODE_BF16>(p, st);
+    case MODE_FP8_TENSOR: return launch_persist_mode<MODE_FP8_TENSOR, BN>(p, st);
+    case MODE_FP8_BLOCK: return launch_persist_mode<MODE_FP8_BLOCK, BN>(p, st);
+    case MODE_MXFP4: return launch_persist_mode<MODE_MXFP4, BN>(p, st);
+    case MODE_NVFP4: return launch_persist_mode<MODE_NVFP4, BN>(p, st);
+    case MODE_BF16: return launch_persist_mode<MODE_BF16, BN>(p, st);
     default: return hipErrorInvalidValue;
   }
+}
+
+hipError_t launch_gemm_persist(int mode, const GemmArgs &p, hipStream_t st, bool narrow) {
+  if (narrow && p.Kb2 == 0) return launch_persist_bn<128>(mode, p, st);
+  return launch_persist_bn<256>(mode, p, st);
 }
 
 bool grouped_persist_supported(const GroupedArgs &p) {

@@ -218,6 +218,7 @@ struct Route {
   int path;
   int variant;    // PATH_PIPE variant
   Plan tiled;     // PATH_TILED plan
+  bool narrow = false;       // PATH_PERSIST: 256x128 tiles
   bool pad_scales = false;   // PATH_PERSIST / PATH_PIPE: E8M0 / E4M3 rows first copied to a padded pitch
 };
 
@@ -334,6 +335,19 @@ static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc1
     r.path = PATH_STREAM;
     return r;
   }
+  // 256x128 persistent tiles where one round of them holds a problem that
+  // takes the 128x128 tiles more than one round (and the 256x256 ones half a
+  // round at most).  One full round costs about 0.65 of a full 256x256 round,
+  // one of 128x128 tiles 0.41, two 0.72 (per-tensor K=4096: 37.3, 57.8, 23.5,
+  // 41.9 us).  us before -> after, per-tensor / block / MXFP4 / NVFP4 / bf16:
+  // 1500x4096x11008 109 -> 83, 109 -> 98, 71 -> 60, 222 -> 159, 188 -> 160;
+  // 2048x4096x4096 42 -> 37, 45 -> 42, 31 -> 28, 90 -> 70, 80 -> 70.  NVFP4,
+  // whose 128x128 tiles spend most of a stage dequantizing, from 0.6 rounds of
+  // those (1024x4096x4096 74 -> 60; 512x4096x4096, half a round, 40 -> 44).
+  const int64_t tn = (int64_t)((M + 255) / 256) * ((N + 127) / 128), cu = device_cu_count();
+  const bool narrow = ragged && persist_on && pipe_forced < 0 && M > 128 && N > 128 && tn <= cu &&
+                      (mode == MODE_NVFP4 ? 10 * t128 > 6 * cu : t128 > cu) &&
+                      persist_supported(mode, M, N, K, Kb, sc4);
   if (mode == MODE_BF16) {   // pipelined, persistent or register-staged tiles
     const int64_t t256 = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
     // one round of 128x128 pipelined tiles (40 to one per CU) beats a
@@ -352,6 +366,10 @@ static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc1
     } else if (persist_on && 6 * t256 >= device_cu_count() && (int64_t)M * N >= 2400000 &&
                persist_supported(mode, M, N, K, Kb, sc4) && (ragged || Kb % 128 == 0)) {
       r.path = PATH_PERSIST;
+    }
+    if (narrow) {
+      r.path = PATH_PERSIST;
+      r.narrow = true;
     }
     return r;
   }
@@ -392,6 +410,10 @@ static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc1
       r.variant = 1;
     }
   }
+  if (narrow && persist_ok) {
+    r.path = PATH_PERSIST;
+    r.narrow = true;
+  }
   r.pad_scales = (r.path == PATH_PERSIST && pad) || (r.path == PATH_PIPE && fp4 && rag);
   return r;
 }
@@ -420,6 +442,40 @@ size_t gemm_workspace_bytes(int mode, int64_t M, int64_t N, int64_t K, bool accu
   if (accumulate || (mode != MODE_MXFP4 && mode != MODE_NVFP4)) return need;
   const Route r = route_for(mode, (int)M, (int)N, (int)K, (int)(K / 2), true, true, true);
   return r.pad_scales ? std::max(need, (size_t)(M + N) * (size_t)padded_pitch(mode, (int)K)) : need;
+}
+
+// The columns [n1, N) of a problem (n1 a multiple of 256).
+static GemmArgs columns_from(int mode, GemmArgs p, int n1) {
+  p.b += (int64_t)n1 * p.Kb;
+  p.c = static_cast<uint8_t *>(p.c) + (int64_t)n1 * (p.out_f32 ? 4 : 2);
+  if (p.sb) {
+    const int64_t off = mode == MODE_FP8_BLOCK ? (int64_t)(n1 / 128) * ((p.K + 127) / 128) * 4
+                                               : (int64_t)n1 * scale_row_len(mode, p.K);
+    p.sb = static_cast<const uint8_t *>(p.sb) + off;
+  }
+  p.N -= n1;
+  p.ws = nullptr;
+  p.ws_bytes = 0;
+  return p;
+}
+
+// Columns to take off a persistent launch so that its 256x256 tiles fill whole
+// rounds, the rest going to a second launch of smaller tiles: a last round of
+// a few tiles costs most of a full one (K=4096: 64 tiles 0.73 of it), the same
+// columns in 128x128 tiles 0.41 at most.  0: leave it whole.  Taken where the
+// columns are at most a quarter of the CUs' worth of tiles, which one round of
+// 128x128 tiles (or the streaming kernel) holds.  us before -> after,
+// per-tensor / block / MXFP4 / NVFP4 / bf16: 2304x7680x4096 (270 tiles) 90 ->
+// 75, 106 -> 93, 63 -> 58, 190 -> 178, 177 -> 145; 4300x4300x4096 (289 tiles)
+// 141 -> 116, 158 -> 132, 113 -> 101, 241 -> 218, 230 -> 185.
+static int strip_columns(const GemmArgs &p) {
+  const int cu = device_cu_count();
+  const int nbm = (p.M + 255) / 256, nbn = (p.N + 255) / 256;
+  const int64_t tiles = (int64_t)nbm * nbn, full = tiles / cu * cu;
+  if (p.accumulate || full == 0 || tiles == full || nbm > cu / 4) return 0;
+  const int keep = (int)(full / nbm);                // whole columns of tiles in whole rounds
+  if ((int64_t)nbm * (nbn - keep) > cu / 4 || keep < 1) return 0;
+  return p.N - keep * 256;
 }
 
 hipError_t launch_gemm(int mode, GemmArgs p, hipStream_t st) {
@@ -479,7 +535,19 @@ hipError_t launch_gemm(int mode, GemmArgs p, hipStream_t st) {
       p.sld = pitch;
     }
     if (r.path == PATH_PIPE) return launch_gemm_pipe(mode, p, r.variant, st);
-    return launch_gemm_persist(mode, p, st);
+    const int strip = r.narrow || r.pad_scales ? 0 : strip_columns(p);
+    if (strip > 0) {
+      GemmArgs main = p;
+      main.N = p.N - strip;
+      const hipError_t e = launch_gemm_persist(mode, main, st, false);
+      if (e != hipSuccess) return e;
+      const GemmArgs rest = columns_from(mode, p, main.N);
+      return route_for(mode, rest.M, rest.N, rest.K, rest.Kb, (sc & 3) == 0, (sc & 15) == 0, false).path ==
+                     PATH_STREAM
+                 ? launch_gemm_stream(mode, rest, st)
+                 : launch_gemm_pipe(mode, rest, 1, st);
+    }
+    return launch_gemm_persist(mode, p, st, r.narrow);
   }
   const Plan pl = r.tiled;
   // split-K into as many [M][N] fp32 slices as the workspace holds (at most

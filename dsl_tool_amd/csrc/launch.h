@@ -95,7 +95,8 @@ bool persist_supported(int mode, int M, int N, int K, int Kb, bool scales4);
 // Rows of whole pairs and scale rows of whole quads.  Other MXFP4 / NVFP4
 // scale rows must come at a padded pitch (GemmArgs::sld).
 bool persist_whole(int mode, int K, int Kb, bool scales16);
-hipError_t launch_gemm_persist(int mode, const GemmArgs &p, hipStream_t st);
+// narrow: 256x128 tiles (no second K segment).
+hipError_t launch_gemm_persist(int mode, const GemmArgs &p, hipStream_t st, bool narrow = false);
 
 // Skinny-M kernels, one launch, no workspace (Kb % 1024 == 0):
 //   M <= 32: FP8_TENSOR and BF16; FP8_BLOCK and MXFP4 with 16-byte aligned scales

@@ -151,3 +151,12 @@ def test_padded_scale_rows_need_their_workspace():
         N.call("dsl_fp4_gemm", qa.data_ptr(), qw.data_ptr(), c.data_ptr(), m, n, k, n, N.OUT_BF16,
                N.FMT_MXFP4, sa.data_ptr(), sw.data_ptr(), None, None, p, b, N.stream_of(a.device))
         assert_close(c, np_f32(want), what=f"mxfp4 workspace {b}")
+
+
+# 256x128 persistent tiles (one round of them, more than one of 128x128), whole
+# and ragged K, and a problem of one round and a few tiles more, whose last
+# columns run as a second launch
+@pytest.mark.parametrize("mode", ["tensor", "block", "mxfp4", "nvfp4", "bf16"])
+@pytest.mark.parametrize("m,n,k", [(1300, 2500, 512), (1281, 4000, 608), (4100, 4200, 512), (2100, 7500, 256)])
+def test_narrow_tiles_and_column_strips(mode, m, n, k):
+    check(mode, m, n, k)
