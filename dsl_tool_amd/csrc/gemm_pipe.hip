@@ -157,6 +157,12 @@ void gemm_pipe_kernel(const GemmArgs p) {
 // (MODE_FP8_GCOL, sb[g][n] as fp8_gemm_groupwise_kernel reads them) the
 // stage also carries the tile's BN weight scales of its group, and each
 // lane folds part * (sa[m,g] * sb[g,n]) for its own four columns.
+//
+// Rings of more than two stages keep the tile's weight-block scales in LDS
+// (at most kBlockPfMaxGroups groups): read from memory in the loop they are a
+// vector load, whose wait drains the ring's copies in flight.
+constexpr int kBlockPfMaxGroups = 512;
+
 template <class Cfg>
 __global__ __launch_bounds__(Cfg::NT) __attribute__((amdgpu_waves_per_eu(Cfg::OCC, Cfg::OCC)))
 void gemm_pipe_block_kernel(const GemmArgs p) {
@@ -182,6 +188,13 @@ void gemm_pipe_block_kernel(const GemmArgs p) {
   const int sblim = (p.N + 127) / 128 - 1;
   sbrow = sbrow > sblim ? sblim : sbrow;
   const float *sbp = static_cast<const float *>(p.sb) + (int64_t)sbrow * nkg;
+  constexpr bool SBL = !Cfg::GCOL && NS > 2;
+  static_assert(!SBL || Cfg::BN <= 128, "one weight-scale block per tile");
+  __shared__ float sb_lds[SBL ? kBlockPfMaxGroups : 1];
+  if constexpr (SBL) {                 // published by the first stage's barrier
+    for (int g = threadIdx.x; g < nkg; g += Cfg::NT) sb_lds[g] = sbp[g];
+    pipe::wait_lds();
+  }
 
   // Eight waves (two per SIMD; waves w and w + 4 share one): a wave cannot
   // issue its MFMAs until its nine copies have gone out, and copies issue at
@@ -213,10 +226,12 @@ void gemm_pipe_block_kernel(const GemmArgs p) {
     for (int j = 0; j < TN; ++j) acc[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
 
   for (int ks = 0; ks < nks; ++ks) {
-    const float sbv = Cfg::GCOL ? 1.f : sbp[ks];
-    if (ks + NS - 2 < nks) pipe::wait_vmcnt<(NS - 2) * D>();
-    else pipe::wait_vmcnt<0>();
+    float sbv = 1.f;
+    if constexpr (!Cfg::GCOL && !SBL) sbv = sbp[ks];
+    // waves issue D or D-1 copies per stage; at the end fewer stages follow
+    pipe::wait_stages_of<D, NS - 2>(nks - 1 - ks < NS - 2 ? nks - 1 - ks : NS - 2, ring.full);
     __syncthreads();
+    if constexpr (SBL) sbv = sb_lds[ks];
     pipe::cut_stage<Cfg>(ks, p.Kb, smem);
     const uint8_t *st = smem + (ks % NS) * Cfg::STAGE;
     const uint8_t *sA = st, *sB = st + Cfg::A_BYTES;
@@ -428,8 +443,6 @@ DSL_DEV void block_pf_step(int ks, int nks, bool rescale, int g_next, float sb_n
 
 // Preconditions (checked by the launcher): K % 512 == 0, K / 128 <=
 // kBlockPfMaxGroups, sa 16-byte aligned.
-constexpr int kBlockPfMaxGroups = 512;
-
 template <class Cfg>
 __global__ __launch_bounds__(Cfg::NT) __attribute__((amdgpu_waves_per_eu(Cfg::OCC, Cfg::OCC)))
 void gemm_pipe_block_pf_kernel(const GemmArgs p) {
@@ -576,17 +589,59 @@ static hipError_t launch_pipe_cfg(const GemmArgs &p, hipStream_t st) {
   return hipGetLastError();
 }
 
+// 64x128 tiles (variant 6), one workgroup per CU and four stages of 128 bytes:
+// where half a round of 128x128 tiles would leave CUs idle, a stage costs its
+// barrier and LDS latency rather than its MFMAs, so whole lines of K per
+// stage, three of them in flight.  512x4096x4096 (256 tiles), us before ->
+// after: per-tensor 17.5 -> 13.0, block 26.6 -> 18.2, groupwise 29.4 -> 18.8,
+// MXFP4 15.6 -> 11.6, bf16 33.2 -> 23.1 (64-byte stages: 14.3, -, -, 15.7,
+// 28.0).  RAG: rows of no whole (pairs of) stages.
+template <bool RAG>
+static hipError_t launch_pipe_small(int mode, const GemmArgs &p, hipStream_t st) {
+  switch (mode) {
+    case MODE_FP8_GCOL: return launch_pipe_cfg<PipeCfg<MODE_FP8_GCOL, 64, 128, 2, 4, 4, 128, 2, 0, RAG>>(p, st);
+    case MODE_FP8_BLOCK: return launch_pipe_cfg<PipeCfg<MODE_FP8_BLOCK, 64, 128, 2, 4, 4, 128, 2, 0, RAG>>(p, st);
+    case MODE_BF16: return launch_pipe_cfg<PipeCfg<MODE_BF16, 64, 128, 1, 4, 4, 128, 1, 1, RAG>>(p, st);
+    case MODE_FP8_TENSOR: return launch_pipe_cfg<PipeCfg<MODE_FP8_TENSOR, 64, 128, 1, 4, 4, 128, 1, 1, RAG>>(p, st);
+    case MODE_MXFP4: return launch_pipe_cfg<PipeCfg<MODE_MXFP4, 64, 128, 2, 4, 4, 128, 2, 0, RAG>>(p, st);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+// One round of 128x128 tiles (variant 7) on the same ring, eight waves for the
+// group-scaled forms: 1024x4096x4096, us against variant 1: per-tensor 19.9 /
+// 22.9, block 26.1 / 29.5, groupwise 27.7 / 32.2, MXFP4 17.4 / 21.3, bf16
+// 36.6 / 41.0.  With more tiles than CUs variant 1 (66 KB of LDS) interleaves
+// two workgroups on a CU and wins: groupwise 1500x4096x4096 38.4 / 48.6.
+template <bool RAG>
+static hipError_t launch_pipe_deep(int mode, const GemmArgs &p, hipStream_t st) {
+  switch (mode) {
+    case MODE_FP8_GCOL: return launch_pipe_cfg<PipeCfg<MODE_FP8_GCOL, 128, 128, 2, 4, 4, 128, 2, 0, RAG>>(p, st);
+    case MODE_FP8_BLOCK: return launch_pipe_cfg<PipeCfg<MODE_FP8_BLOCK, 128, 128, 2, 4, 4, 128, 2, 0, RAG>>(p, st);
+    case MODE_BF16: return launch_pipe_cfg<PipeCfg<MODE_BF16, 128, 128, 2, 2, 4, 128, 1, 1, RAG>>(p, st);
+    case MODE_FP8_TENSOR: return launch_pipe_cfg<PipeCfg<MODE_FP8_TENSOR, 128, 128, 2, 2, 4, 128, 1, 1, RAG>>(p, st);
+    case MODE_MXFP4: return launch_pipe_cfg<PipeCfg<MODE_MXFP4, 128, 128, 2, 4, 4, 128, 2, 0, RAG>>(p, st);
+    default: return hipErrorInvalidValue;
+  }
+}
+
 // Dense FP8 (per-tensor, block-scaled), MXFP4 and NVFP4 GEMM through the
 // LDS-DMA pipeline.  Preconditions (checked by the caller): Kb % 128 == 0 or
-// the RAG forms, 128x128 tiles whatever the variant (Kb % 16 == 0, MXFP4 /
+// the RAG forms, 128x128 or 64x128 tiles (Kb % 16 == 0, MXFP4 /
 // NVFP4 with padded scale rows; 256x256 per-column tiles spilled 80 bytes
 // there), ksplit == 1, 4-byte aligned scales.  Variant 0 is the default for large
-// grids, 1 the 128x128 tile for mid-sized ones; the others are kept as
-// alternatives for tuning (DSL_GEMM_PIPE).
+// grids, 1 the 128x128 tile for mid-sized ones, 7 (not NVFP4) for one round of
+// them, 6 (not NVFP4) the 64x128 tile; the others are kept as alternatives for
+// tuning (DSL_GEMM_PIPE).
 hipError_t launch_gemm_pipe(int mode, const GemmArgs &p, int variant, hipStream_t st) {
   // C += result: fp32 output through the plain epilogue only
   if (p.accumulate && (!p.out_f32 || mode_grouped_k(mode))) return hipErrorInvalidValue;
-  if (p.Kb % 128 != 0) {
+  // whole stages, an even number of them on the prefetch schedule
+  const bool pf = mode == MODE_FP8_TENSOR || mode == MODE_BF16;
+  const bool rag = p.Kb % 128 != 0, rag_deep = p.Kb % (pf ? 256 : 128) != 0;
+  if (variant == 6) return rag_deep ? launch_pipe_small<true>(mode, p, st) : launch_pipe_small<false>(mode, p, st);
+  if (variant == 7) return rag_deep ? launch_pipe_deep<true>(mode, p, st) : launch_pipe_deep<false>(mode, p, st);
+  if (rag) {
     switch (mode) {
       case MODE_FP8_GCOL:
         return launch_pipe_cfg<PipeCfg<MODE_FP8_GCOL, 128, 128, 2, 2, 2, 128, 2, 0, true>>(p, st);

@@ -287,6 +287,18 @@ static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc1
   const bool bf16_pipe_round = mode == MODE_BF16 && pipe_forced != -2 && M > 64 &&
                                (Kb % 128 == 0 || (ragged && 2 * t128 >= device_cu_count())) &&
                                N > 64 && t128 >= 40 && t128 <= device_cu_count();
+  // 64x128 pipelined tiles where one round of them holds the problem (not
+  // NVFP4, which streams): 1.3-1.5 times faster than the 128x128 tiles they
+  // replace there, and than the streaming kernel from a span of about 5
+  // (M=192 N=K=4096, streamed / tiles: per-tensor 11.5 / 10.8 us, block 17.6 /
+  // 16.1, groupwise 18.4 / 16.7; M=128 8.7 / 10.5, 10.0 / 15.9, 10.4 / 16.4);
+  // MXFP4 and bf16 keep their edge of 9 (M=256: 9.0 / 10.5, 18.8 / 19.6).  At
+  // least 24 tiles: fewer leave most CUs without one, and the register-staged
+  // tiles split K over them.
+  const int64_t t64 = (int64_t)((M + 63) / 64) * ((N + 127) / 128);
+  const bool small = ragged && pipe_forced == -1 && mode != MODE_NVFP4 && M > 64 && N > 64 && t64 >= 24 &&
+                     t64 <= device_cu_count() && (mode == MODE_FP8_TENSOR || mode == MODE_BF16 || sc4) &&
+                     (mode != MODE_MXFP4 || Kb % 128 == 0 || padded);
   if (streamable && !skinny_stream && M > 32 && (mode != MODE_NVFP4 || M > 256)) {
     const int bm = stream_blocks64(mode, M, K, Kb, sc16) ? 64 : 32;
     const int64_t span2 = 2 * (int64_t)((M + bm - 1) / bm) * N;   // twice the span
@@ -298,7 +310,12 @@ static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc1
     // 14.7), groupwise per-column up to 12 (14: 21.4 against 15.8), bf16
     // where one round of tiles holds it up to 8 (10: 20.8 against 18.0),
     // other bf16 below 30 (35: 53.5 against 45.4 on the persistent tiles).
-    const int64_t thr2 = mode == MODE_FP8_GCOL ? 13
+    // (whole lines of 128 bytes that are no whole 512 stream slower: 6 there;
+    // bf16 700x1500x1472 20.4 / 14.2; other rows slow the tiles too, K=4160
+    // M=256 N=4096 bf16 22.8 / 26.2, MXFP4 12.8 / 15.8)
+    const bool plain = (stream_whole(mode, K, Kb, sc16) && Kb % 512 == 0) || Kb % 128 != 0;
+    const int64_t thr2 = small ? (mode == MODE_MXFP4 || mode == MODE_BF16 ? (plain ? 9 : 6) : 5)
+                         : mode == MODE_FP8_GCOL ? 13
                          : mode_grouped_k(mode) ? 11
                          : (mode == MODE_BF16 ? (bf16_pipe_round ? 9 : 30)
                                               : (mode == MODE_NVFP4 ? 30 : 9));
@@ -335,6 +352,13 @@ static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc1
     r.path = PATH_STREAM;
     return r;
   }
+  const int one_round = ragged && mode != MODE_NVFP4 && t128 <= device_cu_count() && pipe_forced < 0 ? 7 : 1;
+  if (small) {
+    r.path = PATH_PIPE;
+    r.variant = 6;
+    r.pad_scales = mode == MODE_MXFP4 && Kb % 128 != 0;
+    return r;
+  }
   // 256x128 persistent tiles where one round of them holds a problem that
   // takes the 128x128 tiles more than one round (and the 256x256 ones half a
   // round at most).  One full round costs about 0.65 of a full 256x256 round,
@@ -362,7 +386,7 @@ static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc1
     // 89)
     if (bf16_pipe_round) {
       r.path = PATH_PIPE;
-      r.variant = 1;
+      r.variant = one_round;
     } else if (persist_on && 6 * t256 >= device_cu_count() && (int64_t)M * N >= 2400000 &&
                persist_supported(mode, M, N, K, Kb, sc4) && (ragged || Kb % 128 == 0)) {
       r.path = PATH_PERSIST;
@@ -403,11 +427,11 @@ static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc1
     const bool persist_wins = t256 >= 240 || r128 >= rounds128 * r256;
     if (persist_wins) {
       r.path = PATH_PIPE;
-      r.variant = pipe_forced >= 0 ? pipe_forced : (t256 >= 240 ? 0 : 1);
+      r.variant = pipe_forced >= 0 ? pipe_forced : (t256 >= 240 ? 0 : one_round);
       if (persist_ok) r.path = PATH_PERSIST;
     } else if (M > 64 && N > 64 && t128 >= 40) {
       r.path = PATH_PIPE;
-      r.variant = 1;
+      r.variant = one_round;
     }
   }
   if (narrow && persist_ok) {

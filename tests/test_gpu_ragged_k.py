@@ -160,3 +160,13 @@ def test_padded_scale_rows_need_their_workspace():
 @pytest.mark.parametrize("m,n,k", [(1300, 2500, 512), (1281, 4000, 608), (4100, 4200, 512), (2100, 7500, 256)])
 def test_narrow_tiles_and_column_strips(mode, m, n, k):
     check(mode, m, n, k)
+
+
+# 64x128 and deep-ring 128x128 tiles: one round, ragged rows and columns, whole,
+# odd and partial stages, fewer stages than the ring holds
+@pytest.mark.parametrize("mode", ["tensor", "block", "group", "mxfp4", "bf16"])
+@pytest.mark.parametrize("m,n", [(300, 2050), (1025, 1000), (900, 4000)])
+def test_small_tiles(mode, m, n):
+    unit = {"mxfp4": 32, "bf16": 8}.get(mode, 16)
+    for k in (unit, 128, 256, 640, 1024, 1152 + unit):
+        check(mode, m, n, k)
