@@ -642,6 +642,15 @@ StreamPlan plan_for(int mode, int M, int N, int Kb, bool tail) {
   // K = 4160, N = 4096: M = 64 per-tensor 8.5 us in 32-row blocks against
   // 9.8, block 9.5 against 12.4; M = 128 level, M = 256 bf16 24.2 against 33.2.
   pl.tma = M <= 16 ? 1 : ((M <= 32 || !stream_rows64(M, Kb, tail)) ? 2 : 4);
+  // Few W slices: the smallest row blocks whose workgroups (of one W tile) fit
+  // one round, so that more CUs share the rows (N=512 K=4096, us: bf16 M=64 8.4
+  // -> 6.7, M=100 9.7 -> 5.8, M=200 9.2 -> 7.8; block M=64 6.8 -> 4.8; N=1024
+  // bf16 M=64 10.0 -> 6.7, N=2048 10.5 -> 8.8)
+  for (int t = 1; t < pl.tma; t *= 2)
+    if ((int64_t)((M + 16 * t - 1) / (16 * t)) * ((N + 15) / 16) <= device_cu_count()) {
+      pl.tma = t;
+      break;
+    }
   const char *et = getenv("DSL_GEMM_STREAM_TMA");
   const bool force_tma = et && (et[0] == '1' || et[0] == '2' || (et[0] == '4' && (tail || Kb % 512 == 0))) && !et[1];
   if (force_tma) pl.tma = et[0] - '0';

@@ -492,6 +492,13 @@ static GemmArgs columns_from(int mode, GemmArgs p, int n1) {
 // per-tensor / block / MXFP4 / NVFP4 / bf16: 2304x7680x4096 (270 tiles) 90 ->
 // 75, 106 -> 93, 63 -> 58, 190 -> 178, 177 -> 145; 4300x4300x4096 (289 tiles)
 // 141 -> 116, 158 -> 132, 113 -> 101, 241 -> 218, 230 -> 185.
+static int pipe_variant(int mode, int M, int N) {
+  const int64_t cu = device_cu_count();
+  if (mode == MODE_NVFP4) return 1;
+  if ((int64_t)((M + 63) / 64) * ((N + 127) / 128) <= cu) return 6;
+  return (int64_t)((M + 127) / 128) * ((N + 127) / 128) <= cu ? 7 : 1;
+}
+
 static int strip_columns(const GemmArgs &p) {
   const int cu = device_cu_count();
   const int nbm = (p.M + 255) / 256, nbn = (p.N + 255) / 256;
@@ -569,7 +576,7 @@ hipError_t launch_gemm(int mode, GemmArgs p, hipStream_t st) {
       return route_for(mode, rest.M, rest.N, rest.K, rest.Kb, (sc & 3) == 0, (sc & 15) == 0, false).path ==
                      PATH_STREAM
                  ? launch_gemm_stream(mode, rest, st)
-                 : launch_gemm_pipe(mode, rest, 1, st);
+                 : launch_gemm_pipe(mode, rest, pipe_variant(mode, rest.M, rest.N), st);
     }
     return launch_gemm_persist(mode, p, st, r.narrow);
   }

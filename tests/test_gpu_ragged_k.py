@@ -170,3 +170,12 @@ def test_small_tiles(mode, m, n):
     unit = {"mxfp4": 32, "bf16": 8}.get(mode, 16)
     for k in (unit, 128, 256, 640, 1024, 1152 + unit):
         check(mode, m, n, k)
+
+
+
+@pytest.mark.parametrize("mode", sorted(KS))
+@pytest.mark.parametrize("m,n", [(33, 500), (64, 1030), (100, 260), (200, 130)])
+def test_few_weight_slices(mode, m, n):
+    """Small row blocks where N gives few workgroups."""
+    for k in (512, 4096, KS[mode][2]):
+        check(mode, m, n, k)
