@@ -61,6 +61,7 @@ SIGNATURES = {
     "dsl_quant_fp8_tensor": (_i32, [_vp, _i64, _i64, _i64, _i64, _i32, _vp, _vp, _vp, _sz, _vp]),
     "dsl_quant_fp8_tensor_noalloc": (_i32, [_vp, _i64, _i64, _i64, _i64, _i32, _vp, _vp, _vp]),
     "dsl_quant_fp8_blocks": (_i32, [_vp, _i64, _i64, _i64, _i64, _i32, _i64, _i64, _vp, _vp, _vp]),
+    "dsl_quant_fp8_rows_batched": (_i32, [_vp, _i64, _i64, _i64, _i64, _i64, _i32, _vp, _vp, _vp]),
     "dsl_quant_mxfp4": (_i32, [_vp, _i64, _i64, _i64, _i64, _i32, _vp, _vp, _vp]),
     "dsl_quant_nvfp4": (_i32, [_vp, _i64, _i64, _i64, _i64, _i32, _vp, _vp, _vp, _vp, _sz, _vp]),
     "dsl_quant_workspace_bytes": (_sz, [_i64, _i64]),

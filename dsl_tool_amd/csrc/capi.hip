@@ -150,6 +150,23 @@ int dsl_quant_fp8_blocks(const void *x, int64_t rows, int64_t cols, int64_t sr, 
                     fn);
 }
 
+int dsl_quant_fp8_rows_batched(const void *x, int64_t batch, int64_t rows, int64_t cols, int64_t sb,
+                               int64_t sc, int x_dtype, uint8_t *q, float *scales, void *stream) {
+  const char *fn = "dsl_quant_fp8_rows_batched";
+  int rc = check_input(fn, x, rows, cols, 1, sc, x_dtype);
+  if (rc) return rc;
+  if (batch < 0 || batch > 65535)
+    return fail(DSL_ERR_ARG, "%s: batch=%lld must be in [0, 65535]", fn, (long long)batch);
+  if (batch == 0 || rows == 0 || cols == 0) return ok();
+  if (sc < rows || (batch > 1 && sb <= 0))
+    return fail(DSL_ERR_ARG, "%s: need stride_col >= rows and a positive stride_batch", fn);
+  if ((rc = check_out(fn, q, "q"))) return rc;
+  if (!scales) return fail(DSL_ERR_ARG, "%s: scales is NULL", fn);
+  return hip_status(dsl::launch_quant_fp8_rows_batched(x, x_dtype == DSL_IN_F32, batch, rows, cols, sb, sc, q,
+                                                       scales, static_cast<hipStream_t>(stream)),
+                    fn);
+}
+
 int dsl_quant_mxfp4(const void *x, int64_t rows, int64_t cols, int64_t sr, int64_t sc,
                     int x_dtype, uint8_t *q, uint8_t *e8m0, void *stream) {
   const char *fn = "dsl_quant_mxfp4";

@@ -153,6 +153,28 @@ PyObject *quant_fp8_blocks(PyObject *, PyObject *const *a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// the view of [G, K, N] storage as [G, N, K], one scale per row
+PyObject *quant_fp8_rows_batched(PyObject *, PyObject *const *a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  const Tensor *w = n == 1 ? gpu_tensor(a[0]) : nullptr;
+  if (!w || w->dim() != 3 || w->numel() == 0 || w->stride(1) != 1 || w->stride(2) < w->size(1) ||
+      w->stride(0) <= 0 || w->size(0) > 65535)
+    return none();
+  const bool bf16 = w->scalar_type() == ScalarType::BFloat16;
+  if (!bf16 && w->scalar_type() != ScalarType::Float) return none();
+  Tensor q, s;
+  const bool ok = on_device(*w, [&] {
+    const int64_t g = w->size(0), r = w->size(1), c = w->size(2);
+    q = empty({g * r, c}, ScalarType::Byte, *w);
+    s = empty({g * r, 1}, ScalarType::Float, *w);
+    return dsl_quant_fp8_rows_batched(ptr(*w), g, r, c, w->stride(0), w->stride(2),
+                                      bf16 ? DSL_IN_BF16 : DSL_IN_F32, ptr<uint8_t>(q), ptr<float>(s),
+                                      stream_of(*w)) == DSL_OK;
+  });
+  return ok ? pack({q, s}) : none();
+  END_HANDLE_TH_ERRORS
+}
+
 PyObject *quant_mxfp4(PyObject *, PyObject *const *a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   int dt;
@@ -467,6 +489,7 @@ PyMethodDef methods[] = {DSL_FN(quant_fp8_tensor), DSL_FN(quant_fp8_blocks), DSL
                          DSL_FN(quant_nvfp4),      DSL_FN(fp8_gemm),         DSL_FN(fp4_gemm),
                          DSL_FN(bf16_gemm),        DSL_FN(grouped_fp8_gemm), DSL_FN(rmsnorm_quant),
                          DSL_FN(swiglu_quant),     DSL_FN(moe_projection),   DSL_FN(lora_gemm),
+                         DSL_FN(quant_fp8_rows_batched),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "dsl_fast", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

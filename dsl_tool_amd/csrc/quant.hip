@@ -28,6 +28,7 @@
 // (quot), which give the same codes; the strided path divides and encodes in
 // software.
 #include <mutex>
+#include <type_traits>
 #include <utility>
 
 #include "launch.h"
@@ -611,10 +612,18 @@ __global__ __launch_bounds__(256) void quant_fp8_tile_kernel(
 //
 // KIND_FP8: NC = 8: 1 x gc groups, gc a multiple of 128 (or >= cols);
 //           NC = 16: 128 x 128 tiles.
+// blockIdx.z: matrix of a batch xb elements apart, whose codes and scales
+// follow each other (KIND_FP8, NC = 8).  Groups of several tiles (MULTI) are
+// bound by the latency of their loads and keep several tiles in flight (100
+// registers against 30-63): 16 [2048, 1536] bf16 weights, one scale per row,
+// 45 us where the transposed copy and the row quantizer took 212 + 23.
 // ---------------------------------------------------------------------------
 template <bool VEC, typename T, int KE>
 struct TransTile;
 
+// The loads are unconditional (a branch around each would wait for it before the
+// next is issued): columns past the end re-read the last one, rows past the end
+// the thread's last, and both become zero by selects.
 // bf16: column j of the thread's 8 rows as packed pairs
 template <bool VEC, int KE>
 struct TransTile<VEC, uint16_t, KE> {
@@ -622,20 +631,23 @@ struct TransTile<VEC, uint16_t, KE> {
   DSL_DEV void load(const uint16_t *x, int64_t ld, int nrow, int ncol) {
 #pragma unroll
     for (int j = 0; j < KE; ++j) {
-      v[j] = make_uint4(0, 0, 0, 0);
-      if (j < ncol && nrow > 0) {
-        const uint16_t *p = x + j * ld;
-        if constexpr (VEC) {
-          v[j] = *reinterpret_cast<const uint4 *>(p);
-        } else {
-          uint32_t w[8];
+      const uint16_t *p = x + (int64_t)(j < ncol ? j : ncol - 1) * ld;
+      if constexpr (VEC) {
+        v[j] = *reinterpret_cast<const uint4 *>(p);
+      } else {
+        uint32_t w[8];
 #pragma unroll
-          for (int i = 0; i < 8; ++i) w[i] = i < nrow ? p[i] : 0;
-          v[j] = make_uint4(w[0] | (w[1] << 16), w[2] | (w[3] << 16), w[4] | (w[5] << 16),
-                            w[6] | (w[7] << 16));
-        }
+        for (int i = 0; i < 8; ++i) w[i] = p[i < nrow ? i : 0];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) w[i] = i < nrow ? w[i] : 0;
+        v[j] = make_uint4(w[0] | (w[1] << 16), w[2] | (w[3] << 16), w[4] | (w[5] << 16), w[6] | (w[7] << 16));
       }
     }
+  }
+  DSL_DEV void cut(int nrow, int ncol) {
+#pragma unroll
+    for (int j = 0; j < KE; ++j)
+      if (j >= ncol || nrow <= 0) v[j] = make_uint4(0, 0, 0, 0);
   }
   DSL_DEV float at(int i, int j) const {
     const uint32_t w = i < 2 ? v[j].x : i < 4 ? v[j].y : i < 6 ? v[j].z : v[j].w;
@@ -649,25 +661,29 @@ struct TransTile<VEC, float, KE> {
   DSL_DEV void load(const float *x, int64_t ld, int nrow, int ncol) {
 #pragma unroll
     for (int j = 0; j < KE; ++j) {
+      const float *p = x + (int64_t)(j < ncol ? j : ncol - 1) * ld;
+      if constexpr (VEC) {
+        load8(p, v[j]);
+      } else {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) v[j][i] = 0.f;
-      if (j < ncol && nrow > 0) {
-        const float *p = x + j * ld;
-        if constexpr (VEC) {
-          load8(p, v[j]);
-        } else {
+        for (int i = 0; i < 8; ++i) v[j][i] = p[i < nrow ? i : 0];
 #pragma unroll
-          for (int i = 0; i < 8; ++i) v[j][i] = i < nrow ? p[i] : 0.f;
-        }
+        for (int i = 0; i < 8; ++i) v[j][i] = i < nrow ? v[j][i] : 0.f;
       }
     }
+  }
+  DSL_DEV void cut(int nrow, int ncol) {
+#pragma unroll
+    for (int j = 0; j < KE; ++j)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[j][i] = j >= ncol || nrow <= 0 ? 0.f : v[j][i];
   }
   DSL_DEV float at(int i, int j) const { return v[j][i]; }
 };
 
-template <int KIND, bool VEC, typename T, int NC>
+template <int KIND, bool VEC, typename T, int NC, bool MULTI>
 __global__ __launch_bounds__(NC * 32) void quant_trans_kernel(
-    const T *__restrict__ x, int64_t rows, int64_t cols, int64_t ld, int64_t gc,
+    const T *__restrict__ x, int64_t rows, int64_t cols, int64_t ld, int64_t gc, int64_t xb,
     uint8_t *__restrict__ q, void *__restrict__ scales, const float *__restrict__ partial, int np,
     float *__restrict__ sout) {
   constexpr bool FP4 = KIND == KIND_MX || KIND == KIND_NV;
@@ -688,26 +704,55 @@ __global__ __launch_bounds__(NC * 32) void quant_trans_kernel(
   const int t = threadIdx.x, c = t % NC, kk = t / NC;
   const int64_t n0 = (int64_t)blockIdx.x * NR;
   const int nrow = (int)(rows - n0 - 8 * c < 8 ? rows - n0 - 8 * c : 8);   // rows of this thread
-  const T *xt = x + n0 + 8 * c;
+  const T *xt = x + n0 + (nrow > 0 ? 8 * c : 0);
+  if constexpr (KIND == KIND_FP8 && !TILE) {
+    const int64_t z = blockIdx.z;
+    xt += z * xb;
+    q += z * rows * cols;
+    scales = reinterpret_cast<float *>(scales) + z * rows * ((cols + gc - 1) / gc);
+  }
   const int64_t span = KIND == KIND_FP8 ? gc : KT;                         // columns of this block
   const int64_t c0 = (int64_t)blockIdx.y * span, c1 = c0 + span < cols ? c0 + span : cols;
-  TransTile<VEC, T, KE> d;
-  auto load = [&](int64_t k0) {
-    const int64_t k = k0 + kk * KE;
-    const int64_t left = c1 - k;
-    d.load(xt + k * ld, ld, nrow, (int)(left < 0 ? 0 : (left < KE ? left : KE)));
+  using Tile = TransTile<VEC, T, KE>;
+  Tile d;
+  auto load = [&](Tile &to, int64_t k0) {
+    const int64_t k = k0 + kk * KE, left = c1 - k;
+    const int nc = (int)(left < 0 ? 0 : (left < KE ? left : KE));
+    to.load(xt + (nc > 0 ? k : c1 - 1) * ld, ld, nrow, nc > 0 ? nc : 1);
+  };
+  // the columns and rows of a loaded tile that do not exist become zero
+  auto cut = [&](Tile &of, int64_t k0) {
+    const int64_t left = c1 - (k0 + kk * KE);
+    if (left < KE || nrow <= 0) of.cut(nrow, (int)(left < 0 ? 0 : (left < KE ? left : KE)));
   };
   float s[8], r[8];               // FP8: the row's scale and its reciprocal
   if constexpr (KIND == KIND_FP8) {
     float m[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) m[i] = 0.f;
-    for (int64_t k0 = c0; k0 < c1; k0 += KT) {
-      load(k0);
+    auto take = [&](const Tile &from) {
 #pragma unroll
       for (int i = 0; i < 8; ++i)
 #pragma unroll
-        for (int j = 0; j < KE; ++j) m[i] = fmaxf(m[i], __builtin_fabsf(d.at(i, j)));
+        for (int j = 0; j < KE; ++j) m[i] = fmaxf(m[i], __builtin_fabsf(from.at(i, j)));
+    };
+    if constexpr (!MULTI) {
+      load(d, c0);
+      cut(d, c0);
+      take(d);
+    } else {
+      constexpr int U = F32 ? 2 : 4;            // tiles in flight (past c1: zeros)
+      for (int64_t k0 = c0; k0 < c1; k0 += U * KT) {
+        Tile e[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) load(e[u], k0 + u * KT);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          cut(e[u], k0 + u * KT);
+          take(e[u]);
+        }
+      }
+      load(d, c0);
     }
     if constexpr (TILE) {
 #pragma unroll
@@ -756,10 +801,15 @@ __global__ __launch_bounds__(NC * 32) void quant_trans_kernel(
       r[i] = rt;
     }
   }
-  const bool one = c1 - c0 <= KT;               // FP8: the tile is still in registers
   const int64_t rowb = FP4 ? cols / 2 : cols;   // code bytes per row
   for (int64_t k0 = c0; k0 < c1; k0 += KT) {
-    if (KIND != KIND_FP8 || !one) load(k0);
+    Tile nx;                                    // FP8, several tiles: the next one's loads
+    if constexpr (KIND != KIND_FP8) {
+      load(d, k0);
+    } else if constexpr (MULTI) {
+      load(nx, k0 + KT);
+    }
+    if constexpr (KIND != KIND_FP8 || MULTI) cut(d, k0);
     if constexpr (FP4) {
       constexpr int GL = KIND == KIND_MX ? 4 : 2;          // threads (kk) per scale group
       const int64_t g = (k0 + kk * KE) / (GL * KE), gpr = cols / (GL * KE);
@@ -821,6 +871,7 @@ __global__ __launch_bounds__(NC * 32) void quant_trans_kernel(
       }
     }
     __syncthreads();
+    if constexpr (MULTI) d = nx;
   }
 }
 
@@ -863,20 +914,32 @@ static bool trans_ok(int64_t rows, int64_t cols, int64_t sr, int64_t sc) {
 
 template <int KIND, int NC, typename T>
 static void launch_trans(const T *x, int64_t rows, int64_t cols, int64_t ld, int64_t gc, uint8_t *q,
-                         void *scales, const float *partial, int np, float *sout, hipStream_t st) {
+                         void *scales, const float *partial, int np, float *sout, hipStream_t st,
+                         int64_t batch = 1, int64_t xb = 0) {
   constexpr int KT = (KIND == KIND_MX || KIND == KIND_NV) ? 256 : 128;
   const int64_t span = KIND == KIND_FP8 ? gc : KT;
-  const dim3 grid((unsigned)((rows + 8 * NC - 1) / (8 * NC)), (unsigned)((cols + span - 1) / span));
+  const dim3 grid((unsigned)((rows + 8 * NC - 1) / (8 * NC)), (unsigned)((cols + span - 1) / span),
+                  (unsigned)batch);
   // 16-byte loads of 8 rows (bf16; fp32: two) need whole 8-row runs and
   // aligned columns; rows past the end are masked 8 at a time
-  const bool vec = rows % 8 == 0 && ld % (16 / sizeof(T)) == 0 &&
+  const bool vec = rows % 8 == 0 && ld % (16 / sizeof(T)) == 0 && xb % (16 / sizeof(T)) == 0 &&
                    reinterpret_cast<uintptr_t>(x) % 16 == 0;
-  if (vec)
-    quant_trans_kernel<KIND, true, T, NC><<<grid, 32 * NC, 0, st>>>(x, rows, cols, ld, gc, q, scales,
-                                                                    partial, np, sout);
-  else
-    quant_trans_kernel<KIND, false, T, NC><<<grid, 32 * NC, 0, st>>>(x, rows, cols, ld, gc, q, scales,
-                                                                     partial, np, sout);
+  auto go = [&](auto multi) {
+    constexpr bool MULTI = decltype(multi)::value;
+    if (vec)
+      quant_trans_kernel<KIND, true, T, NC, MULTI><<<grid, 32 * NC, 0, st>>>(x, rows, cols, ld, gc, xb, q,
+                                                                             scales, partial, np, sout);
+    else
+      quant_trans_kernel<KIND, false, T, NC, MULTI><<<grid, 32 * NC, 0, st>>>(x, rows, cols, ld, gc, xb, q,
+                                                                              scales, partial, np, sout);
+  };
+  if constexpr (KIND == KIND_FP8 && NC == 8) {
+    if (gc > KT) {
+      go(std::true_type{});
+      return;
+    }
+  }
+  go(std::false_type{});
 }
 
 // FP8 scale groups the transposed kernel takes: 1 x gc with gc whole 128-column
@@ -1120,6 +1183,20 @@ hipError_t launch_quant_fp8_blocks(const void *xv, bool f32, int64_t rows, int64
     quant_fp8_tile_kernel<true, uint16_t><<<(unsigned)tiles, 256, 0, st>>>(x, rows, cols, sr, sc, gr, gc, q, scales);
   else
     quant_fp8_tile_kernel<false, uint16_t><<<(unsigned)tiles, 256, 0, st>>>(x, rows, cols, sr, sc, gr, gc, q, scales);
+  return hipGetLastError();
+}
+
+// One scale per row of each of `batch` [cols][ld] matrices read as their
+// transposes (batch <= 65535).
+hipError_t launch_quant_fp8_rows_batched(const void *xv, bool f32, int64_t batch, int64_t rows, int64_t cols,
+                                         int64_t xb, int64_t ld, uint8_t *q, float *scales, hipStream_t st) {
+  const int64_t gc = (cols + 127) / 128 * 128;
+  if (f32)
+    launch_trans<KIND_FP8, 8>(static_cast<const float *>(xv), rows, cols, ld, gc, q, scales, nullptr, 0, nullptr,
+                              st, batch, xb);
+  else
+    launch_trans<KIND_FP8, 8>(static_cast<const uint16_t *>(xv), rows, cols, ld, gc, q, scales, nullptr, 0,
+                              nullptr, st, batch, xb);
   return hipGetLastError();
 }
 

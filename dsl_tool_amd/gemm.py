@@ -627,11 +627,9 @@ def grouped_gemm(A: torch.Tensor, B: torch.Tensor, num_groups, scale_a=None, sca
         out_dtype = torch.float32 if A.dtype == torch.float32 else torch.bfloat16
     out_dtype = _as_dtype(out_dtype)
     if X.dtype in _HIGH and B.dtype in _HIGH:
-        # W[g, n, k] rows (a view when B is the transpose of K-major [G, N, K]
-        # storage, else a copy; the high-precision weight is quantized on
-        # every call anyway)
+        # W[g, n, k] rows, read in place from [G, K, N] or [G, N, K] storage
         qx, sx = Q.quant_fp8_blocks(X, 1, K)
-        qw, sw = Q.quant_fp8_blocks(B.transpose(1, 2).reshape(G * Nn, K), 1, K)
+        qw, sw = Q.quant_fp8_rows_batched(B.transpose(1, 2))
     elif X.dtype == _FP8 and B.dtype == _FP8:
         if scale_a is None or scale_b is None:
             raise ValueError("fp8 grouped_gemm needs scale_a [T] and scale_b [G, N]")

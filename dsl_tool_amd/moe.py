@@ -216,8 +216,7 @@ def routed_grouped_gemm(x: torch.Tensor, topk_ids: torch.Tensor, topk_weights: t
         if w.dim() != 3:
             raise ValueError("w must be [E, K, N]")
         E, K, Nn = w.shape
-        wt = w.transpose(1, 2).reshape(E * Nn, K)       # [E*N, K] K-major rows
-        qw, sw = Q.quant_fp8_blocks(wt, 1, K)
+        qw, sw = Q.quant_fp8_rows_batched(w.transpose(1, 2))   # [E*N, K] K-major rows
         qw, sw = qw.reshape(E, Nn, K), sw.reshape(E, Nn)
     _gpu(topk_ids, "topk_ids")
     if topk_ids.dim() != 2:

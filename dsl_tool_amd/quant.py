@@ -74,6 +74,27 @@ def quant_fp8_blocks(x: torch.Tensor, group_rows: int, group_cols: int):
     return q, scales
 
 
+def quant_fp8_rows_batched(w: torch.Tensor):
+    """One E4M3 scale per row of ``w [G, N, K]``: ``(q uint8 [G*N, K], scales
+    float32 [G*N, 1])``, what ``quant_fp8_blocks(w.reshape(G * N, K), 1, K)``
+    gives.  The view of [G, K, N] storage (the reference's grouped B) is read
+    in place instead of being copied to K-major rows first."""
+    G, R, C = w.shape
+    if not (w.device.type == "cuda" and w.dtype in (torch.bfloat16, torch.float32) and w.numel() > 0
+            and R > 1 and C > 1 and w.stride(1) == 1 and w.stride(2) >= R and w.stride(0) > 0 and G <= 65535):
+        return quant_fp8_blocks(w.reshape(G * R, C), 1, C)
+    r = N.fast().quant_fp8_rows_batched(w)
+    if r is not None:
+        return r
+    q = torch.empty((G * R, C), dtype=torch.uint8, device=w.device)
+    scales = torch.empty((G * R, 1), dtype=torch.float32, device=w.device)
+    with torch.cuda.device(w.device):
+        N.call("dsl_quant_fp8_rows_batched", N.ptr(w), G, R, C, w.stride(0), w.stride(2),
+               N.IN_BF16 if w.dtype == torch.bfloat16 else N.IN_F32, N.ptr(q), N.ptr(scales),
+               N.stream_of(w.device))
+    return q, scales
+
+
 def quant_mxfp4(x: torch.Tensor):
     r = N.fast().quant_mxfp4(x)
     if r is not None:

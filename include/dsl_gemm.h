@@ -96,6 +96,15 @@ int dsl_quant_fp8_blocks(const void *x, int64_t rows, int64_t cols,
                          int64_t group_rows, int64_t group_cols,
                          uint8_t *q, float *scales, void *stream);
 
+/* dsl_quant_fp8_blocks with one 1 x cols group per row, over `batch` matrices
+ * of unit row stride (the reference's grouped B[G][K][N] read as [G][N][K],
+ * triton/gemm/gemm_kernels.py:164-182): matrix b is x[b*stride_batch + r +
+ * c*stride_col], stride_col >= rows.  q [batch*rows][cols], scales
+ * [batch*rows].  batch <= 65535. */
+int dsl_quant_fp8_rows_batched(const void *x, int64_t batch, int64_t rows, int64_t cols,
+                               int64_t stride_batch, int64_t stride_col, int x_dtype,
+                               uint8_t *q, float *scales, void *stream);
+
 /* MXFP4: per row and 32 K elements, E8M0 = clamp(floor(log2 amax)-2,
  * -127,127)+127, codes = e2m1_rne_sat(x * 2^-e).  q_packed [R][C/2] (low
  * nibble = even K), e8m0 [R][C/32].  C % 32 == 0.

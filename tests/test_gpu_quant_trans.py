@@ -65,3 +65,18 @@ def test_transposed_sources_odd_columns(c):
         q_ref, s_ref, sg_ref = OQ.quant_nvfp4(ref)
         assert np_f32(sg)[0] == sg_ref
         assert np.array_equal(np_u8(s), s_ref) and np.array_equal(np_u8(q), q_ref)
+
+
+@pytest.mark.parametrize("g,n,k", [(1, 64, 128), (3, 72, 400), (5, 130, 1040), (2, 513, 2064)])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("pad", [0, 3, 8])
+def test_batched_rows_match_oracle(g, n, k, dt, pad):
+    """[G, K, N] weights, one scale per output row, read in place."""
+    gen = torch.Generator().manual_seed(g * n + k)
+    w = (torch.randn((g, k, n), generator=gen) * 0.02).to(dt)
+    buf = torch.zeros((g, k, n + pad), dtype=dt, device=DEV)
+    buf[:, :, :n] = w.to(DEV)
+    q, s = Q.quant_fp8_rows_batched(buf[:, :, :n].transpose(1, 2))
+    q_ref, s_ref = OQ.quant_fp8_blockwise(w.transpose(1, 2).reshape(g * n, k).float().numpy(), 1, k)
+    assert np.array_equal(np_f32(s), s_ref)
+    assert np.array_equal(np_u8(q), q_ref)
