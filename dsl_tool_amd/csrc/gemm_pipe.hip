@@ -639,6 +639,9 @@ hipError_t launch_gemm_pipe(int mode, const GemmArgs &p, int variant, hipStream_
   // whole stages, an even number of them on the prefetch schedule
   const bool pf = mode == MODE_FP8_TENSOR || mode == MODE_BF16;
   const bool rag = p.Kb % 128 != 0, rag_deep = p.Kb % (pf ? 256 : 128) != 0;
+  // the deep rings keep a tile's weight-block scales in LDS: longer K takes
+  // the two-stage 128x128 tiles, which read them from memory
+  if (mode == MODE_FP8_BLOCK && (variant == 6 || variant == 7) && (p.K + 127) / 128 > kBlockPfMaxGroups) variant = 1;
   if (variant == 6) return rag_deep ? launch_pipe_small<true>(mode, p, st) : launch_pipe_small<false>(mode, p, st);
   if (variant == 7) return rag_deep ? launch_pipe_deep<true>(mode, p, st) : launch_pipe_deep<false>(mode, p, st);
   if (rag) {

@@ -179,3 +179,24 @@ def test_few_weight_slices(mode, m, n):
     """Small row blocks where N gives few workgroups."""
     for k in (512, 4096, KS[mode][2]):
         check(mode, m, n, k)
+
+
+@pytest.mark.parametrize("k", [65536, 65536 + 144])
+def test_more_scale_groups_than_the_ring_holds(k):
+    """Block-scaled tiles keep 512 weight scales of a row in LDS; longer K
+    takes the tiles that read them from memory."""
+    m, n = 320, 2048
+    gen = torch.Generator(device=DEV).manual_seed(k)
+    a = torch.randn((m, k), generator=gen, device=DEV).bfloat16()
+    w = torch.randn((n, k), generator=gen, device=DEV).bfloat16()
+    qa, sa = Q.quant_fp8_blocks(a, 1, 128)
+    qw, sw = Q.quant_fp8_blocks(w, 128, 128)
+    c = G.fp8_gemm_packed(qa, qw, sa, sw, block=True, out_dtype=torch.float32)
+    ref = torch.zeros((m, n), dtype=torch.float64, device=DEV)
+    for g in range(0, k, 8192):
+        e = min(g + 8192, k)
+        f = lambda q, s: q[:, g:e].view(torch.float8_e4m3fn).double() * s.double()[:, g // 128:].repeat_interleave(
+            128, 1)[:, :e - g]
+        ref += f(qa, sa) @ f(qw, sw.repeat_interleave(128, 0)[:n]).t()
+    # fp32 sums of k products: sqrt(k) * 2^-24 relative to the largest output, 8x margin
+    assert (c.double() - ref).abs().max() <= 8 * k ** 0.5 * 2.0 ** -24 * ref.abs().max()
