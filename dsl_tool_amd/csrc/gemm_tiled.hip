@@ -206,11 +206,12 @@ static bool env_off(const char *name) {
 // scales are aligned; with misaligned scales the launch may fall back to
 // the register-staged kernels, split-K only if a workspace was passed.
 //   DSL_GEMM_DECODE = 0/off    never use the skinny-M kernel
-//   DSL_GEMM_STREAM = 0/off    never use the streaming kernel (M <= 256)
+//   DSL_GEMM_STREAM = 0/off    never use the streaming kernel
 //   DSL_GEMM_SKINNY = stream   2 <= M <= 16 on the streaming kernel too
 //                              (default: the skinny-M decode kernel there)
 //   DSL_GEMM_PIPE   = 0/off    never use the LDS-DMA pipelined kernels
 //   DSL_GEMM_PIPE   = 1..9     force that pipelined variant for large problems
+//                              (and no 64x128, deep 128x128 or 256x128 tiles)
 //   DSL_GEMM_PERSIST = 0/off   use the per-tile pipelined kernels instead of
 //                              the persistent one for large problems
 enum { PATH_DECODE = 0, PATH_PIPE = 1, PATH_TILED = 2, PATH_PERSIST = 3, PATH_STREAM = 4 };

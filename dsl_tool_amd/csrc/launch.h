@@ -63,7 +63,7 @@ struct GemmArgs {
   size_t ws_bytes;       // bytes at ws; split-K runs only when it holds two slices or more
   int ksplit;            // >= 1
   int out_f32;
-  int accumulate;        // fp32 out only: C += result (register-staged kernels)
+  int accumulate;        // fp32 out only: C += result (streaming, pipelined and register-staged kernels)
   // BF16 on the persistent kernel only: a second K segment, C = A W^T +
   // A2 W2^T with A2 [M][Kb2], W2 [N][Kb2] (Kb2 % 128 == 0; 0: none)
   const uint8_t *a2, *b2;
@@ -85,8 +85,9 @@ struct GemmArgs {
 };
 
 // LDS-DMA pipelined kernel (every mode, no split-K; Kb % 128 == 0, or the
-// ragged forms of variant 1);
-// variant 0: 256x256 tile, 8 waves; 1: 128x128 tile, 4 waves.
+// ragged forms of variants 1, 6 and 7);
+// variant 0: 256x256 tile, 8 waves; 1: 128x128 tile, two workgroups per CU;
+// 6 / 7: 64x128 / 128x128 tile on four 128-byte stages, one workgroup per CU.
 hipError_t launch_gemm_pipe(int mode, const GemmArgs &p, int variant, hipStream_t st);
 
 // Persistent pipelined kernel (Kb >= 128 in whole 16-byte chunks; not

@@ -330,7 +330,10 @@ int dsl_moe_combine(const void *y, int64_t rows, int64_t n, int64_t ldy, const i
  * scale modes / FP4 formats; 0 when none is needed).  The kernel choice
  * depends on the shape and on the scale pointers' alignment; with scale
  * arrays that are not 16-byte aligned a launch may fall back to a kernel
- * that runs without split-K rather than ask for more workspace. */
+ * that runs without split-K rather than ask for more workspace.  For FP4 with
+ * scale rows of no whole 16 bytes the size includes room for a copy of both
+ * scale arrays at a padded pitch (16-byte aligned workspace); a launch given
+ * less takes a kernel that does without the copy. */
 size_t dsl_gemm_workspace_bytes(int op, int64_t m, int64_t n, int64_t k);
 
 #ifdef __cplusplus
