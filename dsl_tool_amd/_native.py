@@ -79,6 +79,9 @@ SIGNATURES = {
     "dsl_lora_gemm_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64]),
     "dsl_lora_gemm": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _vp,
                              _sz, _vp]),
+    "dsl_lora_gemm_ab_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64]),
+    "dsl_lora_gemm_ab": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _vp,
+                                _sz, _vp]),
     "dsl_moe_route_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "dsl_moe_route": (_i32, [_vp, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _sz, _vp]),
     "dsl_moe_permute_quant": (_i32, [_vp, _i64, _i64, _i64, _vp, _i64, _i64, _vp, _vp, _vp]),

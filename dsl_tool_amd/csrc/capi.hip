@@ -431,6 +431,7 @@ struct LoraPlan {
   bool valu;                   // few tokens: fp32 T and the add on the vector ALUs
   bool vt;                     // T (as hi | lo) on the vector ALUs, the add on MFMA
   size_t t32, ws, t2, b2, total;
+  bool plain_bt() const { return valu || rep > 0; }   // B^T is read as it is
 };
 
 // Most tokens for the vector-ALU add (DSL_LORA_VALU_MAX_M overrides it, for
@@ -493,6 +494,11 @@ LoraPlan lora_plan(int64_t m, int64_t n, int64_t k, int64_t lr) {
   return p;
 }
 
+// Bytes behind LoraPlan::total for A^T and, where it is read as it is, B^T.
+size_t lora_pack_bytes(const LoraPlan &pl, int64_t n, int64_t k, int64_t lr) {
+  return align256((size_t)(lr * k) * 2) + (pl.plain_bt() ? align256((size_t)(n * lr) * 2) : 0);
+}
+
 dsl::GemmArgs bf16_args(const void *a, const void *b, void *c, int64_t m, int64_t n, int64_t k,
                         int64_t ldc, bool accumulate, void *ws, size_t ws_bytes) {
   dsl::GemmArgs p;
@@ -526,10 +532,11 @@ size_t dsl_lora_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k, int64_t ra
   return lora_plan(m, n, k, rank * num_loras).total;
 }
 
-int dsl_lora_gemm(const void *x, const void *w, const void *a_t, const void *b_t,
-                  const float *scales, float *y, int64_t m, int64_t n, int64_t k, int64_t rank,
-                  int64_t num_loras, int64_t ldy, void *ws, size_t ws_bytes, void *stream) {
-  const char *fn = "dsl_lora_gemm";
+// packed: a_t and b_t are K-major rows, else the caller's A [L][K][R] and
+// B [L][R][N], packed into the workspace first.
+static int run_lora(const char *fn, const void *x, const void *w, const void *a_t, const void *b_t,
+                    bool packed, const float *scales, float *y, int64_t m, int64_t n, int64_t k,
+                    int64_t rank, int64_t num_loras, int64_t ldy, void *ws, size_t ws_bytes, void *stream) {
   if (rank <= 0 || num_loras <= 0) return fail(DSL_ERR_ARG, "%s: rank and num_loras must be > 0", fn);
   const int64_t lr = rank * num_loras;
   int rc = check_gemm_dims(fn, m, n, k, ldy, 8, DSL_OUT_F32);
@@ -537,14 +544,18 @@ int dsl_lora_gemm(const void *x, const void *w, const void *a_t, const void *b_t
   if (lr % 8 != 0 || lr >= ((int64_t)1 << 20))
     return fail(DSL_ERR_ARG, "%s: rank * num_loras = %lld must be a multiple of 8", fn, (long long)lr);
   if (m == 0 || n == 0) return ok();
-  if ((rc = check_out(fn, x, "x")) || (rc = check_out(fn, w, "w")) || (rc = check_out(fn, a_t, "a_t")) ||
-      (rc = check_out(fn, b_t, "b_t")))
-    return rc;
+  if ((rc = check_out(fn, x, "x")) || (rc = check_out(fn, w, "w"))) return rc;
+  if (packed) {
+    if ((rc = check_out(fn, a_t, "a_t")) || (rc = check_out(fn, b_t, "b_t"))) return rc;
+  } else if (!a_t || !b_t || !aligned(a_t, 2) || !aligned(b_t, 2)) {
+    return fail(DSL_ERR_ARG, "%s: A or B is NULL or misaligned", fn);
+  }
   if (!scales || !y) return fail(DSL_ERR_ARG, "%s: NULL pointer argument", fn);
   if (!aligned(y, 4)) return fail(DSL_ERR_ARG, "%s: y is misaligned", fn);
   const LoraPlan pl = lora_plan(m, n, k, lr);
-  if (!ws || ws_bytes < pl.total || !aligned(ws, 256))
-    return fail(DSL_ERR_WORKSPACE, "%s: workspace of %zu bytes (256-B aligned) required", fn, pl.total);
+  const size_t need = pl.total + (packed ? 0 : lora_pack_bytes(pl, n, k, lr));
+  if (!ws || ws_bytes < need || !aligned(ws, 256))
+    return fail(DSL_ERR_WORKSPACE, "%s: workspace of %zu bytes (256-B aligned) required", fn, need);
   uint8_t *base = static_cast<uint8_t *>(ws);
   float *t32 = reinterpret_cast<float *>(base);
   void *gws = base + pl.t32;
@@ -552,6 +563,17 @@ int dsl_lora_gemm(const void *x, const void *w, const void *a_t, const void *b_t
   uint16_t *b2 = reinterpret_cast<uint16_t *>(base + pl.t32 + pl.ws + pl.t2);
   hipStream_t st = static_cast<hipStream_t>(stream);
   hipError_t e;
+  if (!packed) {
+    uint16_t *at = reinterpret_cast<uint16_t *>(base + pl.total);
+    uint16_t *bt = reinterpret_cast<uint16_t *>(base + pl.total + align256((size_t)(lr * k) * 2));
+    const bool dup = !pl.plain_bt();
+    e = dsl::launch_lora_pack(static_cast<const uint16_t *>(a_t), static_cast<const uint16_t *>(b_t),
+                              (int)num_loras, (int)k, (int)rank, (int)n, at, dup ? b2 : bt,
+                              (int)(dup ? pl.ld2 : lr), dup, st);
+    if (e != hipSuccess) return hip_status(e, fn);
+    a_t = at;
+    b_t = bt;
+  }
   if (pl.valu) {   // few tokens: fp32 T*s, the base GEMM, then Y += T*s B^T
     e = dsl::launch_lora_t(static_cast<const uint16_t *>(x), static_cast<const uint16_t *>(a_t),
                            (int)m, (int)k, (int)lr, (int)rank, scales, t32, nullptr, 0, st);
@@ -581,7 +603,7 @@ int dsl_lora_gemm(const void *x, const void *w, const void *a_t, const void *b_t
     if (e == hipSuccess)
       e = dsl::launch_lora_split(t32, (int)m, (int)lr, (int)pl.ld2, (int)rank, scales, t2, st);
   }
-  if (e == hipSuccess && !pl.rep)
+  if (e == hipSuccess && packed && !pl.rep)
     e = dsl::launch_lora_dup(static_cast<const uint16_t *>(b_t), (int)n, (int)lr, (int)pl.ld2, b2, st);
   if (e != hipSuccess) return hip_status(e, fn);
   dsl::GemmArgs g = bf16_args(x, w, y, m, n, k, ldy, false, gws, pl.ws);
@@ -603,6 +625,26 @@ int dsl_lora_gemm(const void *x, const void *w, const void *a_t, const void *b_t
       e = dsl::launch_gemm(dsl::MODE_BF16, bf16_args(t2, b2, y, m, n, pl.ld2, ldy, true, gws, pl.ws), st);
   }
   return hip_status(e, fn);
+}
+
+int dsl_lora_gemm(const void *x, const void *w, const void *a_t, const void *b_t,
+                  const float *scales, float *y, int64_t m, int64_t n, int64_t k, int64_t rank,
+                  int64_t num_loras, int64_t ldy, void *ws, size_t ws_bytes, void *stream) {
+  return run_lora("dsl_lora_gemm", x, w, a_t, b_t, true, scales, y, m, n, k, rank, num_loras, ldy, ws,
+                  ws_bytes, stream);
+}
+
+size_t dsl_lora_gemm_ab_workspace_bytes(int64_t m, int64_t n, int64_t k, int64_t rank,
+                                        int64_t num_loras) {
+  const size_t base = dsl_lora_gemm_workspace_bytes(m, n, k, rank, num_loras);
+  return base ? base + lora_pack_bytes(lora_plan(m, n, k, rank * num_loras), n, k, rank * num_loras) : 0;
+}
+
+int dsl_lora_gemm_ab(const void *x, const void *w, const void *a, const void *b, const float *scales,
+                     float *y, int64_t m, int64_t n, int64_t k, int64_t rank, int64_t num_loras,
+                     int64_t ldy, void *ws, size_t ws_bytes, void *stream) {
+  return run_lora("dsl_lora_gemm_ab", x, w, a, b, false, scales, y, m, n, k, rank, num_loras, ldy, ws,
+                  ws_bytes, stream);
 }
 
 size_t dsl_moe_route_workspace_bytes(int64_t tokens, int64_t topk, int64_t num_experts) {

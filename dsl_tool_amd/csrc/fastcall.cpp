@@ -471,6 +471,13 @@ PyObject *lora_gemm(PyObject *, PyObject *const *a, Py_ssize_t n) {
     return none();
   Tensor y;
   const bool ok = on_device(*x, [&] {
+    if (la->is_contiguous() && lb->is_contiguous()) {   // packed by the call itself
+      const size_t nb = dsl_lora_gemm_ab_workspace_bytes(m, nn, k, r, l);
+      const Tensor ws = bytes((int64_t)(nb > 256 ? nb : 256), *x);
+      y = empty({m, nn}, ScalarType::Float, *x);
+      return dsl_lora_gemm_ab(ptr(*x), ptr(*w), ptr(*la), ptr(*lb), ptr<float>(*sc), ptr<float>(y), m, nn, k, r,
+                              l, nn, ptr(ws), (size_t)ws.numel(), stream_of(*x)) == DSL_OK;
+    }
     const Tensor at = la->detach().permute({0, 2, 1}).reshape({l * r, k}).contiguous();
     const Tensor bt = lb->detach().permute({2, 0, 1}).reshape({nn, l * r}).contiguous();
     if (!aligned16(at) || !aligned16(bt)) return false;

@@ -252,6 +252,16 @@ int dsl_lora_gemm(const void *x, const void *w, const void *a_t, const void *b_t
                   int64_t rank, int64_t num_loras, int64_t ldy,
                   void *workspace, size_t workspace_bytes, void *stream);
 
+/* dsl_lora_gemm with the adapters in the reference's layout, a [num_loras][k]
+ * [rank] and b [num_loras][rank][n] (both contiguous, 2-byte aligned); they are
+ * packed into the workspace first, which holds that room too. */
+size_t dsl_lora_gemm_ab_workspace_bytes(int64_t m, int64_t n, int64_t k, int64_t rank,
+                                        int64_t num_loras);
+int dsl_lora_gemm_ab(const void *x, const void *w, const void *a, const void *b,
+                     const float *scales, float *y, int64_t m, int64_t n, int64_t k,
+                     int64_t rank, int64_t num_loras, int64_t ldy,
+                     void *workspace, size_t workspace_bytes, void *stream);
+
 /* ------------------------------------------------------------ MoE glue --
  * The steps either side of dsl_grouped_fp8_gemm in an MoE layer.  The
  * reference has no counterpart (its grouped GEMM takes rows already sorted

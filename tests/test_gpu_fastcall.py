@@ -127,3 +127,23 @@ def test_odd_calls_are_left_to_python():
     assert fast.rmsnorm_quant(x, w[0], 1, N.QFMT_MXFP4) is None
     with pytest.raises(ValueError, match="K mismatch"):
         G.fp8_gemm_packed(qa[:, :256].contiguous(), qw, sa, sw)
+
+
+@pytest.mark.parametrize("m,n,k,rank,loras", [
+    (1, 200, 136, 8, 1), (2, 72, 64, 16, 3), (40, 200, 136, 8, 3), (300, 264, 1096, 16, 5),
+    (512, 1024, 512, 16, 4), (700, 2056, 320, 72, 1), (1500, 2048, 1024, 32, 4)])
+def test_lora_adapters_packed_by_the_call(m, n, k, rank, loras):
+    """Contiguous adapters are turned to K-major rows by the call's own kernel;
+    a strided view of the same values takes the copies, with the same bytes."""
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    r = lambda *s: torch.randn(s, generator=g, device="cuda").bfloat16()
+    x, w, a, b = r(m, k), r(n, k).t(), r(loras, k, rank), r(loras, rank, n)
+    s = torch.rand(loras, generator=g, device="cuda")
+    a2 = torch.zeros((loras, k, rank + 1), dtype=a.dtype, device="cuda")
+    a2[:, :, :rank] = a
+    got = G.lora_fused_gemm(x, w, a, b, s)
+    assert torch.equal(got, G.lora_fused_gemm(x, w, a2[:, :, :rank], b, s))
+    ref = x.double() @ w.double()
+    for l in range(loras):
+        ref += s[l].double() * (x.double() @ a[l].double()) @ b[l].double()
+    assert (got.double() - ref).abs().max() <= 2e-5 * ref.abs().max()
