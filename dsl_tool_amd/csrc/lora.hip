@@ -57,41 +57,50 @@ __global__ __launch_bounds__(256) void lora_dup_kernel(const uint16_t *__restric
 
 // The adapters in the caller's layout to the GEMMs' in one launch: A [L][K][R]
 // -> a_t [L*R][K], and B [L*R][N] -> rows n of b_out (pitch ldb): B^T, or with
-// dup B^T | B^T | 0.  64 x 64 tiles turned in LDS, 2-byte reads and writes
+// dup B^T | B^T | 0.  64 x 16 tiles turned in LDS, 2-byte reads and writes
 // along the rows of each side; the first na blocks take A.  A few hundred KB,
 // so launches bound it: one where two copies and the doubling pass took 4.1 +
 // 4.1 + 3.1 us (four adapters of rank 16, K = N = 4096: the layer at M = 4 /
-// 512 / 4096 24.5 / 52.9 / 139.4 -> 20.2 / 49.0 / 135.9 us).
+// 512 / 4096 24.5 / 52.9 / 139.4 -> 20.2 / 49.0 / 135.9 us with 64 x 64 tiles).
+// 64 x 16 tiles, all four loads of a thread in flight: 6.5 -> 4.8 us, the layer
+// at M = 512 47.9 -> 44.7.
 __global__ __launch_bounds__(256) void lora_pack_kernel(const uint16_t *__restrict__ a,
                                                         const uint16_t *__restrict__ b, int L, int K, int R,
                                                         int N, int na, uint16_t *__restrict__ a_t,
                                                         uint16_t *__restrict__ b_out, int ldb, int dup) {
-  __shared__ uint16_t tile[64][66];
+  __shared__ uint16_t tile[64][18];
   const bool is_a = (int)blockIdx.x < na;
   const int LR = L * R, rows = is_a ? K : LR, cols = is_a ? R : N;
   int id = is_a ? blockIdx.x : blockIdx.x - na;
-  const int nc = (cols + 63) / 64, nr = (rows + 63) / 64;
-  const int c0 = id % nc * 64;
+  const int nc = (cols + 15) / 16, nr = (rows + 63) / 64;
+  const int c0 = id % nc * 16;
   id /= nc;
   const int r0 = id % nr * 64, l = id / nr;                 // l: adapter (A only)
   const uint16_t *src = is_a ? a + (int64_t)l * K * R : b;
-  const int h = rows - r0 < 64 ? rows - r0 : 64, w = cols - c0 < 64 ? cols - c0 : 64;
-  for (int i = threadIdx.x; i < h * w; i += 256) {
-    const int r = i / w, c = i - r * w;
-    tile[r][c] = src[(int64_t)(r0 + r) * cols + c0 + c];
+  const int h = rows - r0, w = cols - c0;                   // what exists from here on
+  const int t = threadIdx.x, tc = t & 15, tr = t >> 4, wr = t & 63, wc = t >> 6;
+  uint16_t v[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int r = tr + 16 * j;
+    v[j] = src[(int64_t)(r0 + (r < h ? r : 0)) * cols + c0 + (tc < w ? tc : 0)];
   }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) tile[tr + 16 * j][tc] = v[j];
   __syncthreads();
   uint16_t *dst = is_a ? a_t + (int64_t)l * R * K : b_out;
   const int64_t ld = is_a ? K : ldb;
-  for (int i = threadIdx.x; i < h * w; i += 256) {
-    const int c = i / h, r = i - c * h;
-    uint16_t *p = dst + (c0 + c) * ld + r0 + r;
-    p[0] = tile[r][c];
-    if (!is_a && dup) p[LR] = tile[r][c];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int c = wc + 4 * j;
+    if (c >= w || wr >= h) continue;
+    uint16_t *p = dst + (c0 + c) * ld + r0 + wr;
+    p[0] = tile[wr][c];
+    if (!is_a && dup) p[LR] = tile[wr][c];
   }
   if (!is_a && dup && r0 == 0) {                            // the padding columns
     const int z = ldb - 2 * LR;
-    for (int i = threadIdx.x; i < z * w; i += 256) {
+    for (int i = threadIdx.x; i < z * (w < 16 ? w : 16); i += 256) {
       const int c = i / z;
       dst[(c0 + c) * ld + 2 * LR + (i - c * z)] = 0;
     }
@@ -259,7 +268,7 @@ hipError_t launch_lora_dup(const uint16_t *bt, int N, int LR, int ld2, uint16_t 
 hipError_t launch_lora_pack(const uint16_t *a, const uint16_t *b, int L, int K, int R, int N, uint16_t *a_t,
                             uint16_t *b_out, int ldb, bool dup, hipStream_t st) {
   const int64_t LR = (int64_t)L * R;
-  const int64_t na = (int64_t)L * ((K + 63) / 64) * ((R + 63) / 64), nb = ((LR + 63) / 64) * ((N + 63) / 64);
+  const int64_t na = (int64_t)L * ((K + 63) / 64) * ((R + 15) / 16), nb = ((LR + 63) / 64) * ((N + 15) / 16);
   if (na + nb > 0x7fffffff || ldb < (dup ? 2 : 1) * LR) return hipErrorInvalidValue;
   if (na + nb == 0) return hipSuccess;
   lora_pack_kernel<<<(unsigned)(na + nb), 256, 0, st>>>(a, b, L, K, R, N, (int)na, a_t, b_out, ldb, dup);
