@@ -7,7 +7,10 @@ two share devices, streams and allocations.
 
 There is no fallback: if the library is missing or fails to load, every
 entry point raises ``DslLibraryError``.  ``fast()`` is the CPython extension
-that makes the same calls for well-formed tensors without the ctypes layer.
+that makes the same calls for well-formed tensors without the ctypes layer;
+it saves host time only, and where it is missing or does not load (it is
+bound to the torch build it was compiled against) every call goes through
+ctypes.
 """
 from __future__ import annotations
 
@@ -17,6 +20,7 @@ import importlib.util
 import os
 import re
 import threading
+import warnings
 
 import torch  # noqa: F401  (must precede loading the HIP library, see above)
 
@@ -128,8 +132,9 @@ def lib():
 
 
 class _NoFast:
-    """Stands for the extension while the library is not built: every call is
-    left to the Python path, whose own checks come first."""
+    """Stands for the extension where there is none, or while the library is
+    not built: every call is left to the Python path, whose own checks come
+    first."""
 
     def __getattr__(self, name):
         return lambda *args: None
@@ -141,7 +146,8 @@ _fast = None
 def fast():
     """The ``dsl_fast`` extension (loaded once): functions that take the
     operands of a well-formed call and return its results, or None for the
-    Python path to handle the call."""
+    Python path to handle the call.  Without the extension every call is the
+    Python path's, after one warning."""
     global _fast
     if _fast is not None:
         return _fast
@@ -150,16 +156,15 @@ def fast():
     lib()
     with _lock:
         if _fast is None:
-            if not os.path.exists(FAST_PATH):
-                raise DslLibraryError(
-                    f"extension not built: {FAST_PATH} (run `python -m dsl_tool_amd.build`)")
             loader = importlib.machinery.ExtensionFileLoader("dsl_fast", FAST_PATH)
             try:
                 mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("dsl_fast", loader))
                 loader.exec_module(mod)
-            except ImportError as exc:
-                raise DslLibraryError(f"cannot load {FAST_PATH}: {exc}") from exc
-            _fast = mod
+                _fast = mod
+            except ImportError as exc:     # also where the file is missing
+                _fast = _NoFast()
+                warnings.warn(f"{FAST_PATH} does not load ({exc}); calls take the slower ctypes path "
+                              "(rebuild with `python -m dsl_tool_amd.build`)", RuntimeWarning, stacklevel=3)
     return _fast
 
 

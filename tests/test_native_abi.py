@@ -3,6 +3,7 @@ declares, and rejects bad arguments with a status code before it would
 launch anything (no GPU is touched by any call here)."""
 import ctypes
 import os
+import warnings
 
 import pytest
 
@@ -254,3 +255,25 @@ def test_noalloc_quantizer_validation(lib):
     rc = lib.dsl_quant_fp8_tensor_noalloc(fake, 4, 64, 64, 1, N.IN_BF16, fake, None, None)
     assert rc == N.DSL_ERR_ARG and "scale" in _err(lib)
     assert lib.dsl_quant_fp8_tensor_noalloc(None, 0, 64, 64, 1, N.IN_BF16, None, None, None) == 0
+
+
+@pytest.mark.parametrize("content", [None, b"not a shared object"])
+def test_extension_is_optional(lib, content, tmp_path, monkeypatch):
+    """A missing or unloadable dsl_fast.so leaves every call to the ctypes
+    path, with one warning (no call is refused for it)."""
+    import torch
+
+    from dsl_tool_amd import quant as Q
+    path = tmp_path / "dsl_fast.so"
+    if content is not None:
+        path.write_bytes(content)
+    monkeypatch.setattr(N, "FAST_PATH", str(path))
+    monkeypatch.setattr(N, "_fast", None)
+    with pytest.warns(RuntimeWarning, match="ctypes path"):
+        fast = N.fast()
+    assert fast.fp8_gemm(1, 2) is None and fast.quant_mxfp4() is None
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert N.fast() is fast
+        with pytest.raises(ValueError, match="GPU"):      # the Python path's own check
+            Q.quant_fp8_tensor(torch.zeros(4, 4, dtype=torch.bfloat16))
