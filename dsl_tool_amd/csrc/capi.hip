@@ -801,4 +801,23 @@ int dsl_moe_combine(const void *y, int64_t rows, int64_t n, int64_t ldy, const i
                     fn);
 }
 
+// Not part of the ABI (no header declares them): which kernel a call would take,
+// for the tests; no GPU is touched.  kind: a GEMM mode of launch.h.
+int dsl_test_gemm_route(int kind, int64_t m, int64_t n, int64_t k, int out_dtype, char *buf, size_t len) {
+  dsl::describe_gemm(kind, m, n, k, out_dtype == DSL_OUT_F32, buf, len);
+  return DSL_OK;
+}
+
+const char *dsl_test_grouped_route(int64_t num_groups, int64_t rows, int64_t n, int64_t k, int gather) {
+  static const int32_t some = 0;
+  dsl::GroupedArgs p{};
+  p.G = (int)num_groups;
+  p.rows = (int)rows;
+  p.N = (int)n;
+  p.K = (int)k;
+  p.arow = gather ? &some : nullptr;
+  p.xrows = gather ? (int)rows : 0;
+  return dsl::describe_grouped(p);
+}
+
 }  // extern "C"

@@ -616,13 +616,6 @@ struct StreamPlan {
   int tma, tn;
 };
 
-// Activation tiles by M (16, 32 or 64 rows per workgroup; 256-byte chunks
-// for the skinny ones, 512-byte chunks otherwise; whole rows of an odd number
-// of 256-byte chunks take the 32-row tiles), and the most W tiles
-// per workgroup (4, 2, 1) that still leave >= 192 workgroups: fewer but
-// larger workgroups read A and W fewer times (measured at M = 96..256), as
-// long as they cover most CUs.  DSL_GEMM_STREAM_TMA / DSL_GEMM_STREAM_TN
-// override them (tuning).
 // K whose rows (or scale rows) take the TAIL form of the kernel: rows of no
 // whole 256-byte chunks, FP8 / MXFP4 scale rows of no whole 16 bytes (K %
 // 512), NVFP4 ones (K % 256), or scale arrays that are not 16-byte aligned;
@@ -636,6 +629,13 @@ bool needs_tail(int mode, int M, int K, int Kb, bool scales16) {
 
 bool stream_rows64(int M, int Kb, bool tail) { return tail ? M > 96 : Kb % 512 == 0; }
 
+// Activation tiles by M (16, 32 or 64 rows per workgroup; 256-byte chunks
+// for the skinny ones, 512-byte chunks otherwise; whole rows of an odd number
+// of 256-byte chunks take the 32-row tiles), and the most W tiles
+// per workgroup (4, 2, 1) that still leave >= 192 workgroups: fewer but
+// larger workgroups read A and W fewer times (measured at M = 96..256), as
+// long as they cover most CUs.  DSL_GEMM_STREAM_TMA / DSL_GEMM_STREAM_TN
+// override them (tuning).
 StreamPlan plan_for(int mode, int M, int N, int Kb, bool tail) {
   StreamPlan pl;
   // Ragged rows take the 64-row blocks from 97 rows (in 256-byte chunks):
@@ -761,6 +761,14 @@ bool stream_supported(int mode, int M, int N, int K, int Kb, bool scales4) {
 
 bool stream_blocks64(int mode, int M, int K, int Kb, bool scales16) {
   return stream_rows64(M, Kb, needs_tail(mode, M, K, Kb, scales16));
+}
+
+bool stream_plan(int mode, int M, int N, int K, int Kb, bool scales16, int *tma, int *tn) {
+  const bool tail = needs_tail(mode, M, K, Kb, scales16);
+  const StreamPlan pl = plan_for(mode, M, N, Kb, tail);
+  *tma = pl.tma;
+  *tn = pl.tn;
+  return tail;
 }
 
 hipError_t launch_gemm_stream(int mode, const GemmArgs &p, hipStream_t st) {

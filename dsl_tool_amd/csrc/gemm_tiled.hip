@@ -1,6 +1,7 @@
 // Dense quantized GEMM: C[M,N] = A[M,K] . W[N,K]^T on gfx950 MFMA.
 // Variant selection (tile shape, split-K) lives in launch_gemm below.
 #include <algorithm>
+#include <cstdio>
 #include <cstdlib>
 #include <cstring>
 
@@ -253,22 +254,29 @@ static bool stream_enabled() {
   return on;
 }
 
+// DSL_GEMM_PIPE: -1 unset, -2 off, else the forced variant.
+static int pipe_switch() {
+  static const int forced = [] {
+    if (env_off("DSL_GEMM_PIPE")) return -2;
+    const char *e = getenv("DSL_GEMM_PIPE");
+    return (e && e[0] >= '1' && e[0] <= '9' && !e[1]) ? e[0] - '0' : -1;
+  }();
+  return forced;
+}
+
 // `padded`: a workspace for padded scale rows is there.  `ragged` false: the
-// kernel that serves the shape without the ragged forms (rows and scale rows of
-// whole steps only); the workspace contract is that route's.
-static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc16, bool padded,
-                       bool ragged = true) {
+// kernel that serves the shape without the ragged forms and the one-round tiles
+// (rows and scale rows of whole steps only); the workspace contract is that
+// route's.
+static Route pick_route(int mode, int M, int N, int K, int Kb, bool sc4, bool sc16, bool padded,
+                        bool ragged) {
   static const bool decode_on = !env_off("DSL_GEMM_DECODE");
   const bool stream_on = stream_enabled();
   const char *skinny = getenv("DSL_GEMM_SKINNY");      // read per launch (tests switch it)
   const bool skinny_stream = skinny && strcmp(skinny, "stream") == 0;
   const bool skinny_decode = skinny && strcmp(skinny, "decode") == 0;
   static const bool persist_on = !env_off("DSL_GEMM_PERSIST");
-  static const int pipe_forced = [] {
-    if (env_off("DSL_GEMM_PIPE")) return -2;
-    const char *e = getenv("DSL_GEMM_PIPE");
-    return (e && e[0] >= '1' && e[0] <= '9' && !e[1]) ? e[0] - '0' : -1;
-  }();
+  const int pipe_forced = pipe_switch();
   Route r{PATH_TILED, -1, plan_for(M, N, Kb)};
   bool streamable = stream_on && stream_supported(mode, M, N, K, Kb, sc4) &&
                     (ragged || stream_whole(mode, K, Kb, sc16));
@@ -443,6 +451,10 @@ static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc1
   return r;
 }
 
+static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc16, bool padded) {
+  return pick_route(mode, M, N, K, Kb, sc4, sc16, padded, true);
+}
+
 bool gemm_routes_to_stream(int mode, int64_t M, int64_t N, int64_t K, bool or_pipe, bool accumulate) {
   const int Kb = (mode == MODE_MXFP4 || mode == MODE_NVFP4) ? (int)(K / 2)
                                                             : (mode == MODE_BF16 ? (int)(2 * K) : (int)K);
@@ -455,7 +467,7 @@ bool gemm_routes_to_stream(int mode, int64_t M, int64_t N, int64_t K, bool or_pi
 size_t gemm_workspace_required(int mode, int64_t M, int64_t N, int64_t K, bool accumulate) {
   const int Kb = (mode == MODE_MXFP4 || mode == MODE_NVFP4) ? (int)(K / 2)
                                                             : (mode == MODE_BF16 ? (int)(2 * K) : (int)K);
-  Route r = route_for(mode, (int)M, (int)N, (int)K, Kb, true, true, false, false);
+  Route r = pick_route(mode, (int)M, (int)N, (int)K, Kb, true, true, false, false);
   if (accumulate) r.path = PATH_TILED;
   return (r.path == PATH_TILED && r.tiled.ksplit > 1)
              ? (size_t)r.tiled.ksplit * (size_t)splitk_slice(M, N) * sizeof(float)
@@ -493,13 +505,6 @@ static GemmArgs columns_from(int mode, GemmArgs p, int n1) {
 // per-tensor / block / MXFP4 / NVFP4 / bf16: 2304x7680x4096 (270 tiles) 90 ->
 // 75, 106 -> 93, 63 -> 58, 190 -> 178, 177 -> 145; 4300x4300x4096 (289 tiles)
 // 141 -> 116, 158 -> 132, 113 -> 101, 241 -> 218, 230 -> 185.
-static int pipe_variant(int mode, int M, int N) {
-  const int64_t cu = device_cu_count();
-  if (mode == MODE_NVFP4) return 1;
-  if ((int64_t)((M + 63) / 64) * ((N + 127) / 128) <= cu) return 6;
-  return (int64_t)((M + 127) / 128) * ((N + 127) / 128) <= cu ? 7 : 1;
-}
-
 static int strip_columns(const GemmArgs &p) {
   const int cu = device_cu_count();
   const int nbm = (p.M + 255) / 256, nbn = (p.N + 255) / 256;
@@ -508,6 +513,51 @@ static int strip_columns(const GemmArgs &p) {
   const int keep = (int)(full / nbm);                // whole columns of tiles in whole rounds
   if ((int64_t)nbm * (nbn - keep) > cu / 4 || keep < 1) return 0;
   return p.N - keep * 256;
+}
+
+// Pipelined tiles for those columns: 64x128 or deep 128x128 ones where one round
+// holds them, as pick_route has it.
+static int pipe_variant(int mode, int M, int N) {
+  const int64_t cu = device_cu_count();
+  if (mode == MODE_NVFP4) return 1;
+  if ((int64_t)((M + 63) / 64) * ((N + 127) / 128) <= cu) return 6;
+  return (int64_t)((M + 127) / 128) * ((N + 127) / 128) <= cu ? 7 : 1;
+}
+
+void describe_gemm(int mode, int64_t M, int64_t N, int64_t K, bool, char *buf, size_t len) {
+  const int Kb = (mode == MODE_MXFP4 || mode == MODE_NVFP4) ? (int)(K / 2)
+                                                            : (mode == MODE_BF16 ? (int)(2 * K) : (int)K);
+  auto name = [&](const Route &r, int m, int n, char *to, size_t room) {
+    static const char *const tiles[] = {"256x256", "128x128", "", "", "", "", "64x128 deep", "128x128 deep"};
+    int tma = 0, tn = 0;
+    if (r.path == PATH_STREAM) {
+      const bool tail = stream_plan(mode, m, n, (int)K, Kb, true, &tma, &tn);
+      snprintf(to, room, "stream%s %dx%d", tail ? " tail" : "", 16 * tma, 16 * tn);
+    } else if (r.path == PATH_PIPE) {
+      snprintf(to, room, "pipe %s", r.variant >= 0 && r.variant < 8 ? tiles[r.variant] : "forced");
+    } else if (r.path == PATH_PERSIST) {
+      snprintf(to, room, "persist 256x%d", r.narrow ? 128 : 256);
+    } else if (r.path == PATH_TILED) {
+      snprintf(to, room, "split %dx%d/%d", r.tiled.bm, r.tiled.bn, r.tiled.ksplit);
+    } else {
+      snprintf(to, room, "decode");
+    }
+  };
+  Route r = route_for(mode, (int)M, (int)N, (int)K, Kb, true, true, true);
+  name(r, (int)M, (int)N, buf, len);
+  GemmArgs p{};
+  p.M = (int)M;
+  p.N = (int)N;
+  const int strip = r.path != PATH_PERSIST || r.narrow || r.pad_scales ? 0 : strip_columns(p);
+  if (strip == 0) return;
+  Route rest = route_for(mode, (int)M, strip, (int)K, Kb, true, true, false);
+  if (rest.path != PATH_STREAM) {
+    rest.path = PATH_PIPE;
+    rest.variant = pipe_variant(mode, (int)M, strip);
+  }
+  const size_t used = strlen(buf);
+  snprintf(buf + used, len - used, " + ");
+  name(rest, (int)M, strip, buf + strlen(buf), len - strlen(buf));
 }
 
 hipError_t launch_gemm(int mode, GemmArgs p, hipStream_t st) {

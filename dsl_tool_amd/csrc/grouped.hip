@@ -231,13 +231,17 @@ static void launch_grouped_pipe_cfg(const GroupedArgs &p, hipStream_t st) {
   grouped_pipe_kernel<Cfg><<<(unsigned)grid, Cfg::NT, 0, st>>>(p);
 }
 
-hipError_t launch_grouped_fp8(GroupedArgs p, hipStream_t st) {
-  if (p.rows == 0 || p.N == 0) return hipSuccess;
+enum { GROUPED_NONE, GROUPED_STREAM, GROUPED_PERSIST, GROUPED_PIPE256, GROUPED_PIPE128, GROUPED_TILED };
+
+static int grouped_route(const GroupedArgs &p) {
   const int avg = p.rows / (p.G > 0 ? p.G : 1);
-  if (p.arow) {   // the gather form: streaming tiles at decode sizes, else the persistent kernel
-    if (avg < 48 && grouped_stream_supported(p)) return launch_grouped_stream(p, st);
-    return grouped_persist_supported(p) ? launch_grouped_persist(p, st) : hipErrorInvalidValue;
-  }
+  // Few rows per group (MoE decode): the streaming tiles read each group's W
+  // once with its rows (64 experts, N=1536 K=2048, 32 tokens x top-8: 37.4
+  // against 53.3 us); from 64 rows per group the tiles win again (512
+  // tokens: 63.8 us persistent, 117.9 streaming).
+  if (avg < 48 && grouped_stream_supported(p)) return GROUPED_STREAM;
+  // the gather form has no other kernel than the persistent one
+  if (p.arow) return grouped_persist_supported(p) ? GROUPED_PERSIST : GROUPED_NONE;
   // DSL_GEMM_PERSIST=0 keeps the per-tile pipelined walk below (tuning)
   static const bool persist_on = [] {
     const char *e = getenv("DSL_GEMM_PERSIST");
@@ -246,29 +250,35 @@ hipError_t launch_grouped_fp8(GroupedArgs p, hipStream_t st) {
     for (int i = 0; i < 7 && e[i]; ++i) v[i] = (char)((e[i] >= 'A' && e[i] <= 'Z') ? e[i] + 32 : e[i]);
     return !(strcmp(v, "0") == 0 || strcmp(v, "off") == 0 || strcmp(v, "false") == 0);
   }();
-  // Few rows per group (MoE decode): the streaming tiles read each group's W
-  // once with its rows (64 experts, N=1536 K=2048, 32 tokens x top-8: 37.4
-  // against 53.3 us); from 64 rows per group the tiles win again (512
-  // tokens: 63.8 us persistent, 117.9 streaming).
-  if (avg < 48 && grouped_stream_supported(p)) return launch_grouped_stream(p, st);
   // From there on the persistent 256x256 walk, also for groups well below
   // 256 rows: 64 experts, N=1536 K=2048, 1024 tokens x top-8 (128 rows per
   // expert): 67.6 against 110.2 us on the 128x256 pipelined tiles; 384
   // tokens: 63.8 against 71.9.
-  if (persist_on && grouped_persist_supported(p)) return launch_grouped_persist(p, st);
-  if (p.K % 64 == 0) {
-    // DSL_GROUPED_TILE=256 / 128 forces the 256x256 / 128x256 tile (tuning)
-    static const int forced = [] {
-      const char *e = getenv("DSL_GROUPED_TILE");
-      return e ? atoi(e) : 0;
-    }();
-    if (forced == 256 || (forced != 128 && avg >= 256))
-      launch_grouped_pipe_cfg<PipeCfg<MODE_FP8_TENSOR, 256, 256, 2, 4, 4, 64>>(p, st);
-    else
-      launch_grouped_pipe_cfg<PipeCfg<MODE_FP8_TENSOR, 128, 256, 2, 4, 4, 64>>(p, st);
-    return hipGetLastError();
+  if (persist_on && grouped_persist_supported(p)) return GROUPED_PERSIST;
+  if (p.K % 64 != 0) return GROUPED_TILED;
+  // DSL_GROUPED_TILE=256 / 128 forces the 256x256 / 128x256 tile (tuning)
+  static const int forced = [] {
+    const char *e = getenv("DSL_GROUPED_TILE");
+    return e ? atoi(e) : 0;
+  }();
+  return forced == 256 || (forced != 128 && avg >= 256) ? GROUPED_PIPE256 : GROUPED_PIPE128;
+}
+
+const char *describe_grouped(const GroupedArgs &p) {
+  static const char *const names[] = {"none", "stream", "persist", "pipe 256x256", "pipe 128x256", "tiled"};
+  return names[grouped_route(p)];
+}
+
+hipError_t launch_grouped_fp8(GroupedArgs p, hipStream_t st) {
+  if (p.rows == 0 || p.N == 0) return hipSuccess;
+  switch (grouped_route(p)) {
+    case GROUPED_STREAM: return launch_grouped_stream(p, st);
+    case GROUPED_PERSIST: return launch_grouped_persist(p, st);
+    case GROUPED_PIPE256: launch_grouped_pipe_cfg<PipeCfg<MODE_FP8_TENSOR, 256, 256, 2, 4, 4, 64>>(p, st); break;
+    case GROUPED_PIPE128: launch_grouped_pipe_cfg<PipeCfg<MODE_FP8_TENSOR, 128, 256, 2, 4, 4, 64>>(p, st); break;
+    case GROUPED_TILED: launch_grouped_cfg<TileCfg<MODE_FP8_TENSOR, 128, 128, 2, 2>>(p, st); break;
+    default: return hipErrorInvalidValue;
   }
-  launch_grouped_cfg<TileCfg<MODE_FP8_TENSOR, 128, 128, 2, 2>>(p, st);
   return hipGetLastError();
 }
 

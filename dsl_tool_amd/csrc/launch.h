@@ -117,6 +117,8 @@ bool stream_supported(int mode, int M, int N, int K, int Kb, bool scales4);
 bool stream_whole(int mode, int K, int Kb, bool scales16);
 // Whether M > 32 rows stream in 64-row blocks, else in 32-row blocks.
 bool stream_blocks64(int mode, int M, int K, int Kb, bool scales16);
+// The plan's activation and W tiles per workgroup; whether the TAIL form runs.
+bool stream_plan(int mode, int M, int N, int K, int Kb, bool scales16, int *tma, int *tn);
 hipError_t launch_gemm_stream(int mode, const GemmArgs &p, hipStream_t st);
 
 // Picks a kernel variant for the shape and launches it (plus the split-K
@@ -128,6 +130,9 @@ hipError_t launch_gemm(int mode, GemmArgs args, hipStream_t st);
 // pitch; without it those take a kernel that does not need the copy.
 size_t gemm_workspace_required(int mode, int64_t M, int64_t N, int64_t K, bool accumulate = false);
 size_t gemm_workspace_bytes(int mode, int64_t M, int64_t N, int64_t K, bool accumulate = false);
+// The kernel launch_gemm would run (aligned operands, the queried workspace) as
+// text, for the tests.
+void describe_gemm(int mode, int64_t M, int64_t N, int64_t K, bool f32, char *buf, size_t len);
 // Whether launch_gemm takes the streaming kernel (or_pipe: or the pipelined
 // tiles) for this shape (aligned scales; accumulate: C += result, fp32 out).
 bool gemm_routes_to_stream(int mode, int64_t M, int64_t N, int64_t K, bool or_pipe = false,
@@ -153,6 +158,7 @@ struct GroupedArgs {
   int xrows = 0;
 };
 hipError_t launch_grouped_fp8(GroupedArgs args, hipStream_t st);
+const char *describe_grouped(const GroupedArgs &args);   // for the tests
 // Grouped FP8 on the persistent kernel (K % 16 == 0, 128 <= K < 2^24).
 bool grouped_persist_supported(const GroupedArgs &args);
 hipError_t launch_grouped_persist(const GroupedArgs &args, hipStream_t st);
