@@ -160,6 +160,7 @@ int dsl_quant_fp8_rows_batched(const void *x, int64_t batch, int64_t rows, int64
   if (batch == 0 || rows == 0 || cols == 0) return ok();
   if (sc < rows || (batch > 1 && sb <= 0))
     return fail(DSL_ERR_ARG, "%s: need stride_col >= rows and a positive stride_batch", fn);
+  if (rows >= (int64_t)1 << 29) return fail(DSL_ERR_ARG, "%s: rows=%lld must be < 2^29", fn, (long long)rows);
   if ((rc = check_out(fn, q, "q"))) return rc;
   if (!scales) return fail(DSL_ERR_ARG, "%s: scales is NULL", fn);
   return hip_status(dsl::launch_quant_fp8_rows_batched(x, x_dtype == DSL_IN_F32, batch, rows, cols, sb, sc, q,
@@ -818,6 +819,11 @@ const char *dsl_test_grouped_route(int64_t num_groups, int64_t rows, int64_t n, 
   p.arow = gather ? &some : nullptr;
   p.xrows = gather ? (int)rows : 0;
   return dsl::describe_grouped(p);
+}
+
+int dsl_test_quant_transposed(const void *x, int x_dtype, int64_t rows, int64_t cols, int64_t sr, int64_t sc,
+                              int64_t group_rows, int64_t group_cols) {
+  return dsl::quant_fp8_blocks_transposed(x, x_dtype == DSL_IN_F32, rows, cols, sr, sc, group_rows, group_cols);
 }
 
 }  // extern "C"

@@ -17,6 +17,9 @@ hipError_t launch_quant_fp8_tensor(const void *x, bool f32, int64_t rows, int64_
 hipError_t launch_quant_fp8_blocks(const void *x, bool f32, int64_t rows, int64_t cols,
                                    int64_t sr, int64_t sc, int64_t gr, int64_t gc, uint8_t *q,
                                    float *scales, hipStream_t st);
+// Whether those are read through the transposed-tile kernel (for the tests).
+bool quant_fp8_blocks_transposed(const void *x, bool f32, int64_t rows, int64_t cols, int64_t sr, int64_t sc,
+                                 int64_t gr, int64_t gc);
 hipError_t launch_quant_fp8_rows_batched(const void *x, bool f32, int64_t batch, int64_t rows, int64_t cols,
                                          int64_t xb, int64_t ld, uint8_t *q, float *scales, hipStream_t st);
 hipError_t launch_quant_mxfp4(const void *x, bool f32, int64_t rows, int64_t cols, int64_t sr,

@@ -906,10 +906,33 @@ static bool f32_vec_ok(const void *x, int64_t cols, int64_t sr, int64_t sc) {
 }
 
 // Unit row stride: a [cols][sc] matrix in memory whose contiguous axis is the
-// rows (rows > 1, else the row kernels read it as well).
+// rows (rows > 1, else the row kernels read it as well; the grid's x axis holds
+// 2^32 threads).
 static bool trans_ok(int64_t rows, int64_t cols, int64_t sr, int64_t sc) {
-  return sr == 1 && sc >= rows && rows > 1 && cols > 1 && (rows + 63) / 64 < ((int64_t)1 << 31) &&
+  return sr == 1 && sc >= rows && rows > 1 && cols > 1 && rows < ((int64_t)1 << 29) &&
          (cols + 127) / 128 <= 65535;
+}
+
+// 16-byte loads of 8 rows (bf16; fp32: two) need whole 8-row runs and aligned
+// columns; rows past the end are masked 8 at a time.
+template <typename T>
+static bool trans_vec(const T *x, int64_t rows, int64_t ld, int64_t xb) {
+  constexpr int per = 16 / sizeof(T);
+  return rows % 8 == 0 && ld % per == 0 && xb % per == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
+}
+
+// One scale over more than 256 columns of a row: the transposed kernel walks
+// them in one workgroup per 64 rows, the strided tile kernel starts one per
+// scale, so few scales stay there.  Scales per CU from which the former wins
+// (us, strided / transposed; N rows, one scale each): 4 by whole 8-row runs (N=896
+// K=2048 bf16 18.1 / 19.9, N=1280 28.6 / 20.0; N=64 K=8192 22.9 / 68.0), fp32
+// short groups 6 (N=1024 K=512 7.1 / 9.3), element loads 12 (N=1500 K=2048
+// 31.5 / 60.7, N=4100 K=512 20.7 / 16.2).  Below 16 rows most of a tile's 64
+// rows do not exist (N=2, 1 x 512 groups, K=1048576: 13.8 / 41.4).
+template <typename T>
+static bool trans_long_groups(const T *x, int64_t rows, int64_t cols, int64_t ld, int64_t gc) {
+  const int per_cu = !trans_vec(x, rows, ld, 0) ? 12 : (sizeof(T) == 4 && gc < 2048 ? 6 : 4);
+  return rows >= 16 && rows * ((cols - 1) / gc + 1) >= (int64_t)per_cu * device_cu_count();
 }
 
 template <int KIND, int NC, typename T>
@@ -920,10 +943,7 @@ static void launch_trans(const T *x, int64_t rows, int64_t cols, int64_t ld, int
   const int64_t span = KIND == KIND_FP8 ? gc : KT;
   const dim3 grid((unsigned)((rows + 8 * NC - 1) / (8 * NC)), (unsigned)((cols + span - 1) / span),
                   (unsigned)batch);
-  // 16-byte loads of 8 rows (bf16; fp32: two) need whole 8-row runs and
-  // aligned columns; rows past the end are masked 8 at a time
-  const bool vec = rows % 8 == 0 && ld % (16 / sizeof(T)) == 0 && xb % (16 / sizeof(T)) == 0 &&
-                   reinterpret_cast<uintptr_t>(x) % 16 == 0;
+  const bool vec = trans_vec(x, rows, ld, xb);
   auto go = [&](auto multi) {
     constexpr bool MULTI = decltype(multi)::value;
     if (vec)
@@ -943,21 +963,35 @@ static void launch_trans(const T *x, int64_t rows, int64_t cols, int64_t ld, int
 }
 
 // FP8 scale groups the transposed kernel takes: 1 x gc with gc whole 128-column
-// tiles (or one group per row), 128 x 128.
+// tiles (or one group per row), 128 x 128 (fewer than 8 rows: 4.6 us / 3.7 on the
+// strided kernel, N=4 K=512 fp32).
+template <typename T>
+static bool trans_fp8_takes(const T *x, int64_t rows, int64_t cols, int64_t sr, int64_t sc, int64_t gr,
+                            int64_t gc) {
+  if (!trans_ok(rows, cols, sr, sc)) return false;
+  if (gr == 1 && (gc % 128 == 0 || gc >= cols)) {
+    const int64_t g = gc < cols ? gc : cols;
+    return g <= 256 || trans_long_groups(x, rows, cols, sc, g);
+  }
+  return gr == 128 && gc == 128 && rows >= 8;
+}
+
+bool quant_fp8_blocks_transposed(const void *x, bool f32, int64_t rows, int64_t cols, int64_t sr, int64_t sc,
+                                 int64_t gr, int64_t gc) {
+  return f32 ? trans_fp8_takes(static_cast<const float *>(x), rows, cols, sr, sc, gr, gc)
+             : trans_fp8_takes(static_cast<const uint16_t *>(x), rows, cols, sr, sc, gr, gc);
+}
+
 template <typename T>
 static bool launch_trans_fp8(const T *x, int64_t rows, int64_t cols, int64_t sr, int64_t sc,
                              int64_t gr, int64_t gc, uint8_t *q, float *scales, hipStream_t st) {
-  if (!trans_ok(rows, cols, sr, sc)) return false;
-  if (gr == 1 && (gc % 128 == 0 || gc >= cols)) {
-    const int64_t g = gc >= cols ? (cols + 127) / 128 * 128 : gc;
-    launch_trans<KIND_FP8, 8>(x, rows, cols, sc, g, q, scales, nullptr, 0, nullptr, st);
-    return true;
-  }
-  if (gr == 128 && gc == 128) {
+  if (!trans_fp8_takes(x, rows, cols, sr, sc, gr, gc)) return false;
+  if (gr == 1)
+    launch_trans<KIND_FP8, 8>(x, rows, cols, sc, gc >= cols ? (cols + 127) / 128 * 128 : gc, q, scales, nullptr, 0,
+                              nullptr, st);
+  else
     launch_trans<KIND_FP8, 16>(x, rows, cols, sc, gc, q, scales, nullptr, 0, nullptr, st);
-    return true;
-  }
-  return false;
+  return true;
 }
 
 template <int KIND, int T, int U>
@@ -1238,7 +1272,12 @@ hipError_t launch_quant_nvfp4(const void *xv, bool f32, int64_t rows, int64_t co
     if (f32_vec_ok(xv, cols, sr, sc))
       launch_f32_rows<KIND_NV, 2, 1>(static_cast<const float *>(xv), rows, cols, sr, q, e4m3s,
                                      partial, np, gscale, st);
-    else if (trans_ok(rows, cols, sr, sc))
+    else if (trans_ok(rows, cols, sr, sc) &&
+             (trans_vec(static_cast<const float *>(xv), rows, sc, 0) ||
+              rows * cols >= (cols >= 1024 ? (int64_t)1 << 20 : (int64_t)9 << 18)))
+      // element loads pay on large sources only (us, strided / transposed): N=333
+      // K=2048 15.8 / 15.9, N=1500 25.4 / 22.8; N=4100 K=512 17.4 / 20.4, N=5001
+      // 22.1 / 18.4
       launch_trans<KIND_NV, 8>(static_cast<const float *>(xv), rows, cols, sc, 256, q, e4m3s, partial, np, gscale, st);
     else
       quant_group_scalar_kernel<KIND_NV, float><<<grid_for(rows * (cols / 16), 256), 256, 0, st>>>(

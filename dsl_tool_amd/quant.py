@@ -74,6 +74,22 @@ def quant_fp8_blocks(x: torch.Tensor, group_rows: int, group_cols: int):
     return q, scales
 
 
+def _rows_in_place(G: int, R: int, C: int, esize: int, stride_batch: int, stride_col: int, ptr: int) -> bool:
+    """Whether reading [G, K, N] storage in place beats the copy to rows.  One
+    workgroup walks all of K for 64 rows of one matrix, so few of them leave the
+    chip idle while the copy and the row quantizer fill it (us, copy / in place,
+    bf16: G=1 N=64 K=8192 7.9 / 68, G=2 N=512 K=2048 16.6 / 19.9, G=4 N=512
+    K=2048 26.0 / 20.3; 16 workgroups K=512 8.3 / 7.1).  Rows that are no whole
+    aligned runs of 8 are read element by element, three times slower (G=8 N=300
+    K=2048 30 / 60, G=8 N=1001 K=2048 82 / 62, G=16 N=333 K=2048 56 / 63, fp32
+    87 / 74)."""
+    groups = G * (-(-R // 64))
+    per = 16 // esize
+    if R % 8 == 0 and stride_col % per == 0 and stride_batch % per == 0 and ptr % 16 == 0:
+        return groups >= (16 if C <= 1024 else 32)
+    return groups >= (72 if esize == 4 else 112)
+
+
 def quant_fp8_rows_batched(w: torch.Tensor):
     """One E4M3 scale per row of ``w [G, N, K]``: ``(q uint8 [G*N, K], scales
     float32 [G*N, 1])``, what ``quant_fp8_blocks(w.reshape(G * N, K), 1, K)``
@@ -81,7 +97,8 @@ def quant_fp8_rows_batched(w: torch.Tensor):
     in place instead of being copied to K-major rows first."""
     G, R, C = w.shape
     if not (w.device.type == "cuda" and w.dtype in (torch.bfloat16, torch.float32) and w.numel() > 0
-            and R > 1 and C > 1 and w.stride(1) == 1 and w.stride(2) >= R and w.stride(0) > 0 and G <= 65535):
+            and 1 < R < 1 << 29 and C > 1 and w.stride(1) == 1 and w.stride(2) >= R and w.stride(0) > 0
+            and G <= 65535 and _rows_in_place(G, R, C, w.element_size(), w.stride(0), w.stride(2), w.data_ptr())):
         return quant_fp8_blocks(w.reshape(G * R, C), 1, C)
     r = N.fast().quant_fp8_rows_batched(w)
     if r is not None:

@@ -100,7 +100,9 @@ int dsl_quant_fp8_blocks(const void *x, int64_t rows, int64_t cols,
  * of unit row stride (the reference's grouped B[G][K][N] read as [G][N][K],
  * triton/gemm/gemm_kernels.py:164-182): matrix b is x[b*stride_batch + r +
  * c*stride_col], stride_col >= rows.  q [batch*rows][cols], scales
- * [batch*rows].  batch <= 65535. */
+ * [batch*rows].  batch <= 65535, rows < 2^29.  One workgroup walks the columns
+ * of 64 rows of a matrix: with few of them a copy to rows and
+ * dsl_quant_fp8_blocks are faster (dsl_tool_amd/quant.py chooses so). */
 int dsl_quant_fp8_rows_batched(const void *x, int64_t batch, int64_t rows, int64_t cols,
                                int64_t stride_batch, int64_t stride_col, int x_dtype,
                                uint8_t *q, float *scales, void *stream);

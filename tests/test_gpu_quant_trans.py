@@ -80,3 +80,31 @@ def test_batched_rows_match_oracle(g, n, k, dt, pad):
     q_ref, s_ref = OQ.quant_fp8_blockwise(w.transpose(1, 2).reshape(g * n, k).float().numpy(), 1, k)
     assert np.array_equal(np_f32(s), s_ref)
     assert np.array_equal(np_u8(q), q_ref)
+
+
+@pytest.mark.parametrize("r,c,gr,gc", [
+    (1024, 384, 1, 384), (1536, 384, 1, 384), (1016, 384, 1, 384), (3072, 272, 1, 272), (3071, 272, 1, 272),
+    (64, 8192, 1, 512), (64, 8704, 1, 512), (15, 8192, 1, 512), (7, 384, 128, 128), (8, 384, 128, 128)])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_both_sides_of_the_occupancy_rule(r, c, gr, gc, dt):
+    """Few long scale groups take the strided kernel, many the transposed one."""
+    x, ref = _source(r, c, dt, 0, 0)
+    q, s = Q.quant_fp8_blocks(x, gr, gc)
+    q_ref, s_ref = OQ.quant_fp8_blockwise(ref, gr, gc)
+    assert np.array_equal(np_f32(s), s_ref) and np.array_equal(np_u8(q), q_ref)
+
+
+@pytest.mark.parametrize("r,c", [(333, 2048), (1500, 1024), (513, 1024), (4100, 512), (4616, 512)])
+def test_nvfp4_of_odd_fp32_sources(r, c):
+    x, ref = _source(r, c, torch.float32, 1, 1)
+    q, s, sg = Q.quant_nvfp4(x)
+    q_ref, s_ref, sg_ref = OQ.quant_nvfp4(ref)
+    assert np_f32(sg)[0] == sg_ref
+    assert np.array_equal(np_u8(s), s_ref) and np.array_equal(np_u8(q), q_ref)
+
+
+@pytest.mark.parametrize("g,n,k", [(1, 64, 1040), (2, 512, 400), (4, 512, 144), (16, 64, 400), (32, 40, 144),
+                                   (9, 1001, 80), (3, 72, 400)])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_grouped_weights_in_place_or_copied(g, n, k, dt):
+    test_batched_rows_match_oracle(g, n, k, dt, 0)

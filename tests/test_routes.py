@@ -31,3 +31,48 @@ def test_routes_of_the_common_calls():
     assert route("block", 1500, 22016, 4096) == "persist 256x256 + pipe 64x128 deep"
     assert route("block", 1500, 4096, 11008) == "persist 256x128"
     assert route("bf16", 512, 4096, 4096, F32) == "pipe 64x128 deep"
+
+
+def transposed(rows, cols, gr, gc, f32=False, ptr=1 << 20):
+    f = N.lib().dsl_test_quant_transposed
+    f.restype, f.argtypes = ctypes.c_int, [ctypes.c_void_p, ctypes.c_int] + [ctypes.c_int64] * 6
+    return bool(f(ptr, N.IN_F32 if f32 else N.IN_BF16, rows, cols, 1, rows, gr, gc))
+
+
+@pytest.mark.parametrize("rows,cols,gr,gc,f32,want", [
+    # one scale per row: us of the strided / the transposed kernel
+    (64, 8192, 1, 8192, False, False),      # 22.9 / 68.0
+    (512, 2048, 1, 2048, True, False),      # 13.3 / 27.9
+    (1280, 2048, 1, 2048, False, True),     # 28.6 / 20.0
+    (1024, 512, 1, 512, True, False),       # 7.1 / 9.3
+    (1536, 2048, 1, 2048, True, True),      # 45.0 / 28.3
+    (1500, 2048, 1, 2048, False, False),    # 31.5 / 60.7: rows of no whole runs of 8
+    (4100, 512, 1, 512, False, True),       # 20.7 / 16.2
+    (64, 2048, 1, 512, False, False),       # 4.8 / 7.1
+    (64, 28672, 1, 512, False, True),       # 17.1 / 7.4
+    (2, 1 << 20, 1, 512, False, False),     # 13.8 / 41.4
+    (4, 512, 128, 128, True, False),        # 3.7 / 4.6
+    (8, 512, 128, 128, True, True),         # 5.1 / 4.4
+    (4, 512, 1, 128, False, True),          # 46 / 3.7
+    (4, 512, 1, 256, False, True),
+    ((1 << 29) + 8, 2, 1, 2, False, False)])   # past the grid's threads
+def test_transposed_quantizer_needs_enough_scales(rows, cols, gr, gc, f32, want):
+    assert transposed(rows, cols, gr, gc, f32) == want
+
+
+@pytest.mark.parametrize("g,rows,cols,esize,want", [
+    (1, 64, 8192, 2, False),      # copy and row quantizer 7.9 us, in place 68.3
+    (2, 512, 2048, 2, False),     # 16.6 / 19.9
+    (4, 512, 2048, 2, True),      # 26.0 / 20.3
+    (16, 64, 512, 2, True),       # 8.3 / 7.1
+    (16, 64, 8192, 2, False),     # 45.1 / 69.3
+    (8, 300, 2048, 2, False),     # 30.1 / 60.2: rows of no whole runs of 8
+    (8, 1001, 2048, 2, True),     # 81.8 / 62.2
+    (16, 333, 2048, 4, True),     # 86.6 / 73.8
+    (16, 333, 2048, 2, False)])   # 56.4 / 62.8
+def test_grouped_weights_are_read_in_place_where_that_fills_the_chip(g, rows, cols, esize, want):
+    from dsl_tool_amd import quant as Q
+    assert Q._rows_in_place(g, rows, cols, esize, rows * cols, rows, 1 << 20) == want
+    if rows % 8 == 0:             # a pointer or pitch off the 16-byte grid is read element by element
+        assert not Q._rows_in_place(4, 512, cols, esize, rows * cols, rows, (1 << 20) + 2)
+        assert not Q._rows_in_place(4, 512, cols, esize, 512 * cols, 513, 1 << 20)
