@@ -618,14 +618,12 @@ struct StreamPlan {
 
 // K whose rows (or scale rows) take the TAIL form of the kernel: rows of no
 // whole 256-byte chunks, FP8 / MXFP4 scale rows of no whole 16 bytes (K %
-// 512), NVFP4 ones (K % 256), or scale arrays that are not 16-byte aligned;
-// and, from 129 rows, long rows of an odd number of 256-byte chunks, for its
-// 64-row blocks (bf16 M=256 N=4096 K=4224: 22 us, on the 128x128 tiles 37;
-// M=128: 18.2 against 15.9 in 32-row blocks; the K=128 LoRA add at M=512 N=4096
-// is 4 us faster in 32-row blocks).
-bool needs_tail(int mode, int M, int K, int Kb, bool scales16) {
-  return !stream_whole(mode, K, Kb, scales16) || (Kb % 512 != 0 && M > 128 && Kb >= 1024);
-}
+// 512), NVFP4 ones (K % 256), or scale arrays that are not 16-byte aligned.
+// Whole rows of an odd number of 256-byte chunks keep the plain form in 32-row
+// blocks: the TAIL form, whose 64-row blocks they could take, was slower at 33
+// of 38 sampled sizes of 129 rows or more (bf16 180x1248x1664 7.8 against 5.3
+// us, NVFP4 235x1040x7680 25.1 against 16.5).
+bool needs_tail(int mode, int K, int Kb, bool scales16) { return !stream_whole(mode, K, Kb, scales16); }
 
 bool stream_rows64(int M, int Kb, bool tail) { return tail ? M > 96 : Kb % 512 == 0; }
 
@@ -703,7 +701,7 @@ hipError_t launch_tn(const GemmArgs &p, int tn, hipStream_t st) {
 template <int MODE>
 hipError_t launch_mode(const GemmArgs &p, const StreamPlan &pl, hipStream_t st) {
   const uintptr_t sc = reinterpret_cast<uintptr_t>(p.sa) | reinterpret_cast<uintptr_t>(p.sb);
-  if (needs_tail(MODE, p.M, p.K, p.Kb, (sc & 15) == 0)) {
+  if (needs_tail(MODE, p.K, p.Kb, (sc & 15) == 0)) {
     if (pl.tma == 1) return launch_tn<MODE, 1, 256, true>(p, pl.tn, st);
     if (pl.tma == 2) return launch_tn<MODE, 2, 256, true>(p, pl.tn, st);
     return launch_tn<MODE, 4, 256, true>(p, pl.tn, st);
@@ -760,11 +758,11 @@ bool stream_supported(int mode, int M, int N, int K, int Kb, bool scales4) {
 }
 
 bool stream_blocks64(int mode, int M, int K, int Kb, bool scales16) {
-  return stream_rows64(M, Kb, needs_tail(mode, M, K, Kb, scales16));
+  return stream_rows64(M, Kb, needs_tail(mode, K, Kb, scales16));
 }
 
 bool stream_plan(int mode, int M, int N, int K, int Kb, bool scales16, int *tma, int *tn) {
-  const bool tail = needs_tail(mode, M, K, Kb, scales16);
+  const bool tail = needs_tail(mode, K, Kb, scales16);
   const StreamPlan pl = plan_for(mode, M, N, Kb, tail);
   *tma = pl.tma;
   *tn = pl.tn;
@@ -776,7 +774,7 @@ hipError_t launch_gemm_stream(int mode, const GemmArgs &p, hipStream_t st) {
     return hipErrorInvalidValue;
   if (p.accumulate && (!p.out_f32 || p.lora_scales)) return hipErrorInvalidValue;
   const uintptr_t sc = reinterpret_cast<uintptr_t>(p.sa) | reinterpret_cast<uintptr_t>(p.sb);
-  const StreamPlan pl = plan_for(mode, p.M, p.N, p.Kb, needs_tail(mode, p.M, p.K, p.Kb, (sc & 15) == 0));
+  const StreamPlan pl = plan_for(mode, p.M, p.N, p.Kb, needs_tail(mode, p.K, p.Kb, (sc & 15) == 0));
   switch (mode) {
     case MODE_FP8_TENSOR: return launch_mode<MODE_FP8_TENSOR>(p, pl, st);
     case MODE_FP8_BLOCK: return launch_mode<MODE_FP8_BLOCK>(p, pl, st);

@@ -33,6 +33,16 @@ def test_routes_of_the_common_calls():
     assert route("bf16", 512, 4096, 4096, F32) == "pipe 64x128 deep"
 
 
+@pytest.mark.parametrize("mode,m,n,k", [
+    ("bf16", 180, 1248, 1664),      # 5.3 / 7.8
+    ("tensor", 150, 1368, 1280),    # 3.8 / 5.5
+    ("nvfp4", 235, 1040, 7680),     # 16.5 / 25.1
+    ("nvfp4", 376, 3156, 12800),    # 89 / 113
+    ("mxfp4", 133, 2392, 2560)])    # 5.1 / 7.1
+def test_odd_chunk_rows_keep_the_plain_streaming_form(mode, m, n, k):
+    assert route(mode, m, n, k).startswith("stream 32x")
+
+
 def transposed(rows, cols, gr, gc, f32=False, ptr=1 << 20):
     f = N.lib().dsl_test_quant_transposed
     f.restype, f.argtypes = ctypes.c_int, [ctypes.c_void_p, ctypes.c_int] + [ctypes.c_int64] * 6
