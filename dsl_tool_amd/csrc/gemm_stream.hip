@@ -627,6 +627,20 @@ bool needs_tail(int mode, int K, int Kb, bool scales16) { return !stream_whole(m
 
 bool stream_rows64(int M, int Kb, bool tail) { return tail ? M > 96 : Kb % 512 == 0; }
 
+// Whether the workgroups of bm-row blocks and one W tile run in one round.
+// Workgroups go to the eight XCDs by W slice (gemm_stream_kernel), so with a
+// long K the XCD with the most slices has to hold all their row blocks: 9 slices
+// of 26 blocks are 234 workgroups, but 52 of them share one XCD's 32 CUs (bf16
+// 812x136x11008 in 32-row blocks 38.8 us, in 64-row ones 30.1; MXFP4
+// 698x168x19712, 44 on one XCD, 24.0 against 21.3).  Short chains are latency,
+// and two on a CU overlap (NVFP4 544x144x1024, 34 on one XCD: 4.1 us in 32-row
+// blocks, 7.9 in 64-row ones).
+bool one_round(int M, int N, int bm, int Kb) {
+  const int64_t blocks = (M + bm - 1) / bm, slices = (N + 15) / 16;
+  return blocks * slices <= device_cu_count() &&
+         (Kb <= 6144 || blocks * ((slices + 7) / 8) <= device_cu_count() / 8);
+}
+
 // Activation tiles by M (16, 32 or 64 rows per workgroup; 256-byte chunks
 // for the skinny ones, 512-byte chunks otherwise; whole rows of an odd number
 // of 256-byte chunks take the 32-row tiles), and the most W tiles
@@ -645,7 +659,7 @@ StreamPlan plan_for(int mode, int M, int N, int Kb, bool tail) {
   // -> 6.7, M=100 9.7 -> 5.8, M=200 9.2 -> 7.8; block M=64 6.8 -> 4.8; N=1024
   // bf16 M=64 10.0 -> 6.7, N=2048 10.5 -> 8.8)
   for (int t = 1; t < pl.tma; t *= 2)
-    if ((int64_t)((M + 16 * t - 1) / (16 * t)) * ((N + 15) / 16) <= device_cu_count()) {
+    if (one_round(M, N, 16 * t, Kb)) {
       pl.tma = t;
       break;
     }

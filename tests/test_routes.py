@@ -43,6 +43,17 @@ def test_odd_chunk_rows_keep_the_plain_streaming_form(mode, m, n, k):
     assert route(mode, m, n, k).startswith("stream 32x")
 
 
+@pytest.mark.parametrize("mode,m,n,k,bm", [
+    ("bf16", 812, 136, 11008, 64),     # 30.1 / 38.8
+    ("tensor", 384, 296, 24576, 64),   # 27.1 / 36.0
+    ("block", 357, 280, 18432, 64),    # 24.3 / 33.4
+    ("nvfp4", 544, 144, 1024, 32),     # 4.1 / 7.9: short chains overlap on a CU
+    ("mxfp4", 41, 2592, 8192, 64),     # 6.9 / 9.1: three times the workgroups of one round
+    ("bf16", 64, 512, 4096, 16)])      # 6.7 / 8.4
+def test_streaming_row_blocks_of_one_round(mode, m, n, k, bm):
+    assert route(mode, m, n, k).startswith(f"stream {bm}x")
+
+
 def transposed(rows, cols, gr, gc, f32=False, ptr=1 << 20):
     f = N.lib().dsl_test_quant_transposed
     f.restype, f.argtypes = ctypes.c_int, [ctypes.c_void_p, ctypes.c_int] + [ctypes.c_int64] * 6
