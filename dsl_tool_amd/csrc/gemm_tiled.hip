@@ -264,6 +264,14 @@ static int pipe_switch() {
   return forced;
 }
 
+// The deep rings (variants 6, 7) advance the prefetching modes by pairs of
+// 128-byte stages: an odd or partial last pair takes the ragged form, whose padding
+// stage costs as much as a whole one.  Short K pays for it, and for filling the
+// ring, against variant 1: per-tensor 724x3200x640 8.2 us / 6.3, 410x7680x1664
+// 12.1 / 10.3, level from about 2560; whole pairs to K=1536 6.5 / 6.0.
+static bool prefetches(int mode) { return mode == MODE_FP8_TENSOR || mode == MODE_BF16; }
+static bool deep_pays(int mode, int Kb) { return !prefetches(mode) || Kb >= (Kb % 256 == 0 ? 1536 : 2560); }
+
 // `padded`: a workspace for padded scale rows is there.  `ragged` false: the
 // kernel that serves the shape without the ragged forms and the one-round tiles
 // (rows and scale rows of whole steps only); the workspace contract is that
@@ -361,10 +369,12 @@ static Route pick_route(int mode, int M, int N, int K, int Kb, bool sc4, bool sc
     r.path = PATH_STREAM;
     return r;
   }
-  const int one_round = ragged && mode != MODE_NVFP4 && t128 <= device_cu_count() && pipe_forced < 0 ? 7 : 1;
+  const int one_round = ragged && mode != MODE_NVFP4 && t128 <= device_cu_count() && pipe_forced < 0 &&
+                                deep_pays(mode, Kb) ? 7 : 1;
   if (small) {
     r.path = PATH_PIPE;
-    r.variant = 6;
+    // (an odd pair count at short K: 7.0 us, 6.4 in variant 1, per-tensor K=896)
+    r.variant = prefetches(mode) && Kb % 256 == 128 && Kb < 1536 && t128 >= 40 ? 1 : 6;
     r.pad_scales = mode == MODE_MXFP4 && Kb % 128 != 0;
     return r;
   }
@@ -517,11 +527,11 @@ static int strip_columns(const GemmArgs &p) {
 
 // Pipelined tiles for those columns: 64x128 or deep 128x128 ones where one round
 // holds them, as pick_route has it.
-static int pipe_variant(int mode, int M, int N) {
+static int pipe_variant(int mode, int M, int N, int Kb) {
   const int64_t cu = device_cu_count();
   if (mode == MODE_NVFP4) return 1;
   if ((int64_t)((M + 63) / 64) * ((N + 127) / 128) <= cu) return 6;
-  return (int64_t)((M + 127) / 128) * ((N + 127) / 128) <= cu ? 7 : 1;
+  return (int64_t)((M + 127) / 128) * ((N + 127) / 128) <= cu && deep_pays(mode, Kb) ? 7 : 1;
 }
 
 void describe_gemm(int mode, int64_t M, int64_t N, int64_t K, bool, char *buf, size_t len) {
@@ -553,7 +563,7 @@ void describe_gemm(int mode, int64_t M, int64_t N, int64_t K, bool, char *buf, s
   Route rest = route_for(mode, (int)M, strip, (int)K, Kb, true, true, false);
   if (rest.path != PATH_STREAM) {
     rest.path = PATH_PIPE;
-    rest.variant = pipe_variant(mode, (int)M, strip);
+    rest.variant = pipe_variant(mode, (int)M, strip, Kb);
   }
   const size_t used = strlen(buf);
   snprintf(buf + used, len - used, " + ");
@@ -627,7 +637,7 @@ hipError_t launch_gemm(int mode, GemmArgs p, hipStream_t st) {
       return route_for(mode, rest.M, rest.N, rest.K, rest.Kb, (sc & 3) == 0, (sc & 15) == 0, false).path ==
                      PATH_STREAM
                  ? launch_gemm_stream(mode, rest, st)
-                 : launch_gemm_pipe(mode, rest, pipe_variant(mode, rest.M, rest.N), st);
+                 : launch_gemm_pipe(mode, rest, pipe_variant(mode, rest.M, rest.N, rest.Kb), st);
     }
     return launch_gemm_persist(mode, p, st, r.narrow);
   }

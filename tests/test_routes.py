@@ -54,6 +54,19 @@ def test_streaming_row_blocks_of_one_round(mode, m, n, k, bm):
     assert route(mode, m, n, k).startswith(f"stream {bm}x")
 
 
+@pytest.mark.parametrize("mode,m,n,k,want", [
+    ("tensor", 724, 3200, 640, "pipe 128x128"),         # 6.3 / 8.2
+    ("tensor", 410, 7680, 1664, "pipe 128x128"),        # 10.3 / 12.1
+    ("bf16", 424, 5368, 320, "pipe 128x128"),           # 6.3 / 8.2
+    ("tensor", 350, 6232, 512, "pipe 128x128"),         # 5.9 / 6.4
+    ("tensor", 395, 3400, 896, "pipe 128x128"),         # 6.6 / 7.1
+    ("tensor", 724, 3200, 4096, "pipe 128x128 deep"),   # 19.9 / 22.9
+    ("tensor", 395, 3400, 1664, "pipe 64x128 deep"),
+    ("block", 724, 3200, 640, "pipe 128x128 deep")])    # group-scaled forms gain at any K
+def test_deep_rings_need_a_long_k(mode, m, n, k, want):
+    assert route(mode, m, n, k) == want
+
+
 def transposed(rows, cols, gr, gc, f32=False, ptr=1 << 20):
     f = N.lib().dsl_test_quant_transposed
     f.restype, f.argtypes = ctypes.c_int, [ctypes.c_void_p, ctypes.c_int] + [ctypes.c_int64] * 6
