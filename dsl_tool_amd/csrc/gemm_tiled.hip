@@ -276,7 +276,7 @@ static bool deep_pays(int mode, int Kb) { return !prefetches(mode) || Kb >= (Kb 
 // kernel that serves the shape without the ragged forms and the one-round tiles
 // (rows and scale rows of whole steps only); the workspace contract is that
 // route's.
-static Route pick_route(int mode, int M, int N, int K, int Kb, bool sc4, bool sc16, bool padded,
+static Route pick_route(int mode, int M, int N, int K, int Kb, bool sc4, bool sc16, bool padded, bool f32,
                         bool ragged) {
   static const bool decode_on = !env_off("DSL_GEMM_DECODE");
   const bool stream_on = stream_enabled();
@@ -391,6 +391,17 @@ static Route pick_route(int mode, int M, int N, int K, int Kb, bool sc4, bool sc
   const bool narrow = ragged && persist_on && pipe_forced < 0 && M > 128 && N > 128 && tn <= cu &&
                       (mode == MODE_NVFP4 ? 10 * t128 > 6 * cu : t128 > cu) &&
                       persist_supported(mode, M, N, K, Kb, sc4);
+  // The persistent kernel's last column of tiles stores element by element where
+  // its columns do not all exist (every tile where N % 8 != 0): up to 11 us per
+  // 128 columns of it.  Against variant 1 the 256x128 tiles gain this much per
+  // 1024 bytes of K, so short ragged problems stay there: per-tensor
+  // 583x9952x512 18.5 us / 11.0, block 6720x752x1024 25.3 / 13.5.  (fp32
+  // results: variant 1 stores those element by element too.)
+  static constexpr float narrow_gain[] = {2.0f, 1.2f, 7.2f, 38.f, 2.0f, 0.f};   // by mode; NVFP4: two rounds
+  auto last_tile = [&](int bn) { return N % 8 ? 1.f : (float)(N % bn) / bn; };
+  const float gain = (mode == MODE_NVFP4 && t128 <= cu ? 8.f : narrow_gain[mode]) * Kb / 1024 -
+                     (mode == MODE_MXFP4 ? 2.f : (mode == MODE_NVFP4 ? 1.f : 0.f));
+  const bool narrow_wins = f32 || Kb % 128 != 0 || gain >= 11 * last_tile(128);
   if (mode == MODE_BF16) {   // pipelined, persistent or register-staged tiles
     const int64_t t256 = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
     // one round of 128x128 pipelined tiles (40 to one per CU) beats a
@@ -447,13 +458,21 @@ static Route pick_route(int mode, int M, int N, int K, int Kb, bool sc4, bool sc
     if (persist_wins) {
       r.path = PATH_PIPE;
       r.variant = pipe_forced >= 0 ? pipe_forced : (t256 >= 240 ? 0 : one_round);
-      if (persist_ok) r.path = PATH_PERSIST;
+      // Rows of whole 128 bytes whose scale rows are no whole quads: the tiles
+      // above serve them too, and win on short K (the scales' copy, and up to 24
+      // us for a last column of tiles that is nearly full; block 6569x1520x768
+      // 43.5 us / 16.9, MXFP4 1319x8624x768 33.4 / 15.4; whole columns: block
+      // 4128x7680x768 36.1 / 38.1, MXFP4 7231x4608x1280 45.7 / 50.9).
+      const bool short_k = !f32 && !rag && !persist_whole(mode, K, Kb, sc16) &&
+                           Kb < (mode == MODE_FP8_BLOCK ? 1024 + 6144 * last_tile(256)
+                                                        : 512 + 2560 * last_tile(256));
+      if (persist_ok && !short_k) r.path = PATH_PERSIST;
     } else if (M > 64 && N > 64 && t128 >= 40) {
       r.path = PATH_PIPE;
       r.variant = one_round;
     }
   }
-  if (narrow && persist_ok) {
+  if (narrow && persist_ok && (r.path == PATH_PERSIST || narrow_wins)) {
     r.path = PATH_PERSIST;
     r.narrow = true;
   }
@@ -461,14 +480,14 @@ static Route pick_route(int mode, int M, int N, int K, int Kb, bool sc4, bool sc
   return r;
 }
 
-static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc16, bool padded) {
-  return pick_route(mode, M, N, K, Kb, sc4, sc16, padded, true);
+static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc16, bool padded, bool f32) {
+  return pick_route(mode, M, N, K, Kb, sc4, sc16, padded, f32, true);
 }
 
 bool gemm_routes_to_stream(int mode, int64_t M, int64_t N, int64_t K, bool or_pipe, bool accumulate) {
   const int Kb = (mode == MODE_MXFP4 || mode == MODE_NVFP4) ? (int)(K / 2)
                                                             : (mode == MODE_BF16 ? (int)(2 * K) : (int)K);
-  int path = route_for(mode, (int)M, (int)N, (int)K, Kb, true, true, true).path;
+  int path = route_for(mode, (int)M, (int)N, (int)K, Kb, true, true, true, true).path;
   if (accumulate && K <= kAccShortK && stream_enabled() && stream_supported(mode, (int)M, (int)N, (int)K, Kb, true))
     path = PATH_STREAM;   // as launch_gemm routes C += result
   return path == PATH_STREAM || (or_pipe && path == PATH_PIPE && (!accumulate || !mode_grouped_k(mode)));
@@ -477,7 +496,7 @@ bool gemm_routes_to_stream(int mode, int64_t M, int64_t N, int64_t K, bool or_pi
 size_t gemm_workspace_required(int mode, int64_t M, int64_t N, int64_t K, bool accumulate) {
   const int Kb = (mode == MODE_MXFP4 || mode == MODE_NVFP4) ? (int)(K / 2)
                                                             : (mode == MODE_BF16 ? (int)(2 * K) : (int)K);
-  Route r = pick_route(mode, (int)M, (int)N, (int)K, Kb, true, true, false, false);
+  Route r = pick_route(mode, (int)M, (int)N, (int)K, Kb, true, true, false, true, false);
   if (accumulate) r.path = PATH_TILED;
   return (r.path == PATH_TILED && r.tiled.ksplit > 1)
              ? (size_t)r.tiled.ksplit * (size_t)splitk_slice(M, N) * sizeof(float)
@@ -487,7 +506,7 @@ size_t gemm_workspace_required(int mode, int64_t M, int64_t N, int64_t K, bool a
 size_t gemm_workspace_bytes(int mode, int64_t M, int64_t N, int64_t K, bool accumulate) {
   const size_t need = gemm_workspace_required(mode, M, N, K, accumulate);
   if (accumulate || (mode != MODE_MXFP4 && mode != MODE_NVFP4)) return need;
-  const Route r = route_for(mode, (int)M, (int)N, (int)K, (int)(K / 2), true, true, true);
+  const Route r = route_for(mode, (int)M, (int)N, (int)K, (int)(K / 2), true, true, true, true);
   return r.pad_scales ? std::max(need, (size_t)(M + N) * (size_t)padded_pitch(mode, (int)K)) : need;
 }
 
@@ -534,7 +553,7 @@ static int pipe_variant(int mode, int M, int N, int Kb) {
   return (int64_t)((M + 127) / 128) * ((N + 127) / 128) <= cu && deep_pays(mode, Kb) ? 7 : 1;
 }
 
-void describe_gemm(int mode, int64_t M, int64_t N, int64_t K, bool, char *buf, size_t len) {
+void describe_gemm(int mode, int64_t M, int64_t N, int64_t K, bool f32, char *buf, size_t len) {
   const int Kb = (mode == MODE_MXFP4 || mode == MODE_NVFP4) ? (int)(K / 2)
                                                             : (mode == MODE_BF16 ? (int)(2 * K) : (int)K);
   auto name = [&](const Route &r, int m, int n, char *to, size_t room) {
@@ -553,14 +572,14 @@ void describe_gemm(int mode, int64_t M, int64_t N, int64_t K, bool, char *buf, s
       snprintf(to, room, "decode");
     }
   };
-  Route r = route_for(mode, (int)M, (int)N, (int)K, Kb, true, true, true);
+  Route r = route_for(mode, (int)M, (int)N, (int)K, Kb, true, true, true, f32);
   name(r, (int)M, (int)N, buf, len);
   GemmArgs p{};
   p.M = (int)M;
   p.N = (int)N;
   const int strip = r.path != PATH_PERSIST || r.narrow || r.pad_scales ? 0 : strip_columns(p);
   if (strip == 0) return;
-  Route rest = route_for(mode, (int)M, strip, (int)K, Kb, true, true, false);
+  Route rest = route_for(mode, (int)M, strip, (int)K, Kb, true, true, false, f32);
   if (rest.path != PATH_STREAM) {
     rest.path = PATH_PIPE;
     rest.variant = pipe_variant(mode, (int)M, strip, Kb);
@@ -588,7 +607,7 @@ hipError_t launch_gemm(int mode, GemmArgs p, hipStream_t st) {
   const bool padded = (mode == MODE_MXFP4 || mode == MODE_NVFP4) && p.ws &&
                       (reinterpret_cast<uintptr_t>(p.ws) & 15) == 0 &&
                       p.ws_bytes >= (size_t)((int64_t)p.M + p.N) * (size_t)padded_pitch(mode, p.K);
-  Route r = route_for(mode, p.M, p.N, p.K, p.Kb, (sc & 3) == 0, (sc & 15) == 0, padded);
+  Route r = route_for(mode, p.M, p.N, p.K, p.Kb, (sc & 3) == 0, (sc & 15) == 0, padded, p.out_f32 != 0);
   if (p.lora_scales) {   // the LoRA epilogue: the streaming kernel only
     if (mode != MODE_BF16 || !stream_supported(mode, p.M, p.N, p.K, p.Kb, true) || p.accumulate)
       return hipErrorInvalidValue;
@@ -634,7 +653,7 @@ hipError_t launch_gemm(int mode, GemmArgs p, hipStream_t st) {
       const hipError_t e = launch_gemm_persist(mode, main, st, false);
       if (e != hipSuccess) return e;
       const GemmArgs rest = columns_from(mode, p, main.N);
-      return route_for(mode, rest.M, rest.N, rest.K, rest.Kb, (sc & 3) == 0, (sc & 15) == 0, false).path ==
+      return route_for(mode, rest.M, rest.N, rest.K, rest.Kb, (sc & 3) == 0, (sc & 15) == 0, false, p.out_f32 != 0).path ==
                      PATH_STREAM
                  ? launch_gemm_stream(mode, rest, st)
                  : launch_gemm_pipe(mode, rest, pipe_variant(mode, rest.M, rest.N, rest.Kb), st);

@@ -67,6 +67,29 @@ def test_deep_rings_need_a_long_k(mode, m, n, k, want):
     assert route(mode, m, n, k) == want
 
 
+@pytest.mark.parametrize("mode,m,n,k,want", [
+    # a partial last column of tiles stores element by element
+    ("tensor", 583, 9952, 512, "pipe 128x128"),        # 11.0 / 18.5
+    ("block", 6720, 752, 1024, "pipe 128x128"),        # 13.5 / 25.3
+    ("block", 528, 7016, 512, "pipe 128x128"),         # 9.1 / 17.0
+    ("nvfp4", 716, 4432, 512, "pipe 128x128"),         # 12.8 / 19.6
+    ("tensor", 691, 5632, 768, "persist 256x128"),     # 9.3 / 11.8: whole columns
+    ("tensor", 2048, 4000, 11008, "persist 256x128"),  # ragged, long K
+    ("nvfp4", 1024, 5000, 4096, "persist 256x128"),
+    # scale rows that are no whole quads, rows of whole 128 bytes
+    ("block", 6569, 1520, 768, "pipe 128x128"),        # 16.9 / 43.5
+    ("block", 7493, 2784, 640, "pipe 256x256"),        # 28.1 / 50.5
+    ("mxfp4", 1319, 8624, 768, "pipe 128x128"),        # 15.4 / 33.4
+    ("mxfp4", 1124, 13624, 256, "pipe 256x256"),       # 15.4 / 22.1
+    ("block", 4128, 7680, 768, "pipe 256x256"),        # 38.1 / 36.1: the line is at 1024
+    ("block", 6027, 3072, 1792, "persist 256x256 + pipe 128x128 deep"),    # 46.4 / 58.0
+    ("mxfp4", 6956, 1792, 2304, "persist 256x256")])   # 27.1 / 39.7
+def test_persistent_tiles_need_whole_columns_or_a_long_k(mode, m, n, k, want):
+    assert route(mode, m, n, k) == want
+    if want.startswith("pipe"):      # fp32 results: those tiles store element by element too
+        assert route(mode, m, n, k, F32).startswith("persist")
+
+
 def transposed(rows, cols, gr, gc, f32=False, ptr=1 << 20):
     f = N.lib().dsl_test_quant_transposed
     f.restype, f.argtypes = ctypes.c_int, [ctypes.c_void_p, ctypes.c_int] + [ctypes.c_int64] * 6
