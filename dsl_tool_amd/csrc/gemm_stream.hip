@@ -57,6 +57,7 @@
 // before -> now: M=16 block 12.2 -> 6.6, MXFP4 13.4 -> 5.2, NVFP4 26.2 -> 7.5,
 // per-tensor 11.4 -> 6.1; M=1 per-tensor 10.3 -> 5.5 (K=4160: 10.1 -> 5.8);
 // M=256 MXFP4 76.3 -> 12.4.
+#include <algorithm>
 #include <cstdlib>
 
 #include "stream_core.h"
@@ -781,6 +782,26 @@ bool stream_plan(int mode, int M, int N, int K, int Kb, bool scales16, int *tma,
   *tma = pl.tma;
   *tn = pl.tn;
   return tail;
+}
+
+// Predicted time of the kernel in us, for the router's choice between it and
+// another kernel.  A wave's chunks are a serial chain of items (16 rows of W or
+// A x 256 bytes), `item` us each by mode and form; past one workgroup per CU on
+// the XCD that holds the most (see one_round) the chain and a fixed part repeat;
+// W crosses HBM once per row block, A once per XCD.  Fitted to 6982 ragged and
+// 2871 whole sizes (M to 1024, K to 32768): 5% of the ragged ones are above it
+// by more than 1.3, 5% below it by more than 1.13.
+float stream_estimate(int mode, int M, int N, int K, int Kb, bool scales16) {
+  static constexpr float item[6][2] = {   // plain, TAIL
+      {.20f, .25f}, {.25f, .325f}, {.27f, .36f}, {.55f, .70f}, {.20f, .25f}, {.25f, .325f}};
+  const bool tail = needs_tail(mode, K, Kb, scales16);
+  const StreamPlan pl = plan_for(mode, M, N, Kb, tail);
+  const int chunk = !tail && pl.tma == 4 ? 512 : 256;
+  const int nmb = (M + 16 * pl.tma - 1) / (16 * pl.tma), nnb = (N + 16 * pl.tn - 1) / (16 * pl.tn);
+  const float chain = (float)((Kb + 4 * chunk - 1) / (4 * chunk) * (chunk / 256) * (pl.tma + pl.tn)) * item[mode][tail];
+  const float more = std::max(0.f, (float)nmb * ((nnb + 7) / 8) / (device_cu_count() / 8) - 1);
+  return 2.2f + chain + more * (1.2f + 1.15f * chain) + .06e-6f * N * (float)Kb * nmb +
+         .035e-6f * M * (float)Kb * std::min(nnb, 8);
 }
 
 hipError_t launch_gemm_stream(int mode, const GemmArgs &p, hipStream_t st) {

@@ -1,6 +1,7 @@
 // Dense quantized GEMM: C[M,N] = A[M,K] . W[N,K]^T on gfx950 MFMA.
 // Variant selection (tile shape, split-K) lives in launch_gemm below.
 #include <algorithm>
+#include <cstdint>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -480,14 +481,76 @@ static Route pick_route(int mode, int M, int N, int K, int Kb, bool sc4, bool sc
   return r;
 }
 
-static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc16, bool padded, bool f32) {
-  return pick_route(mode, M, N, K, Kb, sc4, sc16, padded, f32, true);
+// Predicted times in us of the pipelined tiles (one stage of 128 bytes by mode
+// and form; `fill` workgroups per CU, two of variant 1 share one) and of the
+// register-staged tiles split over K (64-byte steps of the longest split, the
+// partial sums written and read, the operands).  Fitted to 10800 sampled sizes,
+// M to 8192 and K to 32768: 4 in 5 within 15%.
+static float pipe_estimate(int mode, const Route &r, int M, int N, int Kb) {
+  static constexpr float deep64[6][2] = {   // whole, ragged
+      {.23f, .36f}, {.42f, .49f}, {.52f, .65f}, {0, 0}, {.25f, .40f}, {.43f, .55f}};
+  static constexpr float deep128[6][2] = {
+      {.40f, .50f}, {.66f, .80f}, {.85f, .98f}, {0, 0}, {.43f, .55f}, {.73f, .86f}};
+  static constexpr float two[6][2] = {
+      {.37f, .46f}, {.67f, .82f}, {.70f, .88f}, {3.9f, 4.0f}, {.42f, .57f}, {.73f, .90f}};
+  const int rag = Kb % (prefetches(mode) && r.variant != 1 ? 256 : 128) != 0, bm = r.variant == 6 ? 64 : 128;
+  const int64_t tiles = (int64_t)((M + bm - 1) / bm) * ((N + 127) / 128), cu = device_cu_count();
+  const float fill = (float)tiles / cu, stages = (float)((Kb + 127) / 128), pad = r.pad_scales ? 4.5f : 0.f;
+  if (r.variant == 6) return 3.3f + .7f * rag + pad + stages * deep64[mode][rag] * (.8f + .2f * fill);
+  if (r.variant == 7) return 4.f + pad + stages * deep128[mode][rag] * (.75f + .25f * fill);
+  if (r.variant != 1) return 0;
+  const float again = (float)((tiles + cu - 1) / cu - 1);
+  return 3.2f + pad + stages * two[mode][rag] * (1.f + .4f * fill + .6f * again) + 2.f * again;
+}
+
+static float split_estimate(int mode, const Plan &pl, int M, int N, int Kb) {
+  static constexpr float step[6] = {.5f, .63f, .80f, 2.6f, .5f, .65f};
+  static constexpr float step256[6] = {1.4f, 6.2f, 6.6f, 10.9f, 1.4f, 6.2f};
+  const float steps = (float)Kb / pl.ksplit / 64, mb = (float)(M + N) * Kb * 1e-6f;
+  const float part = (float)pl.ksplit * M * (float)N * 4e-6f;
+  if (pl.variant == 0) {   // 256x256: few spills per-tensor and bf16, many in the others
+    if (mode != MODE_FP8_TENSOR && mode != MODE_BF16) return steps * step256[mode] + 1.4f * part + 1.2f * mb;
+    if (Kb % 128 == 0) return 13.f + steps * (mode == MODE_BF16 ? .95f : .68f) + .35f * part;
+    return 8.5f + steps * step256[mode] + .35f * part;
+  }
+  static constexpr float fixed[] = {0, 7.3f, 5.2f, 3.9f}, per_part[] = {0, .5f, .65f, .5f},
+                         per_mb[] = {0, .1f, .03f, .12f};
+  return fixed[pl.variant] + steps * step[mode] + per_part[pl.variant] * part + per_mb[pl.variant] * mb;
+}
+
+// 0: not predicted
+static float route_estimate(int mode, const Route &r, int M, int N, int K, int Kb, bool sc16) {
+  if (r.path == PATH_STREAM) return stream_estimate(mode, M, N, K, Kb, sc16);
+  if (r.path == PATH_PIPE) return pipe_estimate(mode, r, M, N, Kb);
+  if (r.path == PATH_TILED && r.tiled.ksplit > 1) return split_estimate(mode, r.tiled, M, N, Kb);
+  return 0;
+}
+
+// A shape takes the ragged forms and the one-round tiles unless the kernel that
+// serves it without them is predicted faster.  Those walk K in one chain per
+// workgroup: where few workgroups and a long K leave CUs idle, the split-K tiles
+// (or, NVFP4 and rows of an odd number of chunks, the other of the two) win:
+// bf16 129x3840x10528 streamed 80 us, split 41; per-tensor 2253x128x29776 on
+// 64x128 tiles 102, split 36; NVFP4 218x13312x256 streamed 45, 128x128 tiles 8.
+// Over 10800 sampled sizes the choice by size alone made 4% slower than the
+// kernels served before it, by up to 5.9 times; this leaves 1%, by 1.7 at most.
+// `ws`: bytes for the split's partial sums (their room is in the contract).
+static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc16, bool padded, bool f32,
+                       size_t ws) {
+  const Route r = pick_route(mode, M, N, K, Kb, sc4, sc16, padded, f32, true);
+  if (r.path != PATH_STREAM && r.path != PATH_PIPE) return r;
+  const Route w = pick_route(mode, M, N, K, Kb, sc4, sc16, padded, f32, false);
+  if (r.path == w.path) return r;
+  if (w.path == PATH_TILED && (w.tiled.ksplit < 2 || ws / sizeof(float) / w.tiled.ksplit < (size_t)splitk_slice(M, N)))
+    return r;
+  const float tr = route_estimate(mode, r, M, N, K, Kb, sc16), tw = route_estimate(mode, w, M, N, K, Kb, sc16);
+  return tr > 0 && tw > 0 && tr > tw ? w : r;
 }
 
 bool gemm_routes_to_stream(int mode, int64_t M, int64_t N, int64_t K, bool or_pipe, bool accumulate) {
   const int Kb = (mode == MODE_MXFP4 || mode == MODE_NVFP4) ? (int)(K / 2)
                                                             : (mode == MODE_BF16 ? (int)(2 * K) : (int)K);
-  int path = route_for(mode, (int)M, (int)N, (int)K, Kb, true, true, true, true).path;
+  int path = route_for(mode, (int)M, (int)N, (int)K, Kb, true, true, true, true, SIZE_MAX).path;
   if (accumulate && K <= kAccShortK && stream_enabled() && stream_supported(mode, (int)M, (int)N, (int)K, Kb, true))
     path = PATH_STREAM;   // as launch_gemm routes C += result
   return path == PATH_STREAM || (or_pipe && path == PATH_PIPE && (!accumulate || !mode_grouped_k(mode)));
@@ -505,8 +568,9 @@ size_t gemm_workspace_required(int mode, int64_t M, int64_t N, int64_t K, bool a
 
 size_t gemm_workspace_bytes(int mode, int64_t M, int64_t N, int64_t K, bool accumulate) {
   const size_t need = gemm_workspace_required(mode, M, N, K, accumulate);
-  if (accumulate || (mode != MODE_MXFP4 && mode != MODE_NVFP4)) return need;
-  const Route r = route_for(mode, (int)M, (int)N, (int)K, (int)(K / 2), true, true, true, true);
+  if (accumulate || (mode != MODE_MXFP4 && mode != MODE_NVFP4) || persist_whole(mode, (int)K, (int)(K / 2), true))
+    return need;                     // no scale rows to pad
+  const Route r = route_for(mode, (int)M, (int)N, (int)K, (int)(K / 2), true, true, true, true, SIZE_MAX);
   return r.pad_scales ? std::max(need, (size_t)(M + N) * (size_t)padded_pitch(mode, (int)K)) : need;
 }
 
@@ -572,14 +636,14 @@ void describe_gemm(int mode, int64_t M, int64_t N, int64_t K, bool f32, char *bu
       snprintf(to, room, "decode");
     }
   };
-  Route r = route_for(mode, (int)M, (int)N, (int)K, Kb, true, true, true, f32);
+  Route r = route_for(mode, (int)M, (int)N, (int)K, Kb, true, true, true, f32, SIZE_MAX);
   name(r, (int)M, (int)N, buf, len);
   GemmArgs p{};
   p.M = (int)M;
   p.N = (int)N;
   const int strip = r.path != PATH_PERSIST || r.narrow || r.pad_scales ? 0 : strip_columns(p);
   if (strip == 0) return;
-  Route rest = route_for(mode, (int)M, strip, (int)K, Kb, true, true, false, f32);
+  Route rest = route_for(mode, (int)M, strip, (int)K, Kb, true, true, false, f32, 0);
   if (rest.path != PATH_STREAM) {
     rest.path = PATH_PIPE;
     rest.variant = pipe_variant(mode, (int)M, strip, Kb);
@@ -607,7 +671,8 @@ hipError_t launch_gemm(int mode, GemmArgs p, hipStream_t st) {
   const bool padded = (mode == MODE_MXFP4 || mode == MODE_NVFP4) && p.ws &&
                       (reinterpret_cast<uintptr_t>(p.ws) & 15) == 0 &&
                       p.ws_bytes >= (size_t)((int64_t)p.M + p.N) * (size_t)padded_pitch(mode, p.K);
-  Route r = route_for(mode, p.M, p.N, p.K, p.Kb, (sc & 3) == 0, (sc & 15) == 0, padded, p.out_f32 != 0);
+  Route r = route_for(mode, p.M, p.N, p.K, p.Kb, (sc & 3) == 0, (sc & 15) == 0, padded, p.out_f32 != 0,
+                      p.ws ? p.ws_bytes : 0);
   if (p.lora_scales) {   // the LoRA epilogue: the streaming kernel only
     if (mode != MODE_BF16 || !stream_supported(mode, p.M, p.N, p.K, p.Kb, true) || p.accumulate)
       return hipErrorInvalidValue;
@@ -653,7 +718,7 @@ hipError_t launch_gemm(int mode, GemmArgs p, hipStream_t st) {
       const hipError_t e = launch_gemm_persist(mode, main, st, false);
       if (e != hipSuccess) return e;
       const GemmArgs rest = columns_from(mode, p, main.N);
-      return route_for(mode, rest.M, rest.N, rest.K, rest.Kb, (sc & 3) == 0, (sc & 15) == 0, false, p.out_f32 != 0).path ==
+      return route_for(mode, rest.M, rest.N, rest.K, rest.Kb, (sc & 3) == 0, (sc & 15) == 0, false, p.out_f32 != 0, 0).path ==
                      PATH_STREAM
                  ? launch_gemm_stream(mode, rest, st)
                  : launch_gemm_pipe(mode, rest, pipe_variant(mode, rest.M, rest.N, rest.Kb), st);

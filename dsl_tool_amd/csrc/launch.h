@@ -122,6 +122,8 @@ bool stream_whole(int mode, int K, int Kb, bool scales16);
 bool stream_blocks64(int mode, int M, int K, int Kb, bool scales16);
 // The plan's activation and W tiles per workgroup; whether the TAIL form runs.
 bool stream_plan(int mode, int M, int N, int K, int Kb, bool scales16, int *tma, int *tn);
+// Predicted time in us (the router compares it with the other kernels').
+float stream_estimate(int mode, int M, int N, int K, int Kb, bool scales16);
 hipError_t launch_gemm_stream(int mode, const GemmArgs &p, hipStream_t st);
 
 // Picks a kernel variant for the shape and launches it (plus the split-K

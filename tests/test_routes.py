@@ -90,6 +90,31 @@ def test_persistent_tiles_need_whole_columns_or_a_long_k(mode, m, n, k, want):
         assert route(mode, m, n, k, F32).startswith("persist")
 
 
+@pytest.mark.parametrize("mode,m,n,k,want", [
+    ("bf16", 129, 3840, 10528, "split"),       # 41 / 80
+    ("bf16", 681, 512, 14872, "split"),        # 48 / 105
+    ("block", 49, 4480, 14960, "split"),       # 26.8 / 53.8
+    ("group", 48, 4736, 12416, "split"),       # 24.2 / 36.1
+    ("tensor", 2253, 128, 29776, "split"),     # 36 / 102
+    ("nvfp4", 218, 13312, 256, "pipe"),        # 8.3 / 44.9
+    ("mxfp4", 87, 4840, 4608, "stream"),       # 7.1 / 10.7
+    ("tensor", 16, 4096, 4224, "stream tail"), # 6.1 / 11.4
+    ("mxfp4", 256, 4096, 4224, "stream tail"), # 12.4 / 76
+    ("block", 16, 4096, 4224, "stream tail")]) # 6.6 / 12.2
+def test_ragged_forms_are_compared_with_the_kernel_they_replaced(mode, m, n, k, want):
+    assert route(mode, m, n, k).startswith(want)
+
+
+def test_a_call_without_the_splits_room_keeps_the_ragged_form():
+    """The split's partial sums are in the workspace contract of its shapes."""
+    for mode, op in (("bf16", N.OP_BF16), ("block", N.OP_FP8), ("mxfp4", N.OP_FP4)):
+        for m, n, k in ((129, 3840, 10528), (36, 4480, 7456), (681, 512, 14880)):
+            r = route(mode, m, n, k)
+            if r.startswith("split"):
+                parts = int(r.split("/")[1])
+                assert N.lib().dsl_gemm_workspace_bytes(op, m, n, k) >= 4 * parts * m * n
+
+
 def transposed(rows, cols, gr, gc, f32=False, ptr=1 << 20):
     f = N.lib().dsl_test_quant_transposed
     f.restype, f.argtypes = ctypes.c_int, [ctypes.c_void_p, ctypes.c_int] + [ctypes.c_int64] * 6
