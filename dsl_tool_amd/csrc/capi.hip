@@ -804,8 +804,9 @@ int dsl_moe_combine(const void *y, int64_t rows, int64_t n, int64_t ldy, const i
 
 // Not part of the ABI (no header declares them): which kernel a call would take,
 // for the tests; no GPU is touched.  kind: a GEMM mode of launch.h.
-int dsl_test_gemm_route(int kind, int64_t m, int64_t n, int64_t k, int out_dtype, char *buf, size_t len) {
-  dsl::describe_gemm(kind, m, n, k, out_dtype == DSL_OUT_F32, buf, len);
+int dsl_test_gemm_route(int kind, int64_t m, int64_t n, int64_t k, int out_dtype, char *buf, size_t len,
+                        int accumulate) {
+  dsl::describe_gemm(kind, m, n, k, out_dtype == DSL_OUT_F32, accumulate != 0, buf, len);
   return DSL_OK;
 }
 

@@ -547,11 +547,33 @@ static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc1
   return tr > 0 && tw > 0 && tr > tw ? w : r;
 }
 
+// C += result streams where the router picks a skinny kernel, and for short K (a
+// LoRA adapter add: W is then small enough to stream once per activation block).
+// K of no whole chunk streams in the TAIL form, one chunk that three of a
+// workgroup's four waves wait for: past about 15K columns over the 64-row blocks
+// the pipelined tiles win where the router picks those (rank 8 to 32, the whole
+// layer, us streamed / tiles: 541x1024x1024 18.1 / 24.2, 300x2992x2624 37.4 /
+// 40.3, 276x3216x576 28.0 / 25.8, 773x3496x896 41.4 / 30.6).
+static bool acc_streams(int mode, int path, int M, int N, int K, int Kb, bool sc4, bool sc16) {
+  if (!stream_enabled() || !stream_supported(mode, M, N, K, Kb, sc4)) return false;
+  if (path == PATH_STREAM || path == PATH_DECODE) return true;
+  return K <= kAccShortK && (path != PATH_PIPE || stream_whole(mode, K, Kb, sc16) ||
+                             (int64_t)((M + 63) / 64) * N <= 15 * 1024);
+}
+
+// C += result (fp32 out, one writer per element): the streaming kernel, the
+// pipelined tiles where the router picks those (not block-scaled), else the
+// register-staged kernels.
+static void accumulate_route(int mode, Route *r, int M, int N, int K, int Kb, bool sc4, bool sc16) {
+  if (acc_streams(mode, r->path, M, N, K, Kb, sc4, sc16)) r->path = PATH_STREAM;
+  else if (r->path != PATH_PIPE || mode_grouped_k(mode)) r->path = PATH_TILED;
+}
+
 bool gemm_routes_to_stream(int mode, int64_t M, int64_t N, int64_t K, bool or_pipe, bool accumulate) {
   const int Kb = (mode == MODE_MXFP4 || mode == MODE_NVFP4) ? (int)(K / 2)
                                                             : (mode == MODE_BF16 ? (int)(2 * K) : (int)K);
   int path = route_for(mode, (int)M, (int)N, (int)K, Kb, true, true, true, true, SIZE_MAX).path;
-  if (accumulate && K <= kAccShortK && stream_enabled() && stream_supported(mode, (int)M, (int)N, (int)K, Kb, true))
+  if (accumulate && acc_streams(mode, path, (int)M, (int)N, (int)K, Kb, true, true))
     path = PATH_STREAM;   // as launch_gemm routes C += result
   return path == PATH_STREAM || (or_pipe && path == PATH_PIPE && (!accumulate || !mode_grouped_k(mode)));
 }
@@ -617,7 +639,8 @@ static int pipe_variant(int mode, int M, int N, int Kb) {
   return (int64_t)((M + 127) / 128) * ((N + 127) / 128) <= cu && deep_pays(mode, Kb) ? 7 : 1;
 }
 
-void describe_gemm(int mode, int64_t M, int64_t N, int64_t K, bool f32, char *buf, size_t len) {
+void describe_gemm(int mode, int64_t M, int64_t N, int64_t K, bool f32, bool accumulate, char *buf,
+                   size_t len) {
   const int Kb = (mode == MODE_MXFP4 || mode == MODE_NVFP4) ? (int)(K / 2)
                                                             : (mode == MODE_BF16 ? (int)(2 * K) : (int)K);
   auto name = [&](const Route &r, int m, int n, char *to, size_t room) {
@@ -637,10 +660,12 @@ void describe_gemm(int mode, int64_t M, int64_t N, int64_t K, bool f32, char *bu
     }
   };
   Route r = route_for(mode, (int)M, (int)N, (int)K, Kb, true, true, true, f32, SIZE_MAX);
+  if (accumulate && f32) accumulate_route(mode, &r, (int)M, (int)N, (int)K, Kb, true, true);
   name(r, (int)M, (int)N, buf, len);
   GemmArgs p{};
   p.M = (int)M;
   p.N = (int)N;
+  p.accumulate = accumulate;
   const int strip = r.path != PATH_PERSIST || r.narrow || r.pad_scales ? 0 : strip_columns(p);
   if (strip == 0) return;
   Route rest = route_for(mode, (int)M, strip, (int)K, Kb, true, true, false, f32, 0);
@@ -678,17 +703,9 @@ hipError_t launch_gemm(int mode, GemmArgs p, hipStream_t st) {
       return hipErrorInvalidValue;
     return launch_gemm_stream(mode, p, st);
   }
-  // C += result (fp32 out, one writer per element): the streaming kernel
-  // where the router picks a skinny kernel or K is short (a LoRA adapter
-  // add: W is then small enough to stream once per activation block), the
-  // pipelined tiles where the router picks those (not block-scaled), else
-  // the register-staged kernels
   if (p.accumulate) {
-    if ((r.path == PATH_STREAM || r.path == PATH_DECODE || p.K <= kAccShortK) && p.out_f32 &&
-        stream_enabled() && stream_supported(mode, p.M, p.N, p.K, p.Kb, (sc & 3) == 0))
-      r.path = PATH_STREAM;
-    else if (!(r.path == PATH_PIPE && p.out_f32 && !mode_grouped_k(mode)))
-      r.path = PATH_TILED;
+    if (p.out_f32) accumulate_route(mode, &r, p.M, p.N, p.K, p.Kb, (sc & 3) == 0, (sc & 15) == 0);
+    else r.path = PATH_TILED;
   }
   p.ksplit = 1;
   if (r.path == PATH_DECODE) return launch_gemm_decode(mode, p, st);

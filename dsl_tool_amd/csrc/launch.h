@@ -136,8 +136,8 @@ hipError_t launch_gemm(int mode, GemmArgs args, hipStream_t st);
 size_t gemm_workspace_required(int mode, int64_t M, int64_t N, int64_t K, bool accumulate = false);
 size_t gemm_workspace_bytes(int mode, int64_t M, int64_t N, int64_t K, bool accumulate = false);
 // The kernel launch_gemm would run (aligned operands, the queried workspace) as
-// text, for the tests.
-void describe_gemm(int mode, int64_t M, int64_t N, int64_t K, bool f32, char *buf, size_t len);
+// text, for the tests (accumulate: C += result).
+void describe_gemm(int mode, int64_t M, int64_t N, int64_t K, bool f32, bool accumulate, char *buf, size_t len);
 // Whether launch_gemm takes the streaming kernel (or_pipe: or the pipelined
 // tiles) for this shape (aligned scales; accumulate: C += result, fp32 out).
 bool gemm_routes_to_stream(int mode, int64_t M, int64_t N, int64_t K, bool or_pipe = false,

@@ -11,12 +11,12 @@ MODES = {"tensor": 0, "block": 1, "mxfp4": 2, "nvfp4": 3, "bf16": 4, "group": 5}
 BF16, F32 = N.OUT_BF16, N.OUT_F32
 
 
-def route(mode, m, n, k, out=BF16):
+def route(mode, m, n, k, out=BF16, accumulate=False):
     f = N.lib().dsl_test_gemm_route
     f.restype, f.argtypes = ctypes.c_int, [ctypes.c_int] + [ctypes.c_int64] * 3 + [
-        ctypes.c_int, ctypes.c_char_p, ctypes.c_size_t]
+        ctypes.c_int, ctypes.c_char_p, ctypes.c_size_t, ctypes.c_int]
     buf = ctypes.create_string_buffer(96)
-    assert f(MODES[mode], m, n, k, out, buf, len(buf)) == 0
+    assert f(MODES[mode], m, n, k, out, buf, len(buf), int(accumulate)) == 0
     return buf.value.decode()
 
 
@@ -158,3 +158,13 @@ def test_grouped_weights_are_read_in_place_where_that_fills_the_chip(g, rows, co
     if rows % 8 == 0:             # a pointer or pitch off the 16-byte grid is read element by element
         assert not Q._rows_in_place(4, 512, cols, esize, rows * cols, rows, (1 << 20) + 2)
         assert not Q._rows_in_place(4, 512, cols, esize, 512 * cols, 513, 1 << 20)
+
+
+@pytest.mark.parametrize("m,n,k,want", [     # the whole layer at rank 8 to 32
+    (541, 1024, 64, "stream tail 64x32"),    # 18.1 / 24.2
+    (300, 2992, 64, "stream tail 64x64"),    # 37.4 / 40.3
+    (276, 3216, 64, "pipe 128x128"),         # 25.8 / 28.0
+    (773, 3496, 64, "pipe 128x128"),         # 30.6 / 41.4
+    (773, 3496, 128, "stream 32x64")])       # whole chunks stream
+def test_adapter_adds_of_no_whole_chunk_stream_few_columns(m, n, k, want):
+    assert route("bf16", m, n, k, F32, accumulate=True) == want
