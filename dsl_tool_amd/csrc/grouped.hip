@@ -7,6 +7,7 @@
 // binary search.  Empty groups own zero tiles and are never touched.
 // Epilogue: y = (acc * sx[row]) * sw[g, col] (per-row activation scale,
 // per-channel weight scale).
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 
@@ -231,6 +232,39 @@ static void launch_grouped_pipe_cfg(const GroupedArgs &p, hipStream_t st) {
   grouped_pipe_kernel<Cfg><<<(unsigned)grid, Cfg::NT, 0, st>>>(p);
 }
 
+// Whether groups of a few rows go to the streaming tiles.  Rows of K of no whole
+// 256 bytes (their last chunk partial) have two exceptions where workgroups are
+// many (an estimate: the group sizes are on the device): K of less than one chunk
+// of 64-byte steps, more than four per CU, all latency (64 experts, N=2824 K=128,
+// 17 rows each: 32.4 us, 19.4 on the persistent tiles; 32 experts, N=976 K=192, 4
+// rows: 5.9 / 8.4); and long K with more than 32 rows, more than two per CU, whose
+// two row blocks read W twice (64 experts, N=1912 K=3776, 34 rows: 194 / 125;
+// N=672 K=1408, 34 rows: 29.9 / 34.3).
+static bool stream_few_rows(const GroupedArgs &p, int avg) {
+  if (avg >= 48 || !grouped_stream_supported(p)) return false;
+  if (p.K % 256 == 0) return true;
+  const int bm = avg <= 4 ? 16 : 32;
+  const int64_t blocks = std::min<int64_t>(p.rows, (int64_t)p.G * ((std::max(avg, 1) + bm - 1) / bm));
+  const int64_t wgs = blocks * ((p.N + 63) / 64), cu = device_cu_count();
+  if (p.K % 64 == 0 && p.K < 256 && wgs > 4 * cu) return false;
+  return avg <= 32 || (int64_t)p.rows * p.K < (int64_t)p.G * 57344 || wgs <= 2 * cu;
+}
+
+// Whether ragged K takes the persistent walk.  Past one round of the smaller
+// tiles (estimated from the average group) it is 1.5-2.5 times faster; within one
+// it gains about 6 us, loses 4 per 1024 of K to the longer chain of a 256x256 tile
+// and 21 per 256 columns of a partial last tile, which stores element by element:
+// N=1280 K=448 14.7 us / 24.1 on the 128x256 tiles, N=704 K=144 31.6 / 18.5 on the
+// 128x128 ones, N=984 K=688 33.6 / 22.2.  Short K that the above turned away
+// from streaming keeps to the small tiles.
+static bool persist_ragged(const GroupedArgs &p, int avg) {
+  const int bn = p.K % 64 == 0 ? 256 : 128;      // the kernels below: 128x256 or 128x128 tiles
+  if (p.K % 64 == 0 && avg >= 256) return true;  // (256x256 ones)
+  if (avg < 48 && p.K < 256) return false;
+  const double tiles = (double)((p.N + bn - 1) / bn) * (p.rows / 128.0 + p.G / 2.0);
+  return tiles > device_cu_count() || 21 * ((p.N % 256) / 256.0) + 4 * (p.K / 1024.0) < 6;
+}
+
 enum { GROUPED_NONE, GROUPED_STREAM, GROUPED_PERSIST, GROUPED_PIPE256, GROUPED_PIPE128, GROUPED_TILED };
 
 static int grouped_route(const GroupedArgs &p) {
@@ -239,7 +273,7 @@ static int grouped_route(const GroupedArgs &p) {
   // once with its rows (64 experts, N=1536 K=2048, 32 tokens x top-8: 37.4
   // against 53.3 us); from 64 rows per group the tiles win again (512
   // tokens: 63.8 us persistent, 117.9 streaming).
-  if (avg < 48 && grouped_stream_supported(p)) return GROUPED_STREAM;
+  if (stream_few_rows(p, avg)) return GROUPED_STREAM;
   // the gather form has no other kernel than the persistent one
   if (p.arow) return grouped_persist_supported(p) ? GROUPED_PERSIST : GROUPED_NONE;
   // DSL_GEMM_PERSIST=0 keeps the per-tile pipelined walk below (tuning)
@@ -254,7 +288,8 @@ static int grouped_route(const GroupedArgs &p) {
   // 256 rows: 64 experts, N=1536 K=2048, 1024 tokens x top-8 (128 rows per
   // expert): 67.6 against 110.2 us on the 128x256 pipelined tiles; 384
   // tokens: 63.8 against 71.9.
-  if (persist_on && grouped_persist_supported(p)) return GROUPED_PERSIST;
+  if (persist_on && grouped_persist_supported(p) && (p.K % 128 == 0 || persist_ragged(p, avg)))
+    return GROUPED_PERSIST;
   if (p.K % 64 != 0) return GROUPED_TILED;
   // DSL_GROUPED_TILE=256 / 128 forces the 256x256 / 128x256 tile (tuning)
   static const int forced = [] {

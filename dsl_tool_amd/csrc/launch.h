@@ -157,8 +157,8 @@ struct GroupedArgs {
   int out_f32;
   // gather form: x is [xrows][K] and sorted row r reads x row arow[r]
   // (persistent kernel, and the grouped streaming tiles; launch_grouped_fp8
-  // sends groups of fewer than 48 rows on average to the streaming tiles,
-  // the rest to the persistent kernel)
+  // sends groups of fewer than 48 rows on average to the streaming tiles where
+  // those are faster, the rest to the persistent kernel)
   const int32_t *arow = nullptr;
   int xrows = 0;
 };

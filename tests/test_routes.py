@@ -115,6 +115,45 @@ def test_a_call_without_the_splits_room_keeps_the_ragged_form():
                 assert N.lib().dsl_gemm_workspace_bytes(op, m, n, k) >= 4 * parts * m * n
 
 
+@pytest.mark.parametrize("m,n,k,want", [     # the whole layer at rank 8 to 32
+    (541, 1024, 64, "stream tail 64x32"),    # 18.1 / 24.2
+    (300, 2992, 64, "stream tail 64x64"),    # 37.4 / 40.3
+    (276, 3216, 64, "pipe 128x128"),         # 25.8 / 28.0
+    (773, 3496, 64, "pipe 128x128"),         # 30.6 / 41.4
+    (773, 3496, 128, "stream 32x64")])       # whole chunks stream
+def test_adapter_adds_of_no_whole_chunk_stream_few_columns(m, n, k, want):
+    assert route("bf16", m, n, k, F32, accumulate=True) == want
+
+
+def grouped_route(g, rows, n, k, gather=False):
+    f = N.lib().dsl_test_grouped_route
+    f.restype, f.argtypes = ctypes.c_char_p, [ctypes.c_int64] * 4 + [ctypes.c_int]
+    return f(g, rows, n, k, int(gather)).decode()
+
+
+@pytest.mark.parametrize("g,rows,n,k,want", [
+    (64, 1147, 2824, 128, "persist"),        # 19.4 / 32.4: K of less than a chunk
+    (64, 99, 2456, 64, "pipe 128x256"),      # 11.5 / 20.1
+    (64, 2202, 1912, 3776, "persist"),       # 128.7 / 193.8: two row blocks read W twice
+    (64, 2367, 352, 2896, "tiled"),          # 34.7 / 42.0
+    (32, 1036, 1112, 2944, "stream"),        # 34.8 / 40.6
+    (64, 256, 1536, 2048, "stream"),
+    (8, 73, 3736, 128, "stream"),            # 6.5 / 9.5
+    (2, 1982, 704, 144, "tiled"),            # 18.5 / 31.6: a round of small tiles, partial columns
+    (2, 1351, 2656, 3376, "tiled"),          # 48.2 / 56.9
+    (8, 891, 648, 3264, "pipe 128x256"),     # 38.7 / 50.7
+    (16, 1165, 1280, 448, "persist"),        # 14.7 / 24.1: whole columns
+    (16, 8192, 2048, 1168, "persist")])      # many tiles
+def test_grouped_routes(g, rows, n, k, want):
+    assert grouped_route(g, rows, n, k) == want
+
+
+def test_gathered_groups_have_the_persistent_or_the_streaming_kernel():
+    assert grouped_route(64, 1147, 2824, 128, True) == "persist"
+    assert grouped_route(64, 256, 1536, 1152, True) == "stream"
+    assert grouped_route(64, 8192, 1536, 2048, True) == "persist"
+
+
 def transposed(rows, cols, gr, gc, f32=False, ptr=1 << 20):
     f = N.lib().dsl_test_quant_transposed
     f.restype, f.argtypes = ctypes.c_int, [ctypes.c_void_p, ctypes.c_int] + [ctypes.c_int64] * 6
@@ -158,13 +197,3 @@ def test_grouped_weights_are_read_in_place_where_that_fills_the_chip(g, rows, co
     if rows % 8 == 0:             # a pointer or pitch off the 16-byte grid is read element by element
         assert not Q._rows_in_place(4, 512, cols, esize, rows * cols, rows, (1 << 20) + 2)
         assert not Q._rows_in_place(4, 512, cols, esize, 512 * cols, 513, 1 << 20)
-
-
-@pytest.mark.parametrize("m,n,k,want", [     # the whole layer at rank 8 to 32
-    (541, 1024, 64, "stream tail 64x32"),    # 18.1 / 24.2
-    (300, 2992, 64, "stream tail 64x64"),    # 37.4 / 40.3
-    (276, 3216, 64, "pipe 128x128"),         # 25.8 / 28.0
-    (773, 3496, 64, "pipe 128x128"),         # 30.6 / 41.4
-    (773, 3496, 128, "stream 32x64")])       # whole chunks stream
-def test_adapter_adds_of_no_whole_chunk_stream_few_columns(m, n, k, want):
-    assert route("bf16", m, n, k, F32, accumulate=True) == want
