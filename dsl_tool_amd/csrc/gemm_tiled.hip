@@ -619,12 +619,13 @@ static GemmArgs columns_from(int mode, GemmArgs p, int n1) {
 // 128x128 tiles (or the streaming kernel) holds.  us before -> after,
 // per-tensor / block / MXFP4 / NVFP4 / bf16: 2304x7680x4096 (270 tiles) 90 ->
 // 75, 106 -> 93, 63 -> 58, 190 -> 178, 177 -> 145; 4300x4300x4096 (289 tiles)
-// 141 -> 116, 158 -> 132, 113 -> 101, 241 -> 218, 230 -> 185.
+// 141 -> 116, 158 -> 132, 113 -> 101, 241 -> 218, 230 -> 185.  Not under
+// DSL_GEMM_PIPE, which names the tiles or forbids them.
 static int strip_columns(const GemmArgs &p) {
   const int cu = device_cu_count();
   const int nbm = (p.M + 255) / 256, nbn = (p.N + 255) / 256;
   const int64_t tiles = (int64_t)nbm * nbn, full = tiles / cu * cu;
-  if (p.accumulate || full == 0 || tiles == full || nbm > cu / 4) return 0;
+  if (p.accumulate || pipe_switch() != -1 || full == 0 || tiles == full || nbm > cu / 4) return 0;
   const int keep = (int)(full / nbm);                // whole columns of tiles in whole rounds
   if ((int64_t)nbm * (nbn - keep) > cu / 4 || keep < 1) return 0;
   return p.N - keep * 256;

@@ -2,6 +2,9 @@
 counts 256 CUs).  The sizes are measured ones at which an earlier rule picked
 the slower kernel; us of both in the comments, taken kernel first."""
 import ctypes
+import os
+import subprocess
+import sys
 
 import pytest
 
@@ -197,3 +200,19 @@ def test_grouped_weights_are_read_in_place_where_that_fills_the_chip(g, rows, co
     if rows % 8 == 0:             # a pointer or pitch off the 16-byte grid is read element by element
         assert not Q._rows_in_place(4, 512, cols, esize, rows * cols, rows, (1 << 20) + 2)
         assert not Q._rows_in_place(4, 512, cols, esize, 512 * cols, 513, 1 << 20)
+
+
+@pytest.mark.parametrize("value", ["off", "1"])
+def test_pipe_switch_also_holds_for_column_strips(value):
+    """DSL_GEMM_PIPE=off never uses the pipelined kernels; a number names one."""
+    call = "from tests.test_routes import route; print(route('bf16', 4300, 4300, 4096))"
+    env = dict(os.environ, DSL_GEMM_PIPE=value)
+    got = subprocess.run([sys.executable, "-c", call], env=env, capture_output=True, text=True, check=True,
+                         cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__)))).stdout.strip()
+    assert route("bf16", 4300, 4300, 4096).startswith("persist 256x256 + pipe")
+    assert got == "persist 256x256"
+
+
+def test_column_strips_of_few_rows_stream_their_rest():
+    assert route("tensor", 1000, 16640, 1024).startswith("persist 256x256 + stream")
+    assert route("bf16", 1000, 16640, 1024).startswith("persist 256x256 + stream")
