@@ -1199,6 +1199,7 @@ hipError_t launch_gemm_persist(int mode, const GemmArgs &p, hipStream_t st, bool
 }
 
 bool grouped_persist_supported(const GroupedArgs &p) {
+  if (p.arow && p.K % 128 != 0) return false;   // dsl_moe_grouped_fp8_gemm takes whole pairs only
   return p.K % 16 == 0 && p.K >= 128 && p.K < (1 << 24) && p.G >= 1 && p.G <= kMaxGroups;
 }
 
@@ -1221,7 +1222,6 @@ hipError_t launch_grouped_persist(const GroupedArgs &p, hipStream_t st) {
     // x rows are addressed by 32-bit offsets row * K
     if (p.xrows < 1 || (int64_t)p.xrows * p.K >= ((int64_t)1 << 32) || p.xrows >= (1 << 24))
       return hipErrorInvalidValue;
-    if (p.K % 128 != 0) return launch_grouped_persist_cfg<PersCfg<MODE_FP8_TENSOR, true, true, true>>(p, st);
     return launch_grouped_persist_cfg<PersCfg<MODE_FP8_TENSOR, true, true>>(p, st);
   }
   if (p.K % 128 != 0) return launch_grouped_persist_cfg<PersCfg<MODE_FP8_TENSOR, true, false, true>>(p, st);

@@ -155,6 +155,7 @@ def test_gathered_groups_have_the_persistent_or_the_streaming_kernel():
     assert grouped_route(64, 1147, 2824, 128, True) == "persist"
     assert grouped_route(64, 256, 1536, 1152, True) == "stream"
     assert grouped_route(64, 8192, 1536, 2048, True) == "persist"
+    assert grouped_route(64, 8192, 1536, 1168, True) == "none"   # refused by dsl_moe_grouped_fp8_gemm
 
 
 def transposed(rows, cols, gr, gc, f32=False, ptr=1 << 20):
