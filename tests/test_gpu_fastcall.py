@@ -147,3 +147,56 @@ def test_lora_adapters_packed_by_the_call(m, n, k, rank, loras):
     for l in range(loras):
         ref += s[l].double() * (x.double() @ a[l].double()) @ b[l].double()
     assert (got.double() - ref).abs().max() <= 2e-5 * ref.abs().max()
+
+
+def test_native_calls_run_on_the_current_stream_and_in_threads():
+    """The extension looks up the stream itself and runs without the GIL: calls on
+    side streams and from threads of their own give the bytes of calls in order."""
+    import threading
+    shapes = [(33, 200, 640), (16, 512, 1024)]
+    want = {}
+    for s in shapes:
+        want[s] = {nm: [t.clone() for t in _flat(f())] for nm, f in _calls(*s).items()}
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(s):
+        try:
+            st = torch.cuda.Stream()
+            with torch.cuda.stream(st):
+                calls = _calls(*s)
+                got = [{nm: _flat(f()) for nm, f in calls.items()} for _ in range(4)]
+                busy = torch.empty(1 << 22, device=DEV).normal_()      # later work on the stream's freed scratch
+                busy.mul_(2)
+            st.synchronize()
+            for r in got:
+                for nm, ts in r.items():
+                    bad.extend(nm for a, b in zip(ts, want[s][nm])
+                               if not torch.equal(a.view(torch.uint8), b.view(torch.uint8)))
+        except Exception as exc:          # a thread's error is the test's
+            bad.append(repr(exc))
+
+    threads = [threading.Thread(target=work, args=(s,)) for s in shapes * 2]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad, bad
+
+
+def test_a_call_waits_for_its_stream_only():
+    """Work queued on a side stream first: the call's result needs it, so a launch
+    on another stream would read the inputs before they are written."""
+    x = torch.zeros((512, 4096), dtype=torch.bfloat16, device=DEV)
+    src = _bf16((512, 4096), 21)
+    big = torch.empty(1 << 28, device=DEV)
+    torch.cuda.synchronize()
+    st = torch.cuda.Stream()
+    with torch.cuda.stream(st):
+        for _ in range(4):
+            big.fill_(1.0)                # a few hundred microseconds
+        x.copy_(src)
+        q, s = Q.quant_fp8_blocks(x, 1, 128)
+    st.synchronize()
+    q_ref, s_ref = Q.quant_fp8_blocks(src, 1, 128)
+    assert torch.equal(q, q_ref) and torch.equal(s, s_ref)
