@@ -449,8 +449,14 @@ LoraPlan lora_plan(int64_t m, int64_t n, int64_t k, int64_t lr) {
   LoraPlan p;
   p.ld2 = (2 * lr + 63) / 64 * 64;
   // T^T = A^T X^T on the streaming kernel when the adapter columns are few
-  // enough to be its skinny M; its epilogue writes hi | lo itself.
-  p.tt = lr <= 256 && (k % 128 == 0 || k % 64 != 0) && dsl::stream_supported(dsl::MODE_BF16, (int)lr, (int)m, (int)k, (int)(2 * k), true);
+  // enough to be its skinny M; its epilogue writes hi | lo itself.  Rows of an odd
+  // number of 64 elements would take that kernel's TAIL form while the plain GEMM
+  // of T (then split into hi | lo) has whole 128-byte stages: over 300 sampled
+  // layers the layer took 0.74 to 1.16 times as long streamed (3336x1992x6592,
+  // rank 128: 197 us, 170 by the GEMM; 1506x3016x6336, rank 16: 175 / 154), so
+  // they keep the GEMM.
+  p.tt = lr <= 256 && k % 128 != 64 &&
+         dsl::stream_supported(dsl::MODE_BF16, (int)lr, (int)m, (int)k, (int)(2 * k), true);
   // One pass (the adapter term as a second K segment of the persistent
   // kernel) unless both the base GEMM and the adapter add would take the
   // streaming kernel or the 128x128 pipelined tiles (up to 1024 rows at

@@ -58,9 +58,11 @@
 // LDS, with one more barrier per tile (zeroing the fragments in registers
 // instead spilled in the loop).  FP8 block: a row's last scale quad
 // is the row's last 16 bytes, overlapping the quad before it; the readers take
-// their scale at its distance from the quad's first.  E8M0 / E4M3 scale rows
-// that are no whole quads are first copied to a padded pitch (gemm_tiled.hip;
-// overlapping quads there cost registers: 8-12 bytes of spill).
+// their scale at its distance from the quad's first (256x256 tiles: 12 bytes
+// of spill, reloaded only where a row's last pair is cut and once per tile).
+// E8M0 / E4M3 scale rows that are no whole quads are first copied to a padded
+// pitch (gemm_tiled.hip): read as overlapping quads they spilled 8-12 bytes too,
+// on two formats whose loops have no register to spare.
 //
 // Epilogue: each wave converts its accumulators (v_cvt_pk_bf16_f32),
 // regroups them across lanes (v_permlane32_swap, v_permlane16_swap) and

@@ -164,7 +164,8 @@ struct GroupedArgs {
 };
 hipError_t launch_grouped_fp8(GroupedArgs args, hipStream_t st);
 const char *describe_grouped(const GroupedArgs &args);   // for the tests
-// Grouped FP8 on the persistent kernel (K % 16 == 0, 128 <= K < 2^24).
+// Grouped FP8 on the persistent kernel (K % 16 == 0, 128 <= K < 2^24; the gather
+// form K % 128 == 0).
 bool grouped_persist_supported(const GroupedArgs &args);
 hipError_t launch_grouped_persist(const GroupedArgs &args, hipStream_t st);
 // Grouped FP8 on the streaming tiles (few rows per group; K % 16 == 0).
@@ -230,11 +231,11 @@ hipError_t launch_lora_apply(const float *t, const uint16_t *b_t, float *y, int 
                              int64_t ldy, hipStream_t st);
 hipError_t launch_lora_split(const float *t32, int M, int LR, int ld2, int rank,
                              const float *scales, uint16_t *t2, hipStream_t st);
-// bt [N][LR] -> b2 [N][ld2] = bt | bt | 0.
 // A [L][K][R], B [L*R][N] -> a_t [L*R][K] and B^T (dup: B^T | B^T | 0) of
 // pitch ldb, one launch.
 hipError_t launch_lora_pack(const uint16_t *a, const uint16_t *b, int L, int K, int R, int N, uint16_t *a_t,
                             uint16_t *b_out, int ldb, bool dup, hipStream_t st);
+// bt [N][LR] -> b2 [N][ld2] = bt | bt | 0.
 hipError_t launch_lora_dup(const uint16_t *bt, int N, int LR, int ld2, uint16_t *b2,
                            hipStream_t st);
 

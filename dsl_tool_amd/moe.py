@@ -8,8 +8,7 @@ An MoE FFN projection, on the device end to end:
     out = moe_combine(y, route, topk_weights)       # weighted sum over each token's experts
 
 ``routed_grouped_gemm`` runs the four steps (registered as
-``moe.routed_grouped_gemm``).  Where the persistent grouped kernel takes the
-GEMM (groups averaging 48 rows or more, K % 128 == 0) the middle two are
+``moe.routed_grouped_gemm``).  Where K % 128 == 0 the middle two are
 ``moe_quant_tokens`` (codes in token order, scales per sorted row) and
 ``moe_grouped_fp8_gemm``, which reads each sorted row's A through
 ``route.src_token``: the codes are written once per token instead of topk
@@ -177,7 +176,7 @@ def gather_applies(tokens: int, topk: int, num_experts: int, k: int) -> bool:
     """Whether the routed GEMM reads A through the row map: k % 128 == 0,
     tokens < 2^24 and tokens * k < 2^32.  Groups averaging 48 rows or more
     take the persistent grouped kernel, fewer the streaming grouped tiles
-    (k % 256 == 0; else the persistent kernel again)."""
+    (of an odd number of 128s where those are faster)."""
     return (k % 128 == 0 and 1 <= num_experts <= 2048
             and tokens < (1 << 24) and tokens * k < (1 << 32))
 

@@ -173,6 +173,9 @@ int dsl_fp8_gemm(const uint8_t *a, const uint8_t *b, void *c,
  *                  the scaled MFMA; global_a/global_b unused (may be NULL).
  *   DSL_FMT_NVFP4: scale_a [M][K/16], scale_b [N][K/16] E4M3 bytes,
  *                  global_a/global_b -> one float each (device).
+ * The scale arrays may start at any byte.  They are read in aligned 4-byte words,
+ * so up to 3 bytes on either side of an array may be read with its first and last
+ * words (never another word; what they hold reaches no result).
  * K % 32 == 0.  Replaces fp4_gemm / fp4_gemm_kernel
  * (cuda/gemm/fp4_gemm.cu:92-146). */
 int dsl_fp4_gemm(const uint8_t *a, const uint8_t *b, void *c,
@@ -338,8 +341,12 @@ int dsl_moe_combine(const void *y, int64_t rows, int64_t n, int64_t ldy, const i
                     void *out, int64_t ldo, int out_dtype, void *stream);
 
 /* Workspace bytes dsl_fp8_gemm / dsl_fp4_gemm / dsl_bf16_gemm need for this
- * shape (op = DSL_OP_FP8, DSL_OP_FP4 or DSL_OP_BF16; for FP8 / FP4 the larger of the plans of the op's two
- * scale modes / FP4 formats; 0 when none is needed).  The kernel choice
+ * shape (op = DSL_OP_FP8, DSL_OP_FP4 or DSL_OP_BF16; for FP8 / FP4 the largest of the plans of the op's
+ * scale modes / FP4 formats; 0 when none is needed).  It is the room of the
+ * split-K partial sums of shapes that have no kernel for whole rows, up to 16 fp32
+ * copies of C, and required of every call of such a shape (DSL_ERR_WORKSPACE),
+ * although most of them now take a kernel for partial rows that leaves it unread:
+ * split K remains the faster one for few rows or columns and a long K.  The kernel choice
  * depends on the shape and on the scale pointers' alignment; with scale
  * arrays that are not 16-byte aligned a launch may fall back to a kernel
  * that runs without split-K rather than ask for more workspace.  For FP4 with

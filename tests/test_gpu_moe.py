@@ -231,7 +231,7 @@ def _expert_weights(E, Nn, K, seed):
 # rows per group on average the gather streams (the streaming grouped tiles
 # over the permuted copy are the reference): decode sizes with 16- and
 # 32-row blocks, K of an odd number of 256-byte chunks, ragged N, and
-# K % 256 != 0 (the persistent kernel again).
+# K % 256 != 0 (a partial last chunk).
 GATHER_CASES = [(512, 4, 16, 1024, 768), (300, 3, 2, 128, 520), (1000, 2, 5, 256, 256),
                 (2000, 1, 1, 384, 300), (4096, 8, 64, 2048, 1536),
                 (32, 8, 64, 2048, 1536), (1, 8, 64, 2048, 1536), (200, 8, 64, 2048, 1536),
