@@ -470,8 +470,6 @@ LoraPlan lora_plan(int64_t m, int64_t n, int64_t k, int64_t lr) {
                            dsl::gemm_routes_to_stream(dsl::MODE_BF16, m, n, p.ld2, true, true);
   p.one_pass = dsl::persist_supported(dsl::MODE_BF16, (int)m, (int)n, (int)k, (int)(2 * (k + p.ld2)), true) &&
                (2 * k) % 128 == 0 && m > 256 && !both_stream;
-  // hi | lo against B^T | B^T without the copy (one pass only): B^T's rows
-  // must be whole pairs (64 bf16), a power of two of them, filling ld2 / 2
   // Up to 256 tokens T comes from the vector-ALU kernel, which splits A^T's
   // rows over workgroups (the streaming kernel's T^T runs the 64 adapter rows
   // as one row block: one workgroup streams all of A^T); for the fewest
@@ -488,6 +486,8 @@ LoraPlan lora_plan(int64_t m, int64_t n, int64_t k, int64_t lr) {
     p.total = p.t32 + p.ws;
     return p;
   }
+  // hi | lo against B^T | B^T without the copy (one pass only): B^T's rows
+  // must be whole pairs (64 bf16), a power of two of them, filling ld2 / 2
   const int64_t pr = lr / 64;
   p.rep = (p.one_pass && lr % 64 == 0 && (pr & (pr - 1)) == 0 && p.ld2 == 2 * lr) ? (int)pr : 0;
   const size_t ws1 = dsl::gemm_workspace_bytes(dsl::MODE_BF16, m, lr, k);

@@ -176,7 +176,7 @@ def gather_applies(tokens: int, topk: int, num_experts: int, k: int) -> bool:
     """Whether the routed GEMM reads A through the row map: k % 128 == 0,
     tokens < 2^24 and tokens * k < 2^32.  Groups averaging 48 rows or more
     take the persistent grouped kernel, fewer the streaming grouped tiles
-    (of an odd number of 128s where those are faster)."""
+    (K of an odd number of 128s only where those are faster)."""
     return (k % 128 == 0 and 1 <= num_experts <= 2048
             and tokens < (1 << 24) and tokens * k < (1 << 32))
 
