@@ -539,6 +539,11 @@ static Route route_for(int mode, int M, int N, int K, int Kb, bool sc4, bool sc1
                        size_t ws) {
   const Route r = pick_route(mode, M, N, K, Kb, sc4, sc16, padded, f32, true);
   if (r.path != PATH_STREAM && r.path != PATH_PIPE) return r;
+  // The second pick and the estimates cost host time (0.13 us of a 5.4 us call of
+  // 3 rows): not for up to 16 rows, which stream at least as fast as either of the
+  // others (groupwise 5x45352x1184 14.0 us, split 16.0; MXFP4 3x36464x256 10.1 /
+  // 10.1 on tiles), nor for a whole K, which streams either way.
+  if (r.path == PATH_STREAM && (M <= 16 || stream_whole(mode, K, Kb, sc16))) return r;
   const Route w = pick_route(mode, M, N, K, Kb, sc4, sc16, padded, f32, false);
   if (r.path == w.path) return r;
   if (w.path == PATH_TILED && (w.tiled.ksplit < 2 || ws / sizeof(float) / w.tiled.ksplit < (size_t)splitk_slice(M, N)))

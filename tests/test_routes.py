@@ -118,6 +118,14 @@ def test_a_call_without_the_splits_room_keeps_the_ragged_form():
                 assert N.lib().dsl_gemm_workspace_bytes(op, m, n, k) >= 4 * parts * m * n
 
 
+@pytest.mark.parametrize("mode,m,n,k", [
+    ("group", 5, 45352, 1184),      # 14.0 / 16.0
+    ("block", 5, 44096, 1200),      # 14.5 / 16.6
+    ("mxfp4", 3, 36464, 256)])      # 10.1 / 10.1
+def test_up_to_16_rows_of_ragged_k_stream(mode, m, n, k):
+    assert route(mode, m, n, k).startswith("stream tail")
+
+
 @pytest.mark.parametrize("m,n,k,want", [     # the whole layer at rank 8 to 32
     (541, 1024, 64, "stream tail 64x32"),    # 18.1 / 24.2
     (300, 2992, 64, "stream tail 64x64"),    # 37.4 / 40.3
