@@ -11,6 +11,7 @@ from dsl_tool_amd import _native as N
 from dsl_tool_amd import gemm as G
 from dsl_tool_amd import quant as Q
 from dsl_tool_amd import workloads as W
+from tests.test_gpu_lora import test_lora_fused_gemm as check_lora
 from tests.test_gpu_random_shapes import test_random_shape as check
 from tests.test_routes import BF16, F32, grouped_route, route
 from tests.util import assert_close
@@ -68,6 +69,17 @@ def test_routed_grouped_kernel(counts, n, k, want):
     wd = (qw.view(torch.float8_e4m3fn).double() * sw.double()).float().view(g, n, k)
     ref = torch.cat([xd[off[e]:off[e + 1]] @ wd[e].t() for e in range(g)])
     assert_close(y, ref.cpu().numpy(), what=f"grouped {want} {g}x{t} {n}x{k}")
+
+
+@pytest.mark.parametrize("m,n,k,r,l,want", [   # want: the adapter add
+    (541, 1024, 1032, 8, 4, "stream tail"), (300, 1000, 832, 8, 2, "stream tail"),
+    (773, 3496, 832, 8, 2, "pipe 128x128"), (773, 3496, 1096, 16, 2, "pipe 128x128"),
+    (773, 3496, 576, 16, 4, "stream 32x"), (700, 1200, 1096, 16, 4, "stream 32x")])
+def test_lora_adapter_adds(m, n, k, r, l, want):
+    """K of whole 64s that are no whole 128s (T from the plain GEMM) and ragged K."""
+    got = route("bf16", m, n, (2 * r * l + 63) // 64 * 64, F32, accumulate=True)
+    assert got.startswith(want) and "deep" not in got, got
+    check_lora(m, n, k, r, l)
 
 
 def test_unaligned_scales_do_not_take_a_split_they_have_no_room_for():
